@@ -201,6 +201,10 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
 
 /* Workspace bytes the chunk-parallel scan needs for these inputs (shapes and
  * dtype are read; pointers are not); 0 when the shape runs single-pass only.
+ * For small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4; 128 rows of
+ * (token, rank) or more, up to 512 sequences) it holds zero-padded f32 copies
+ * the chunk-parallel kernels run on; without it those shapes run as one
+ * workgroup per sequence.
  * No reference counterpart (see m3_scan_inputs.workspace). */
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
 
@@ -264,8 +268,9 @@ typedef struct m3_scan_grads {
  * chunk states are recomputed; the forward outputs are not needed.  The
  * chunk kernels take head_dim 64, d_state 64/128, rank 1/2/4 with aligned
  * buffers; their partial sums inside a workgroup are accumulated with LDS
- * atomics, so repeated calls agree to f32 rounding, not bit for bit.  Other
- * shapes (and alignments) take the reverse mode of the recurrence token by
+ * atomics, so repeated calls agree to f32 rounding, not bit for bit.  Small
+ * heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens on) run
+ * them on zero-padded copies in the workspace.  Other shapes (and alignments) take the reverse mode of the recurrence token by
  * token, one workgroup per sequence with states recomputed from checkpoints
  * every 32 tokens (deterministic, and slow: a fallback), up to per-token
  * vectors of 64 KB (2 head_dim rank + 4 d_state rank + 3 d_state/2 floats;

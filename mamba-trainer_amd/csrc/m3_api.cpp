@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -491,7 +492,11 @@ static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
         a.gate_z = gate_z;
         a.gate_stride = gate_stride;
     }
-    if (chunked) {
+    const size_t pad_need = need > 0 || !ws_aligned ? 0 : m3::scan_pad_workspace(a);
+    if (pad_need > 0 && in->workspace != nullptr && in->workspace_bytes >= pad_need) {
+        e = m3::launch_scan_pad(a, in->workspace, s);
+        if (e == hipSuccess) g_launches.fetch_add(m3::scan_pad_launches(a), std::memory_order_relaxed);
+    } else if (chunked) {
         e = m3::launch_scan_chunked(a, in->workspace, s);
         if (e == hipSuccess)
             g_launches.fetch_add(m3::scan_chunked_launches(a), std::memory_order_relaxed);
@@ -532,7 +537,9 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
 
 }  // extern "C"
 
-static size_t workspace_bytes_for(const m3_scan_inputs *in, int path) {
+// pads: the padded copies of small heads included (m3_scan_no_alloc's static
+// scratch runs those shapes without a workspace, as a caller who passes none).
+static size_t workspace_bytes_for(const m3_scan_inputs *in, int path, bool pads) {
     if (in == nullptr || !dtype_ok(in->dtype) || in->seq == 0) return 0;
     m3::ScanLaunch a{};
     a.path = path;
@@ -549,13 +556,14 @@ static size_t workspace_bytes_for(const m3_scan_inputs *in, int path) {
     alignas(16) static float dummy[4] = {0, 0, 0, 0};
     a.x = a.b = a.c = dummy;
     a.y = dummy;
-    return m3::scan_chunked_workspace(a);
+    const size_t need = m3::scan_chunked_workspace(a);
+    return need == 0 && pads ? m3::scan_pad_workspace(a) : need;
 }
 
 extern "C" {
 
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in) {
-    return workspace_bytes_for(in, g_scan_path.load(std::memory_order_relaxed));
+    return workspace_bytes_for(in, g_scan_path.load(std::memory_order_relaxed), true);
 }
 
 m3_status m3_debug_scan_options(int32_t path, int32_t lookback_mode, int32_t lookback_spin) {
@@ -639,10 +647,10 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
     local.workspace = nullptr;
     local.workspace_bytes = 0;
     int path = g_scan_path.load(std::memory_order_relaxed);
-    size_t need = workspace_bytes_for(&local, path);
+    size_t need = workspace_bytes_for(&local, path, false);
     if (need > kNoAllocScratchBytes && path == 0) {
         // the fused launch's records do not fit: the three launches' may
-        const size_t three = workspace_bytes_for(&local, 1);
+        const size_t three = workspace_bytes_for(&local, 1, false);
         if (three <= kNoAllocScratchBytes) {
             path = 1;
             need = three;
@@ -805,8 +813,13 @@ m3_status m3_scan_backward(const m3_scan_inputs *in, const m3_scan_grads *g, voi
                 return fail(M3_ERR_UNSUPPORTED,
                             "the scan backward needs 16-byte aligned gradient buffers");
     }
-    const size_t need = generic ? m3::scan_backward_generic_workspace(a)
-                                : m3::scan_backward_workspace(a);
+    // small heads run the chunk kernels on padded copies where the workspace
+    // is the query's (a smaller one that holds the token walk's still runs it)
+    const size_t pad_need = generic ? m3::scan_backward_pad_workspace(a) : 0;
+    const bool pad = pad_need > 0 && in->workspace_bytes >= pad_need;
+    const size_t need = pad ? pad_need
+                            : generic ? m3::scan_backward_generic_workspace(a)
+                                      : m3::scan_backward_workspace(a);
     if (in->workspace == nullptr || in->workspace_bytes < need ||
         (reinterpret_cast<uintptr_t>(in->workspace) & 255u) != 0)
         return fail(M3_ERR_ARGUMENT, "the backward needs a 256-byte aligned workspace of %zu bytes",
@@ -827,14 +840,20 @@ m3_status m3_scan_backward(const m3_scan_inputs *in, const m3_scan_grads *g, voi
     gr.dh0 = st ? g->dh0 : nullptr;
     gr.dlast_u0 = st ? g->dlast_u0 : nullptr;
     gr.dangle0 = (st && st->angle && in->theta) ? g->dangle0 : nullptr;
-    if (generic) {
+    // the chunk kernels' launches
+    const uint64_t launches = (in->theta ? 5 : 4) + (g->dlast_u ? 2 : 0);
+    if (pad) {
+        e = m3::launch_scan_backward_pad(a, gr, in->workspace, s);
+        if (e != hipSuccess) return hip_fail(e, "scan backward launch");
+        g_launches.fetch_add(launches + 2, std::memory_order_relaxed);
+    } else if (generic) {
         e = m3::launch_scan_backward_generic(a, gr, in->workspace, s);
         if (e != hipSuccess) return hip_fail(e, "scan backward launch");
         g_launches.fetch_add(2, std::memory_order_relaxed);
     } else {
         e = m3::launch_scan_backward(a, gr, in->workspace, s);
         if (e != hipSuccess) return hip_fail(e, "scan backward launch");
-        g_launches.fetch_add((in->theta ? 5 : 4) + (g->dlast_u ? 2 : 0), std::memory_order_relaxed);
+        g_launches.fetch_add(launches, std::memory_order_relaxed);
     }
     if (g->dd_skip != nullptr && in->d_skip == nullptr) {
         e = hipMemsetAsync(g->dd_skip, 0, H * sizeof(float), s);
@@ -851,7 +870,8 @@ size_t m3_scan_backward_workspace_bytes(const m3_scan_inputs *in) {
     a.theta = in->theta ? dummy : nullptr;
     a.h0 = a.last_u0 = nullptr;
     const size_t w = m3::scan_backward_workspace(a);
-    return w ? w : m3::scan_backward_generic_workspace(a);
+    if (w) return w;
+    return std::max(m3::scan_backward_pad_workspace(a), m3::scan_backward_generic_workspace(a));
 }
 
 m3_status m3_ssd_chunked(const m3_ssd_args *in, void *y, float *final_state, void *stream) {

@@ -167,6 +167,19 @@ size_t scan_backward_generic_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward_generic(const ScanLaunch &a, const ScanGrads &g, void *workspace,
                                         hipStream_t stream);
 
+// The heads of small models (head_dim up to 32, d_state up to 64, rank 1, 2 or
+// 4) on zero-padded copies through the kernels above (scan_pad.hip): whether
+// that is the faster form, the workspace it takes (0 where it is not), its
+// kernel launches and the launch.
+bool scan_pad_wanted(const ScanLaunch &a);
+size_t scan_pad_workspace(const ScanLaunch &a);
+int scan_pad_launches(const ScanLaunch &a);
+hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream);
+bool scan_backward_pad_wanted(const ScanLaunch &a);
+size_t scan_backward_pad_workspace(const ScanLaunch &a);
+hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,
+                                    hipStream_t stream);
+
 // Largest head_dim / d_state the scan kernels are instantiated for.
 constexpr size_t kScanMaxHeadDim = 128;
 constexpr size_t kScanMaxState = 256;

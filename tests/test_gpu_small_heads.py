@@ -1,0 +1,142 @@
+"""Small heads (head_dim <= 32, d_state <= 64) on zero-padded copies through
+the chunk kernels: the forward and the backward against the f64 oracles at the
+smallest and largest padded sizes, ragged windows, every option, and the
+kernels the call took (its launch count); a workspace too small for the padded
+copies runs the kernels of before.
+
+Bars as in test_gpu_scan.py and test_gpu_backward.py: rel-L2 <= 1e-5 for f32
+storage, <= 1e-2 for bf16.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from cases import baseline_inputs, rel_l2
+from gpu_util import dev, host, oracle_scan, run_scan
+from test_gpu_backward import BF16_TOL, F32_TOL, NAMES, _run
+
+# B, T, H, P, N, R, theta, skip, state, dtype
+CASES = [
+    (2, 128, 3, 3, 6, 1, True, True, True, "f32"),       # the shortest window, far from a tile
+    (1, 129, 2, 32, 64, 1, True, True, True, "f32"),     # the largest head, one token over
+    (1, 200, 2, 16, 16, 1, True, True, True, "bf16"),
+    (1, 131, 2, 1, 2, 1, True, False, False, "f32"),     # one column, one pair
+    (2, 150, 1, 17, 5, 1, False, True, True, "f32"),     # odd d_state, real dynamics
+    (1, 70, 3, 5, 1, 2, False, False, True, "f32"),      # d_state 1
+    (1, 33, 2, 32, 32, 4, True, True, True, "bf16"),     # rank 4
+    (1, 75, 2, 8, 64, 2, True, True, True, "bf16"),      # rank 2
+]
+SHORT = [(2, 8, 2, 16, 16, 1, True, True, True, "f32"), (1, 7, 2, 16, 16, 1, True, True, True, "f32")]
+
+
+def _launches(fn):
+    from mamba3 import _lib
+    before = _lib.lib().m3_launch_count()
+    out = fn()
+    return out, _lib.lib().m3_launch_count() - before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=[repr(c) for c in CASES])
+def test_forward_against_f64(case):
+    B, T, H, P, N, R, theta, skip, state, dtype = case
+    rng = np.random.default_rng(B * T + P * N + R)
+    inp = baseline_inputs(rng, B, T, H, P, N, R, theta=theta, dtype=dtype, theta_per_head=False,
+                          state=state)
+    d_skip = rng.uniform(-1, 1, H).astype(np.float32) if skip else None
+    st = (inp["h0"], inp["last_u0"], inp.get("angle0")) if state else None
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    (y, h, lu, ang), n = _launches(lambda: run_scan(inp, dtype=tdt, theta=theta, skip=d_skip,
+                                                    state=st))
+    assert n == 5   # the copies, the three chunk launches, the copies back
+    y64, h64, lu64, ang64 = oracle_scan(inp, theta=theta, skip=d_skip, state=st)
+    assert rel_l2(y, y64) <= (BF16_TOL if dtype == "bf16" else F32_TOL)
+    # the state is f32 whatever the storage
+    assert rel_l2(h, h64) <= F32_TOL and rel_l2(lu, lu64) <= F32_TOL
+    if theta:
+        d = np.abs(ang - ang64)
+        assert np.max(np.minimum(d, 2 * np.pi - d)) <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES + SHORT, ids=[repr(c) for c in CASES + SHORT])
+def test_backward_against_f64_reverse_mode(case):
+    (g, ref), n = _launches(lambda: _run(case))
+    theta = case[6]
+    # from 8 tokens on: the copies, the chunk kernels and the outgoing last_u's
+    # two, the copies back; below, the token walk and the head sums
+    assert n == (2 if case[1] < 8 else (9 if theta else 8))
+    tol = BF16_TOL if case[-1] == "bf16" else F32_TOL
+    checked = 0
+    for k in NAMES:
+        mine = getattr(g, k)
+        if mine is None or ref.get(k) is None:
+            continue
+        assert rel_l2(host(mine), ref[k]) <= tol, (k, rel_l2(host(mine), ref[k]))
+        checked += 1
+    assert checked >= 6
+
+
+def _query(B, T, H, P, N, R, dtype):
+    from mamba3 import _lib
+    cin = _lib.ScanInputsC(B, T, H, P, N, R, dtype, None, None, None, None, None, None, None, None,
+                           None, 64, 1, None, 0)
+    L = _lib.lib()
+    return (int(L.m3_scan_workspace_bytes(C.byref(cin))),
+            int(L.m3_scan_backward_workspace_bytes(C.byref(cin))))
+
+
+def test_workspace_queries_at_the_edges():
+    """Padded copies are asked for at head_dim <= 32, d_state <= 64 and rank 1,
+    2 or 4; the forward from 128 rows and up to 512 sequences."""
+    from mamba3 import _lib
+    f32, bf16 = _lib.M3_F32, _lib.M3_BF16
+    assert _query(2, 128, 4, 16, 16, 1, f32)[0] > 0 and _query(2, 127, 4, 16, 16, 1, f32)[0] == 0
+    assert _query(2, 32, 4, 16, 16, 4, bf16)[0] > 0 and _query(2, 31, 4, 16, 16, 4, bf16)[0] == 0
+    assert _query(64, 128, 8, 16, 16, 1, f32)[0] > 0 and _query(64, 128, 9, 16, 16, 1, f32)[0] == 0
+    for P, N, R in ((33, 16, 1), (16, 65, 1), (16, 16, 3)):
+        assert _query(2, 256, 4, P, N, R, f32)[0] == 0
+    # the widened forward's copies are f32; the backward keeps the storage type
+    assert _query(2, 256, 4, 16, 16, 1, bf16)[0] == _query(2, 256, 4, 16, 16, 1, f32)[0]
+    assert _query(2, 256, 4, 16, 16, 1, bf16)[1] < _query(2, 256, 4, 16, 16, 1, f32)[1]
+
+
+@pytest.mark.gpu
+def test_a_smaller_workspace_runs_the_kernels_of_before():
+    from mamba3 import _lib
+    L = _lib.lib()
+    B, T, H, P, N = 1, 160, 2, 16, 16
+    rng = np.random.default_rng(5)
+    inp = baseline_inputs(rng, B, T, H, P, N, 1, theta=True, theta_per_head=False)
+    t = {k: dev(v) for k, v in inp.items() if v is not None}
+    cin = _lib.ScanInputsC(B, T, H, P, N, 1, _lib.M3_F32, t["x"].data_ptr(), t["b"].data_ptr(),
+                           t["c"].data_ptr(), t["dt"].data_ptr(), t["a_log"].data_ptr(),
+                           t["lam"].data_ptr(), t["theta"].data_ptr(), None, None, 64, 0, None, 0)
+    fw, bw = (int(q(C.byref(cin))) for q in (L.m3_scan_workspace_bytes,
+                                            L.m3_scan_backward_workspace_bytes))
+    ws = torch.empty(max(fw, bw), dtype=torch.uint8, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    outs = []
+    for size, launches in ((fw, 5), (fw - 1, 1)):
+        cin.workspace, cin.workspace_bytes = ws.data_ptr(), size
+        y = torch.empty_like(t["x"])
+        cout = _lib.ScanOutputC(y.data_ptr(), _lib.SsmStateC())
+        _, n = _launches(lambda: _lib.check(L.m3_scan(C.byref(cin), C.byref(cout), stream)))
+        assert n == launches
+        outs.append(host(y))
+    assert rel_l2(outs[0], outs[1]) <= F32_TOL
+    dy = dev(rng.standard_normal((B, T, H, P, 1)).astype(np.float32))
+    grads = []
+    for size, launches in ((bw, 7), (bw - 1, 2)):
+        cin.workspace, cin.workspace_bytes = ws.data_ptr(), size
+        g = {k: torch.empty_like(t[k]) for k in ("x", "b", "c", "dt", "lam", "a_log", "theta")}
+        gc = _lib.ScanGradsC(dy.data_ptr(), None, None,
+                             *[g[k].data_ptr() for k in ("x", "b", "c", "dt", "lam", "a_log",
+                                                         "theta")], None, None, None, None)
+        _, n = _launches(lambda: _lib.check(L.m3_scan_backward(C.byref(cin), C.byref(gc), stream)))
+        assert n == launches
+        grads.append({k: host(v) for k, v in g.items()})
+    for k in grads[0]:
+        assert rel_l2(grads[0][k], grads[1][k]) <= F32_TOL, k
