@@ -1,0 +1,179 @@
+// Linear::apply for a handful of rows (a decode step of one or a few
+// sequences) on gfx950:
+//   y[m, n] = (x[m, :] . w^T[n, :]) * scale[n] + res[m, n]
+// bf16 x [M, K] and w^T [N, K], f32 accumulation, the per-column scale and the
+// residual in the epilogue, bf16 y (nn/linear.rs:155-185).
+//
+// The product is a stream over the weights, each read once; what bounds a
+// call of a few MB is how soon enough of it is in flight.  A workgroup owns 16
+// NT columns of y and its WK waves split K: wave q takes the 64-k blocks q, q +
+// WK, ..., each lane loading its weights and x straight into the registers the
+// MFMA reads them from (row c, k = 16 g .. 16 g + 15 of the block: two 16-byte
+// loads a tile, whole 128-byte lines a row; no LDS, no barrier on the way),
+// two groups of U blocks in flight.  bf16 MFMA 16x16x32 forms y^T = W^T X^T,
+// so one to sixteen rows cost the same; rows and columns past the end read as
+// zeros.  The waves' partial sums meet in LDS, in wave order.
+//
+// Measured on MI355X (us per call, captured, weights from HBM, against the
+// product's route before: hipBLASLt from 4096 columns on, skinny_gemm.hip
+// below), K x N at 1 / 16 rows: 1536 x 10800 11.6 -> 8.4 / 13.5 -> 11.6 (33 MB,
+// 4.0 TB/s); 1536 x 1536 7.1 -> 4.2 / 7.3 -> 5.3; 1536 x 32000 24.9 -> 18.4
+// (5.3 TB/s) / 25.9 -> 22.1; 768 x 5400 6.1 -> 4.6 / 6.1 -> 5.3.  One row of 8 or
+// 16 waves splitting K, or two column tiles a wave, were slower there (9.1,
+// 10.3 and 10.0 at 1536 x 10800).
+#include "m3_internal.hpp"
+#include "scan_common.hpp"
+
+namespace m3 {
+
+namespace {
+
+using namespace scan;
+
+template <int MT, int NT, int WK, int U>
+__global__ void __launch_bounds__(64 * WK)
+few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w,
+                const float *scale, const void *res, void *y) {
+    __shared__ __attribute__((aligned(16))) f32x4 part[WK][NT * MT][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const uint32_t n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+    const rsrc_t rx = make_rsrc(x, M * K * 2u), rw = make_rsrc(w, N * K * 2u);
+    const int nb = static_cast<int>(K / 64);
+    uint32_t ow[NT], ox[MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) ow[i] = ((n0 + 16 * i + c) * K + 16 * g) * 2u;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) ox[j] = ((m0 + 16 * j + c) * K + 16 * g) * 2u;
+
+    struct Group {
+        u32x4 w[U][NT][2], x[U][MT][2];
+    };
+    auto load = [&](int b, Group &d) {   // blocks b, b + WK, ... of this wave
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kb = b + u * WK;
+            if (kb >= nb) break;
+            const uint32_t o = static_cast<uint32_t>(kb) * 128u;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                d.w[u][i][0] = bld16(rw, ow[i] + o);
+                d.w[u][i][1] = bld16(rw, ow[i] + o + 16);
+            }
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                d.x[u][j][0] = bld16(rx, ox[j] + o);
+                d.x[u][j][1] = bld16(rx, ox[j] + o + 16);
+            }
+        }
+    };
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mul = [&](int b, const Group &d) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (b + u * WK >= nb) break;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j)
+                        acc[i][j] = mfma_bf16(__builtin_bit_cast(bf16x8, d.w[u][i][h]),
+                                              __builtin_bit_cast(bf16x8, d.x[u][j][h]), acc[i][j]);
+        }
+    };
+    Group d0, d1;
+    load(wave, d0);
+#pragma unroll 1
+    for (int b = wave; b < nb; b += 2 * U * WK) {
+        load(b + U * WK, d1);
+        mul(b, d0);
+        load(b + 2 * U * WK, d0);
+        mul(b + U * WK, d1);
+    }
+
+    // ---- the waves' sums, then lane (c, g) of tile (i, j) holds y[m][n .. n + 3]
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) part[wave][i * MT + j][lane] = acc[i][j];
+    __syncthreads();
+    for (int t = wave; t < NT * MT; t += WK) {
+        f32x4 v = part[0][t][lane];
+#pragma unroll
+        for (int q = 1; q < WK; ++q) v += part[q][t][lane];
+        const uint32_t n = n0 + 16 * (t / MT) + 4 * g, m = m0 + 16 * (t % MT) + c;
+        if (n >= N || m >= M) continue;
+        if (scale) v = v * *reinterpret_cast<const f32x4 *>(scale + n);
+        const size_t o = static_cast<size_t>(m) * N + n;
+        if (res) {
+            const u32x2 rv = *reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(res) + o);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                v[r] += __uint_as_float((r & 1) ? (rv[r >> 1] & 0xFFFF0000u) : (rv[r >> 1] << 16));
+        }
+        *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(y) + o) =
+            u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+}
+
+template <int MT, int NT, int WK, int U>
+void launch_cfg(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w, const float *scale,
+                const void *res, void *y, hipStream_t s) {
+    const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT));
+    hipLaunchKernelGGL((few_rows_kernel<MT, NT, WK, U>), grid, dim3(64 * WK), 0, s, M, K, N, x, w,
+                       scale, res, y);
+}
+
+// The x a call reads from L2, every row once per workgroup of 32 columns.
+size_t x_reads(size_t m, size_t k, size_t n) { return (n + 31) / 32 * m * k * 2; }
+
+}  // namespace
+
+// Where the lines lie (us per call, this kernel against the other route):
+// - to 16 rows it is the faster one at every size (above).
+// - 17 to 32 rows, under 4096 columns: 1536 x 1536 5.8 against 7.6 (17 rows),
+//   6.6 against 7.6 (32); 768 x 768 4.4 against 4.9 (32).  At 48 rows 8.6
+//   against 7.7 and 5.4 against 4.9: x's re-reads by every column tile take
+//   over, and skinny_gemm.hip's tiles hold more rows.
+// - from 4096 columns on, x's re-reads bound it: 768 x 5400 (8 MB of them at
+//   32 rows, 17 at 64) 5.8 against 7.2 and 7.4 against 7.7, 768 x 6192 (19 MB
+//   at 64) 7.6 against 7.8; 1536 x 10800 (33 MB at 32 rows) 15.7 against 13.5.
+bool few_rows_supported(size_t m, size_t k, size_t n, const void *x, const void *w, bool w_transposed,
+                        const float *scale, const void *res, const void *y) {
+    auto al = [](const void *p, uintptr_t b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
+    if (!w_transposed || m < 1 || k < 64 || k % 64 != 0 || n < 16 || n % 4 != 0) return false;
+    if (k * n * 2 >= (size_t(1) << 31) || !al(x, 16) || !al(w, 16) || !al(scale, 16) || !al(res, 8) ||
+        !al(y, 8))
+        return false;
+    if (m <= 16) return true;
+    if (n < 4096) return m <= 32;
+    return m <= 64 && x_reads(m, k, n) <= (size_t(20) << 20);
+}
+
+hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const void *w,
+                           const float *scale, const void *res, void *y, hipStream_t s) {
+    const uint32_t M = static_cast<uint32_t>(m), K = static_cast<uint32_t>(k),
+                   N = static_cast<uint32_t>(n);
+    // two column tiles a wave halve x's re-reads of wide products (16 rows at
+    // 1536 x 10800 11.6 against 12.5, at 1536 x 32000 22.1 against 27.5); up
+    // to four rows there is next to nothing to re-read (10.0 against 8.4)
+    if (m <= 16 && (m <= 4 || n < 4096))
+        launch_cfg<1, 1, 4, 3>(M, K, N, x, w, scale, res, y, s);
+    else if (m <= 16)
+        launch_cfg<1, 2, 4, 2>(M, K, N, x, w, scale, res, y, s);
+    else if (m <= 32 && n < 4096)
+        launch_cfg<2, 1, 4, 2>(M, K, N, x, w, scale, res, y, s);
+    else if (m <= 32)
+        launch_cfg<2, 2, 4, 2>(M, K, N, x, w, scale, res, y, s);
+    else
+        launch_cfg<4, 2, 8, 1>(M, K, N, x, w, scale, res, y, s);
+    return hipGetLastError();
+}
+
+}  // namespace m3

@@ -15,7 +15,9 @@
 //
 // Up to 512 rows and 4096 columns (K a multiple of 128, N of 8, 16-byte
 // aligned buffers) the product runs on the weight-streaming kernel of
-// skinny_gemm.hip instead, with the same epilogue.
+// skinny_gemm.hip instead, with the same epilogue; up to 16 rows, and up to 64
+// where few_rows_supported says, on the one of few_rows.hip (a transposed
+// weight, K a multiple of 64, N of 4).
 //
 // Plan choice follows the reference's tuned plans (tensor/matmul.rs:1636-1943:
 // timing probes once per shape): the first call for a shape asks hipBLASLt's
@@ -170,7 +172,9 @@ hipError_t launch_linear(size_t m, size_t k, size_t n, const void *x, const void
                          bool w_transposed, const float *col_scale, const void *residual, void *y,
                          void *workspace, size_t workspace_bytes, hipStream_t s) {
     if (m == 0 || n == 0) return hipSuccess;
-    // few rows (a decode step's tokens): the weight-streaming kernel
+    // few rows (a decode step's tokens): the weight-streaming kernels
+    if (few_rows_supported(m, k, n, x, w, w_transposed, col_scale, residual, y))
+        return launch_few_rows(m, k, n, x, w, col_scale, residual, y, s);
     if (skinny_gemm_supported(m, k, n, x, w, col_scale, residual, y))
         return launch_skinny_gemm(m, k, n, x, w, w_transposed, col_scale, residual, y, s);
     int dev = 0;
