@@ -51,7 +51,7 @@ __device__ __forceinline__ float rot_hi(float x1, float x2, float cs, float sn) 
 // Prologue shared by both bodies: angle advance, rotation of B and C into
 // LDS (rank-last [N][R] layout kept), x into LDS, and the coefficients.  bh
 // indexes the state, ib the inputs (bh except with in_bstride).
-template <typename T, bool FACT = false>
+template <typename T, bool FACT = false, int NT = kStepThreads>
 __device__ __forceinline__ void step_prologue(const StepLaunch &a, size_t bh, size_t ib,
                                               float *bt, float *ct, float *xs, float &alpha,
                                               float &beta, float &gamma, float *bpt = nullptr,
@@ -65,7 +65,7 @@ __device__ __forceinline__ void step_prologue(const StepLaunch &a, size_t bh, si
     const size_t bc_base = ib * N * R;
     const size_t bp_base = bh * N * R;
     if (a.theta != nullptr) {
-        for (size_t i = tid; i < half; i += kStepThreads) {
+        for (size_t i = tid; i < half; i += NT) {
             // phi = wrap(prev + dt * theta)   (fused.rs:1549-1553)
             const float prev = a.angle[bh * half + i];
             float raw = ld<T>(a.theta, ib * half + i) * step + prev;
@@ -100,13 +100,13 @@ __device__ __forceinline__ void step_prologue(const StepLaunch &a, size_t bh, si
         // odd N: the unpaired last component is not rotated (N is even whenever
         // theta is given; validation enforces it)
     } else {
-        for (size_t i = tid; i < N * R; i += kStepThreads) {
+        for (size_t i = tid; i < N * R; i += NT) {
             bt[i] = ld<T>(a.b, bc_base + i);
             ct[i] = ld<T>(a.c, bc_base + i);
             if constexpr (FACT) bpt[i] = ld<T>(a.b_prev, bp_base + i);
         }
     }
-    for (size_t i = tid; i < P * R; i += kStepThreads) {
+    for (size_t i = tid; i < P * R; i += NT) {
         xs[i] = ld<T>(a.x, ib * P * R + i);
         if constexpr (FACT) xps[i] = ld<T>(a.x_prev, bh * P * R + i);
     }
@@ -181,7 +181,7 @@ __device__ __forceinline__ void step_conv8(const MixerStepLaunch &m, size_t bq, 
 // lambda -- then step_prologue's angle advance, rotation and coefficients on
 // those values.  CONV: x, B and C through the causal convolution first
 // (step_conv8), which also writes the new history of this head's channels.
-template <int R, bool FACT, bool CONV>
+template <int R, bool FACT, bool CONV, int NT, bool EARLY>
 __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh, float *bt,
                                              float *ct, float *xs, float &alpha, float &beta,
                                              float &gamma, float *bpt, float *braw, float *craw,
@@ -207,6 +207,21 @@ __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh
     const int grp = h / per_group;
     const int nx = P * R / 8;
     const size_t C = static_cast<size_t>(din) + 2 * static_cast<size_t>(bcw);
+    // EARLY: what the second half of the prologue reads is loaded with the
+    // row, not after the barrier (half <= 64: one pair a thread)
+    float prev0 = 0.0f, bp0[FACT ? 2 * R : 1];
+    if constexpr (EARLY) {
+        if (a.theta != nullptr && tid < half) {
+            prev0 = a.angle[bh * half + tid];
+            if constexpr (FACT)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    bp0[r] = ld<bf16_t>(a.b_prev, bh * N * R + tid * R + r);
+                    bp0[R + r] = ld<bf16_t>(a.b_prev, bh * N * R + (tid + half) * R + r);
+                }
+        }
+    }
+    const float a_log = a.a_log[h];
     if (tid < 2 * lq) {
         // B (lanes 0 .. lq-1) and C (lq .. 2 lq-1): eight states of every rank
         const int which = tid / lq, q = tid - which * lq;
@@ -263,9 +278,9 @@ __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh
     const float lam = scal[1];
     const size_t bc_base = bh * N * R;
     if (a.theta != nullptr) {
-        for (int i = tid; i < half; i += kStepThreads) {
+        for (int i = tid; i < half; i += NT) {
             // phi = wrap(prev + dt * theta)   (fused.rs:1549-1553)
-            const float prev = a.angle[bh * half + i];
+            const float prev = EARLY ? prev0 : a.angle[bh * half + i];
             float raw = thv[i] * step + prev;
             float phi = wrap_angle(raw);
             a.angle[bh * half + i] = phi;
@@ -275,8 +290,9 @@ __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh
                 float ps, pc;
                 sincosf(prev, &ps, &pc);
                 for (int r = 0; r < R; ++r) {
-                    const float b1 = ld<bf16_t>(a.b_prev, bc_base + i * R + r);
-                    const float b2 = ld<bf16_t>(a.b_prev, bc_base + (i + half) * R + r);
+                    const float b1 = EARLY ? bp0[r] : ld<bf16_t>(a.b_prev, bc_base + i * R + r);
+                    const float b2 = EARLY ? bp0[R + r]
+                                           : ld<bf16_t>(a.b_prev, bc_base + (i + half) * R + r);
                     bpt[i * R + r] = rot_lo(b1, b2, pc, ps);
                     bpt[(i + half) * R + r] = rot_hi(b1, b2, pc, ps);
                 }
@@ -291,13 +307,13 @@ __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh
             }
         }
     } else {
-        for (int i = tid; i < N * R; i += kStepThreads) {
+        for (int i = tid; i < N * R; i += NT) {
             bt[i] = braw[i];
             ct[i] = craw[i];
             if constexpr (FACT) bpt[i] = ld<bf16_t>(a.b_prev, bc_base + i);
         }
     }
-    const float A = 0.0f - expf(a.a_log[h]);
+    const float A = 0.0f - expf(a_log);
     alpha = expf(step * A);
     beta = (1.0f - lam) * step * alpha;
     gamma = lam * step;
@@ -306,8 +322,12 @@ __device__ __forceinline__ void mix_prologue(const MixerStepLaunch &m, size_t bh
 // Vector body: N % 4 == 0 and G = N / 4 lanes per row with G a power of two
 // that divides 64.  Each lane owns four consecutive state columns of a row.
 // MIX: the fused mixer step (mix_prologue in, the gate out); CONV: its
-// convolution.
-template <typename T, int RK, bool FACT, bool MIX = false, bool CONV = false>
+// convolution.  NT threads; EARLY: the state's first rows, the gate's z and
+// the factored x are loaded before the prologue, so that every input of the
+// workgroup is in flight at once (step_form says where each form runs).  The
+// arithmetic is the same, result for result.
+template <typename T, int RK, bool FACT, bool MIX = false, bool CONV = false, int NT = kStepThreads,
+          bool EARLY = false>
 __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
                                               const MixerStepLaunch *m = nullptr) {
     extern __shared__ float smem[];
@@ -324,14 +344,61 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
     float *craw = braw + N * R;
     float *thv = craw + N * R;
     float *scal = thv + N / 2;
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int G = static_cast<int>(N / 4);          // lanes per row
+    const int rows_per_wave = 64 / G;
+    const int rows_per_pass = rows_per_wave * (NT / 64);
+    const int col4 = (lane % G) * 4;
+    const float dskip = a.d_skip ? a.d_skip[bh % a.heads] : 0.0f;
+    f32x4 *h4 = reinterpret_cast<f32x4 *>(a.h + bh * P * N);
+    f32x4 *u4 = reinterpret_cast<f32x4 *>(a.last_u + bh * P * N);
+    constexpr int kBatch = NT > kStepThreads ? 2 : 4;   // rows in flight per lane
+    const int base0 = wave * rows_per_wave + lane / G;
+    f32x4 hv[kBatch], lv[kBatch];
+    auto load_rows = [&](int base) {
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int p = base + k * rows_per_pass;
+            if (p < static_cast<int>(P)) {
+                const size_t idx = (static_cast<size_t>(p) * N + col4) / 4;
+                hv[k] = __builtin_nontemporal_load(&h4[idx]);
+                if constexpr (!FACT) lv[k] = __builtin_nontemporal_load(&u4[idx]);
+            }
+        }
+    };
+    // the gate's z of this head, and where its row goes
+    const uint16_t *z = nullptr;
+    if constexpr (MIX)
+        z = static_cast<const uint16_t *>(m->projected) + (bh / a.heads) * m->width +
+            (bh % a.heads) * P * R;
+    uint16_t zv[kBatch][R];
+    auto load_z = [&](int base) {
+        if constexpr (MIX && EARLY) {
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int p = base + k * rows_per_pass;
+                    if (p < static_cast<int>(P)) zv[k][r] = z[p * R + r];
+                }
+        }
+    };
+    if constexpr (EARLY) {
+        load_rows(base0);
+        load_z(base0);
+        if constexpr (FACT && MIX) {
+            for (size_t i = threadIdx.x; i < P * R; i += NT) xps[i] = ld<T>(a.x_prev, bh * P * R + i);
+        }
+    }
     float alpha, beta, gamma;
     if constexpr (MIX)
-        mix_prologue<R, FACT, CONV>(*m, bh, bt, ct, xs, alpha, beta, gamma, bpt, braw, craw, thv,
+        mix_prologue<R, FACT, CONV, NT, EARLY>(*m, bh, bt, ct, xs, alpha, beta, gamma, bpt, braw, craw, thv,
                                     scal);
     else
-        step_prologue<T, FACT>(a, bh, bh, bt, ct, xs, alpha, beta, gamma, bpt, xps);
-    if constexpr (FACT && MIX) {
-        for (size_t i = threadIdx.x; i < P * R; i += kStepThreads)
+        step_prologue<T, FACT, NT>(a, bh, bh, bt, ct, xs, alpha, beta, gamma, bpt, xps);
+    if constexpr (FACT && MIX && !EARLY) {
+        for (size_t i = threadIdx.x; i < P * R; i += NT)
             xps[i] = ld<T>(a.x_prev, bh * P * R + i);
     }
     __syncthreads();
@@ -341,25 +408,15 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
         T *xp = static_cast<T *>(a.x_prev) + bh * P * R;
         T *bp = static_cast<T *>(a.b_prev) + bh * N * R;
         if constexpr (MIX) {
-            for (size_t i = threadIdx.x; i < P * R; i += kStepThreads) xp[i] = from_f32<T>(xs[i]);
-            for (size_t i = threadIdx.x; i < N * R; i += kStepThreads) bp[i] = from_f32<T>(braw[i]);
+            for (size_t i = threadIdx.x; i < P * R; i += NT) xp[i] = from_f32<T>(xs[i]);
+            for (size_t i = threadIdx.x; i < N * R; i += NT) bp[i] = from_f32<T>(braw[i]);
         } else {
             const T *xb = static_cast<const T *>(a.x) + bh * P * R;
             const T *bb = static_cast<const T *>(a.b) + bh * N * R;
-            for (size_t i = threadIdx.x; i < P * R; i += kStepThreads) xp[i] = xb[i];
-            for (size_t i = threadIdx.x; i < N * R; i += kStepThreads) bp[i] = bb[i];
+            for (size_t i = threadIdx.x; i < P * R; i += NT) xp[i] = xb[i];
+            for (size_t i = threadIdx.x; i < N * R; i += NT) bp[i] = bb[i];
         }
     }
-
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int G = static_cast<int>(N / 4);          // lanes per row
-    const int rows_per_wave = 64 / G;
-    const int rows_per_pass = rows_per_wave * (kStepThreads / 64);
-    const int col4 = (lane % G) * 4;
-    const float dskip = a.d_skip ? a.d_skip[bh % a.heads] : 0.0f;
-    f32x4 *h4 = reinterpret_cast<f32x4 *>(a.h + bh * P * N);
-    f32x4 *u4 = reinterpret_cast<f32x4 *>(a.last_u + bh * P * N);
 
     // B~ columns this lane touches, hoisted out of the row loop.
     float bcol[4][R], ccol[4][R], pcol[4][FACT ? R : 1];
@@ -372,23 +429,14 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
             if constexpr (FACT) pcol[j][r] = bpt[(col4 + j) * R + r];
         }
 
-    constexpr int kBatch = 4;   // rows in flight per lane
-    for (int base = wave * rows_per_wave + lane / G; base < static_cast<int>(P);
-         base += rows_per_pass * kBatch) {
-        f32x4 hv[kBatch], lv[kBatch];
-        int rows[kBatch];
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-            rows[k] = base + k * rows_per_pass;
-            if (rows[k] < static_cast<int>(P)) {
-                size_t idx = (static_cast<size_t>(rows[k]) * N + col4) / 4;
-                hv[k] = __builtin_nontemporal_load(&h4[idx]);
-                if constexpr (!FACT) lv[k] = __builtin_nontemporal_load(&u4[idx]);
-            }
+    for (int base = base0; base < static_cast<int>(P); base += rows_per_pass * kBatch) {
+        if (!EARLY || base != base0) {
+            load_rows(base);
+            load_z(base);
         }
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-            const int p = rows[k];
+            const int p = base + k * rows_per_pass;
             // every lane of a row group shares `p`, so the guard is uniform per group
             const bool live = p < static_cast<int>(P);
             float ypart[R];
@@ -439,14 +487,12 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
                     // the gate: silu(z) * y with y rounded to bf16 first, as
                     // m3_mixer_gate reads it (models/mamba3.rs:468-477); y
                     // alone where a post-gate norm comes between
-                    const uint16_t *z = static_cast<const uint16_t *>(m->projected) +
-                                        (bh / a.heads) * m->width + (bh % a.heads) * P * R;
                     uint16_t *o = static_cast<uint16_t *>(m->out) + bh * P * R;
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
                         const uint16_t yb = mixm::to_bits(__builtin_fmaf(xs[p * R + r], dskip, ypart[r]));
-                        o[p * R + r] = m->gate ? mixm::to_bits(bf16_bits_to_f32(yb) *
-                                                               mixm::silu_fast(mixm::bf(z, p * R + r)))
+                        const float zf = EARLY ? bf16_bits_to_f32(zv[k][r]) : mixm::bf(z, p * R + r);
+                        o[p * R + r] = m->gate ? mixm::to_bits(bf16_bits_to_f32(yb) * mixm::silu_fast(zf))
                                                : yb;
                     }
                 } else {
@@ -460,10 +506,10 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
     }
 }
 
-template <typename T, int RK, bool FACT>
-__global__ void __launch_bounds__(kStepThreads)
+template <typename T, int RK, bool FACT, int NT, bool EARLY>
+__global__ void __launch_bounds__(NT)
 step_kernel_vec(StepLaunch a) {
-    step_body_vec<T, RK, FACT>(a, blockIdx.x);
+    step_body_vec<T, RK, FACT, false, false, NT, EARLY>(a, blockIdx.x);
 }
 
 // Several layers' steps in one launch: workgroup w steps (batch, head)
@@ -493,10 +539,10 @@ step_kernel_vec_layers(StepLaunch base, StepLayerTable t) {
     step_body_vec<T, RK, FACT>(a, blockIdx.x - l * per);
 }
 
-template <int RK, bool FACT, bool CONV>
-__global__ void __launch_bounds__(kStepThreads)
+template <int RK, bool FACT, bool CONV, int NT, bool EARLY>
+__global__ void __launch_bounds__(NT)
 mixer_step_kernel(MixerStepLaunch m) {
-    step_body_vec<bf16_t, RK, FACT, true, CONV>(m.s, blockIdx.x, &m);
+    step_body_vec<bf16_t, RK, FACT, true, CONV, NT, EARLY>(m.s, blockIdx.x, &m);
 }
 
 // Generic body for shapes the vector body does not cover (odd N, N > 256,
@@ -535,15 +581,97 @@ step_kernel_generic(StepLaunch a) {
     }
 }
 
+// The form of a launch of (batch, head) workgroups.  Measured on MI355X
+// (head_dim 64, us per layer, captured, caches from HBM; workgroups: 256
+// threads / the form taken).  A grid of at most one workgroup per CU is the
+// chain of its memory round trips, which kWide shortens (all loads first, two
+// rows a lane); to three per CU that still holds for kEarly; past it the
+// occupancy that the early loads cost counts for more, except for the fused
+// mixer step, whose prologue is the longest.
+//   mixer step, d_state 128:  24 9.95 / 5.63, 240 11.8 / 7.6 (kWide); 384 15.5 /
+//     13.1, 768 22.3 / 19.9, 1536 39.7 / 36.2, 6144 145.5 / 135.7 (kEarly); with
+//     the convolution 24 10.9 / 6.6, 6144 146 / 143 (kHalf; kEarly 147)
+//   mixer step, factored:     24 9.9 / 6.6, 768 15.9 / 13.4, 1536 23.5 / (24.0)
+//   step, d_state 128, f32:   24 7.9 / 5.0, 768 21.4 / 20.2, 6144 138.5 / 135.0
+//     (kHalf; kEarly 137.5); factored 24 7.9 / 5.1, 768 14.5 / 13.2, 1536 23.6 /
+//     (24.4); d_state 64 16 5.0 / 3.8, 512 9.3 / 7.5, 4096 48.6 / 46.8 (kHalf)
+//   step, rank 4:             24 16.6 / 13.1, 240 19.1 / 16.3 (kEarly; kWide spills
+//     from rank 4 on), 384 22.0 / (21.5), 768 28.8 / (31.7)
+enum class StepForm { kBase, kHalf, kEarly, kWide };   // 256, 512, 512 and 1024 threads
+StepForm step_form(const StepLaunch &a, bool mix, bool conv) {
+    const size_t wg = a.batch * a.heads, N = a.d_state;
+    const bool fact = a.last_u == nullptr;
+    if (wg <= 256) return a.rank <= 2 ? StepForm::kWide : StepForm::kEarly;
+    if (a.rank != 1) return StepForm::kBase;
+    if (wg <= 768) return StepForm::kEarly;
+    if (fact || (mix ? N != 128 : N < 64)) return StepForm::kBase;
+    return mix && !conv ? StepForm::kEarly : StepForm::kHalf;
+}
+
+template <typename T, int RK, bool FACT>
+void launch_vec_form(const StepLaunch &a, size_t smem, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned int>(a.batch * a.heads));
+    const StepForm f = step_form(a, false, false);
+    if constexpr (RK <= 2) {
+        if (f == StepForm::kWide) {
+            hipLaunchKernelGGL((step_kernel_vec<T, RK, FACT, 1024, true>), grid, dim3(1024), smem, s, a);
+            return;
+        }
+    }
+    if constexpr (RK == 1 && !FACT) {
+        if (f == StepForm::kHalf) {
+            hipLaunchKernelGGL((step_kernel_vec<T, RK, FACT, 512, false>), grid, dim3(512), smem, s, a);
+            return;
+        }
+    }
+    if (f == StepForm::kEarly)
+        hipLaunchKernelGGL((step_kernel_vec<T, RK, FACT, 512, true>), grid, dim3(512), smem, s, a);
+    else
+        hipLaunchKernelGGL((step_kernel_vec<T, RK, FACT, kStepThreads, false>), grid,
+                           dim3(kStepThreads), smem, s, a);
+}
 template <typename T, int RK>
 hipError_t launch_vec(const StepLaunch &a, size_t smem, hipStream_t s) {
     if (a.last_u == nullptr)
-        hipLaunchKernelGGL((step_kernel_vec<T, RK, true>), dim3(a.batch * a.heads),
-                           dim3(kStepThreads), smem, s, a);
+        launch_vec_form<T, RK, true>(a, smem, s);
     else
-        hipLaunchKernelGGL((step_kernel_vec<T, RK, false>), dim3(a.batch * a.heads),
-                           dim3(kStepThreads), smem, s, a);
+        launch_vec_form<T, RK, false>(a, smem, s);
     return hipGetLastError();
+}
+
+template <int RK, bool FACT, bool CONV>
+void launch_mix_form(const MixerStepLaunch &m, size_t smem, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned int>(m.s.batch * m.s.heads));
+    const StepForm f = step_form(m.s, true, CONV);
+    if constexpr (RK <= 2) {
+        if (f == StepForm::kWide) {
+            hipLaunchKernelGGL((mixer_step_kernel<RK, FACT, CONV, 1024, true>), grid, dim3(1024), smem, s, m);
+            return;
+        }
+    }
+    if constexpr (RK == 1 && !FACT && CONV) {
+        if (f == StepForm::kHalf) {
+            hipLaunchKernelGGL((mixer_step_kernel<RK, FACT, CONV, 512, false>), grid, dim3(512), smem, s, m);
+            return;
+        }
+    }
+    if (f == StepForm::kEarly)
+        hipLaunchKernelGGL((mixer_step_kernel<RK, FACT, CONV, 512, true>), grid, dim3(512), smem, s, m);
+    else
+        hipLaunchKernelGGL((mixer_step_kernel<RK, FACT, CONV, kStepThreads, false>), grid,
+                           dim3(kStepThreads), smem, s, m);
+}
+template <int RK>
+void launch_mix(const MixerStepLaunch &m, size_t smem, hipStream_t s) {
+    const bool fact = m.s.last_u == nullptr;
+    if (m.conv_k && fact)
+        launch_mix_form<RK, true, true>(m, smem, s);
+    else if (m.conv_k)
+        launch_mix_form<RK, false, true>(m, smem, s);
+    else if (fact)
+        launch_mix_form<RK, true, false>(m, smem, s);
+    else
+        launch_mix_form<RK, false, false>(m, smem, s);
 }
 
 template <typename T>
@@ -684,29 +812,13 @@ hipError_t launch_mixer_step(const MixerStepLaunch &m, hipStream_t stream) {
     const bool fact = a.last_u == nullptr;
     const size_t smem =
         ((fact ? 5 : 4) * N * R + (fact ? 2 : 1) * P * R + N / 2 + 2) * sizeof(float);
-    const dim3 grid(static_cast<unsigned int>(a.batch * a.heads));
-#define M3_MIX2(RK, CV)                                                                            \
-    if (fact)                                                                                      \
-        hipLaunchKernelGGL((mixer_step_kernel<RK, true, CV>), grid, dim3(kStepThreads), smem,      \
-                           stream, m);                                                             \
-    else                                                                                           \
-        hipLaunchKernelGGL((mixer_step_kernel<RK, false, CV>), grid, dim3(kStepThreads), smem,     \
-                           stream, m);
-#define M3_MIX(RK)                                                                                 \
-    if (m.conv_k) {                                                                                \
-        M3_MIX2(RK, true)                                                                          \
-    } else {                                                                                       \
-        M3_MIX2(RK, false)                                                                         \
-    }
     switch (R) {
-        case 1: M3_MIX(1) break;
-        case 2: M3_MIX(2) break;
-        case 4: M3_MIX(4) break;
-        case 8: M3_MIX(8) break;
+        case 1: launch_mix<1>(m, smem, stream); break;
+        case 2: launch_mix<2>(m, smem, stream); break;
+        case 4: launch_mix<4>(m, smem, stream); break;
+        case 8: launch_mix<8>(m, smem, stream); break;
         default: return hipErrorNotSupported;
     }
-#undef M3_MIX
-#undef M3_MIX2
     return hipGetLastError();
 }
 
