@@ -92,6 +92,17 @@ m3_status m3_linear_nt(size_t m, size_t k, size_t n, const void *x, const void *
                        const float *col_scale, const void *residual, void *y, void *workspace,
                        size_t workspace_bytes, void *stream);
 
+/* m3_rms_norm of x's rows (weight `gain` [k] f32 or NULL, `eps`), then
+ * m3_linear_nt of the normed rows, in one launch: RmsNorm -> Linear of the
+ * stack (src/models/hybrid.rs:446-456) for the rows of a decode step.  The
+ * operand is bf16(x * gain) and the row's factor multiplies the f32 sums, so
+ * one rounding to bf16 stands where m3_rms_norm's output has one.  Up to 4
+ * rows, k a multiple of 64, n of 4, 16-byte aligned buffers; anything else is
+ * M3_ERR_UNSUPPORTED before any device work. */
+m3_status m3_norm_linear_nt(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,
+                            const void *w_t, const float *col_scale, const void *residual, void *y,
+                            void *stream);
+
 /* Shapes of one mixer (SsmConfig fields, config.rs:84-128). */
 typedef struct m3_mixer_dims {
     size_t tokens;            /* batch * seq */

@@ -30,25 +30,43 @@ namespace {
 
 using namespace scan;
 
-template <int MT, int NT, int WK, int U>
+// NORM: x is RMS-normalised on the way (nn/norm.rs:95-105), x rsqrt(mean x^2 +
+// eps) gain.  The operand is bf16(x gain); the row's factor, known only when
+// all of K has been read, multiplies the sums in f32: as many roundings as the
+// norm's own bf16 output has.  The waves form the operand's rows in LDS while
+// the first weights are on their way.  Measured (us, a norm and a product
+// against this, K x N at 1 / 4 rows): 1536 x 10800 11.2 -> 9.8 / 12.0 -> 10.7,
+// 1536 x 32000 21.1 -> 20.3 / 22.4 -> 21.9, 768 x 5400 6.7 -> 5.0 / 7.1 -> 6.0.
+// Past four rows forming them in every workgroup costs what the norm's launch
+// does (8 rows 7.0 -> 7.5 at 768 x 5400).  Scaling the lanes' own x registers
+// instead, sixteen lanes a row for one live row, took 15.2 us a call over a
+// decode step's projections against 12.2.
+constexpr uint32_t kNormRows = 4;
+template <int MT, int NT, int WK, int U, bool NORM>
 __global__ void __launch_bounds__(64 * WK)
-few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w,
-                const float *scale, const void *res, void *y) {
+few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const float *gain, float eps,
+                const void *w, const float *scale, const void *res, void *y) {
+    static_assert(!NORM || MT == 1, "the normed rows are one tile's");
+    extern __shared__ __attribute__((aligned(16))) unsigned char xs[];   // NORM: [M][2 K + 16]
     __shared__ __attribute__((aligned(16))) f32x4 part[WK][NT * MT][64];
+    __shared__ float squares[NORM ? WK : 1][kNormRows];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
     const uint32_t n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
     const rsrc_t rx = make_rsrc(x, M * K * 2u), rw = make_rsrc(w, N * K * 2u);
     const int nb = static_cast<int>(K / 64);
+    const uint32_t pitch = 2 * K + 16;   // of a row in LDS
     uint32_t ow[NT], ox[MT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) ow[i] = ((n0 + 16 * i + c) * K + 16 * g) * 2u;
 #pragma unroll
-    for (int j = 0; j < MT; ++j) ox[j] = ((m0 + 16 * j + c) * K + 16 * g) * 2u;
+    for (int j = 0; j < MT; ++j)
+        ox[j] = NORM ? min(static_cast<uint32_t>(c), M - 1) * pitch + 32 * g
+                     : ((m0 + 16 * j + c) * K + 16 * g) * 2u;
 
     struct Group {
-        u32x4 w[U][NT][2], x[U][MT][2];
+        u32x4 w[U][NT][2], x[U][NORM ? 1 : MT][2];
     };
     auto load = [&](int b, Group &d) {   // blocks b, b + WK, ... of this wave
 #pragma unroll
@@ -61,11 +79,12 @@ few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w
                 d.w[u][i][0] = bld16(rw, ow[i] + o);
                 d.w[u][i][1] = bld16(rw, ow[i] + o + 16);
             }
+            if constexpr (!NORM)
 #pragma unroll
-            for (int j = 0; j < MT; ++j) {
-                d.x[u][j][0] = bld16(rx, ox[j] + o);
-                d.x[u][j][1] = bld16(rx, ox[j] + o + 16);
-            }
+                for (int j = 0; j < MT; ++j) {
+                    d.x[u][j][0] = bld16(rx, ox[j] + o);
+                    d.x[u][j][1] = bld16(rx, ox[j] + o + 16);
+                }
         }
     };
     f32x4 acc[NT][MT];
@@ -76,19 +95,69 @@ few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w
     auto mul = [&](int b, const Group &d) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (b + u * WK >= nb) break;
+            const int kb = b + u * WK;
+            if (kb >= nb) break;
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int i = 0; i < NT; ++i)
+                for (int j = 0; j < MT; ++j) {
+                    u32x4 xv;
+                    if constexpr (NORM)
+                        xv = *reinterpret_cast<const u32x4 *>(xs + ox[j] + kb * 128 + 16 * h);
+                    else
+                        xv = d.x[u][j][h];
 #pragma unroll
-                    for (int j = 0; j < MT; ++j)
+                    for (int i = 0; i < NT; ++i)
                         acc[i][j] = mfma_bf16(__builtin_bit_cast(bf16x8, d.w[u][i][h]),
-                                              __builtin_bit_cast(bf16x8, d.x[u][j][h]), acc[i][j]);
+                                              __builtin_bit_cast(bf16x8, xv), acc[i][j]);
+                }
         }
     };
     Group d0, d1;
-    load(wave, d0);
+    float sq[kNormRows] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (NORM) {
+        // eight k of every row a thread; the rows and the gain are asked for
+        // before the weights, which arrive in order behind them
+        constexpr uint32_t STEP = 64 * WK * 8;
+        u32x4 v[kNormRows];
+        f32x4 gn[2];
+        auto load_rows = [&](uint32_t i) {   // rows past M read as zeros
+            gn[0] = gn[1] = f32x4{1.f, 1.f, 1.f, 1.f};
+            if (gain != nullptr && i < K) {
+                gn[0] = *reinterpret_cast<const f32x4 *>(gain + i);
+                gn[1] = *reinterpret_cast<const f32x4 *>(gain + i + 4);
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kNormRows; ++r) v[r] = bld16(rx, (r * K + i) * 2u);
+        };
+        auto form_rows = [&](uint32_t i) {
+#pragma unroll
+            for (uint32_t r = 0; r < kNormRows; ++r) {
+                if (r >= M || i >= K) continue;
+                u32x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = __uint_as_float(v[r][e] << 16);
+                    const float hi = __uint_as_float(v[r][e] & 0xFFFF0000u);
+                    sq[r] = __builtin_fmaf(lo, lo, sq[r]);
+                    sq[r] = __builtin_fmaf(hi, hi, sq[r]);
+                    o[e] = pack_bf16x2(lo * gn[e >> 1][2 * (e & 1)], hi * gn[e >> 1][2 * (e & 1) + 1]);
+                }
+                *reinterpret_cast<u32x4 *>(xs + r * pitch + i * 2) = o;
+            }
+        };
+        uint32_t i = tid * 8;
+        load_rows(i);
+        load(wave, d0);
+        form_rows(i);
+        for (i += STEP; i < K; i += STEP) {
+            load_rows(i);
+            form_rows(i);
+        }
+        __syncthreads();
+    } else {
+        load(wave, d0);
+    }
 #pragma unroll 1
     for (int b = wave; b < nb; b += 2 * U * WK) {
         load(b + U * WK, d1);
@@ -102,11 +171,27 @@ few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w
     for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int j = 0; j < MT; ++j) part[wave][i * MT + j][lane] = acc[i][j];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int r = 0; r < static_cast<int>(kNormRows); ++r) {
+            const float ss = group_sum(sq[r], 64);
+            if (lane == 0) squares[wave][r] = ss;
+        }
+    }
     __syncthreads();
+    float norm = 1.0f;
+    if constexpr (NORM) {
+        const int row = min(c, static_cast<int>(kNormRows) - 1);
+        float ss = squares[0][row];
+#pragma unroll
+        for (int q = 1; q < WK; ++q) ss += squares[q][row];
+        norm = 1.0f / sqrtf(ss / static_cast<float>(K) + eps);
+    }
     for (int t = wave; t < NT * MT; t += WK) {
         f32x4 v = part[0][t][lane];
 #pragma unroll
         for (int q = 1; q < WK; ++q) v += part[q][t][lane];
+        if constexpr (NORM) v = v * norm;
         const uint32_t n = n0 + 16 * (t / MT) + 4 * g, m = m0 + 16 * (t % MT) + c;
         if (n >= N || m >= M) continue;
         if (scale) v = v * *reinterpret_cast<const f32x4 *>(scale + n);
@@ -122,12 +207,12 @@ few_rows_kernel(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w
     }
 }
 
-template <int MT, int NT, int WK, int U>
+template <int MT, int NT, int WK, int U, bool NORM = false>
 void launch_cfg(uint32_t M, uint32_t K, uint32_t N, const void *x, const void *w, const float *scale,
-                const void *res, void *y, hipStream_t s) {
+                const void *res, void *y, hipStream_t s, const float *gain = nullptr, float eps = 0.0f) {
     const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT));
-    hipLaunchKernelGGL((few_rows_kernel<MT, NT, WK, U>), grid, dim3(64 * WK), 0, s, M, K, N, x, w,
-                       scale, res, y);
+    hipLaunchKernelGGL((few_rows_kernel<MT, NT, WK, U, NORM>), grid, dim3(64 * WK),
+                       NORM ? M * (2 * K + 16) : 0, s, M, K, N, x, gain, eps, w, scale, res, y);
 }
 
 // The x a call reads from L2, every row once per workgroup of 32 columns.
@@ -173,6 +258,23 @@ hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const vo
         launch_cfg<2, 2, 4, 2>(M, K, N, x, w, scale, res, y, s);
     else
         launch_cfg<4, 2, 8, 1>(M, K, N, x, w, scale, res, y, s);
+    return hipGetLastError();
+}
+
+bool norm_few_rows_supported(size_t m, size_t k, size_t n, const void *x, const float *gain,
+                             const void *w, const float *scale, const void *res, const void *y) {
+    // (the rows' copies in LDS, beside the partial sums)
+    return m <= kNormRows && m * (2 * k + 16) <= (size_t(50) << 10) &&
+           reinterpret_cast<uintptr_t>(gain) % 16 == 0 &&
+           few_rows_supported(m, k, n, x, w, true, scale, res, y);
+}
+
+hipError_t launch_norm_few_rows(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,
+                                const void *w, const float *scale, const void *res, void *y,
+                                hipStream_t s) {
+    const uint32_t M = static_cast<uint32_t>(m), K = static_cast<uint32_t>(k),
+                   N = static_cast<uint32_t>(n);
+    launch_cfg<1, 1, 4, 3, true>(M, K, N, x, w, scale, res, y, s, gain, eps);
     return hipGetLastError();
 }
 

@@ -241,6 +241,12 @@ bool few_rows_supported(size_t m, size_t k, size_t n, const void *x, const void 
                         const float *scale, const void *res, const void *y);
 hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const void *w,
                            const float *scale, const void *res, void *y, hipStream_t s);
+// The same after an RMSNorm of x's rows (gain [k] or null), up to four rows.
+bool norm_few_rows_supported(size_t m, size_t k, size_t n, const void *x, const float *gain,
+                             const void *w, const float *scale, const void *res, const void *y);
+hipError_t launch_norm_few_rows(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,
+                                const void *w, const float *scale, const void *res, void *y,
+                                hipStream_t s);
 hipError_t launch_linear(size_t m, size_t k, size_t n, const void *x, const void *w,
                          bool w_transposed, const float *col_scale, const void *residual, void *y,
                          void *workspace, size_t workspace_bytes, hipStream_t s);

@@ -95,6 +95,23 @@ m3_status m3_linear_nt(size_t m, size_t k, size_t n, const void *x, const void *
                        stream);
 }
 
+m3_status m3_norm_linear_nt(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,
+                            const void *w_t, const float *col_scale, const void *residual, void *y,
+                            void *stream) {
+    if (k == 0) return m3::api_fail(M3_ERR_SHAPE, "Linear with zero input features");
+    if (!(eps >= 0.0f)) return m3::api_fail(M3_ERR_CONFIG, "RmsNorm eps must be non-negative");
+    if (m == 0 || n == 0) return m3::api_ok();
+    if (x == nullptr || w_t == nullptr || y == nullptr)
+        return m3::api_fail(M3_ERR_ARGUMENT, "linear buffers are NULL");
+    if (!m3::norm_few_rows_supported(m, k, n, x, gain, w_t, col_scale, residual, y))
+        return m3::api_fail(M3_ERR_UNSUPPORTED, "the normed product covers up to 4 rows, k a "
+                            "multiple of 64, n of 4 and 16-byte aligned buffers (got %zu, %zu, %zu)",
+                            m, k, n);
+    return launched(m3::launch_norm_few_rows(m, k, n, x, gain, eps, w_t, col_scale, residual, y,
+                                             as_stream(stream)),
+                    "normed linear launch");
+}
+
 size_t m3_mixer_in_proj_width(const m3_mixer_dims *d) {
     if (d == nullptr) return 0;
     const size_t din = d->heads * d->head_dim * d->rank;

@@ -123,14 +123,14 @@ class Mamba3Lm:
             raise ConfigError(f"invalid configuration: cache has {len(cache)} entries but the "
                               f"stack has {len(self.layers)} layers")
         x = self.embed.lookup(ids)
+        if ids.shape[1] == 1:
+            for (norm, mixer), c in zip(self.layers, cache):
+                mixer.step_normed_(x, norm, c, residual=x, out=x)
+            return self.head.apply_normed(x, self.norm_f)
         normed = torch.empty_like(x)
-        single = ids.shape[1] == 1
         for i, (norm, mixer) in enumerate(self.layers):
             norm.apply(x, out=normed)
-            if single:
-                mixer.step_(normed, cache[i], residual=x, out=x)
-            else:
-                _, cache[i] = mixer.apply_with_state(normed, cache[i], residual=x, out=x)
+            _, cache[i] = mixer.apply_with_state(normed, cache[i], residual=x, out=x)
         return self.logits_from(self.norm_f.apply(x))
 
     def capture_decode(self, cache: List[MixerCache], batch: int) -> "DecodeGraph":
@@ -155,7 +155,8 @@ class DecodeGraph:
 
     def __init__(self, lm: Mamba3Lm, cache: List[MixerCache], batch: int):
         dev = cache[0].ssm.h.device
-        self.ids = torch.zeros((batch, 1), dtype=torch.int64, device=dev)
+        # int32, as the embedding reads them: the copy into it converts
+        self.ids = torch.zeros((batch, 1), dtype=torch.int32, device=dev)
         scratch = [c.clone() for c in cache]
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))

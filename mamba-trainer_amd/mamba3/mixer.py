@@ -282,7 +282,16 @@ class Mamba3Mixer:
                  self.a_log, sq(proj.theta), self.d_skip, cache.ssm)
         return self.finish(y.reshape(proj.x.shape), proj, residual=residual, out=out)
 
-    def _step_fused(self, input: torch.Tensor, cache: MixerCache, residual, out):
+    def step_normed_(self, input: torch.Tensor, norm: RmsNorm, cache: MixerCache,
+                     residual: Optional[torch.Tensor] = None,
+                     out: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """step_(norm.apply(input)): a stack's norm before its mixer, on the
+        input projection where the step is fused and the rows are few."""
+        y = self._step_fused(input, cache, residual, out, norm)
+        return self.step_(norm.apply(input), cache, residual, out) if y is None else y
+
+    def _step_fused(self, input: torch.Tensor, cache: MixerCache, residual, out,
+                    norm: Optional[RmsNorm] = None):
         """step_ through m3_mixer_step (prologue, state step and gate in one
         launch; the same results as the composed path bit for bit), or
         m3_mixer_step_conv with the convolution (its history updated in place
@@ -290,7 +299,7 @@ class Mamba3Mixer:
         launch); None where it does not apply (its shapes, a cache it cannot
         take, or an in-place history shared by several heads of a group)."""
         c = self.cfg
-        if input.dim() != 3 or input.shape[2] != c.d_model:
+        if input.dim() != 3 or input.shape[1] != 1 or input.shape[2] != c.d_model:
             return None
         B = input.shape[0]
         H, P, N, R = c.n_heads, c.head_dim, c.d_state, c.mode.rank()
@@ -330,7 +339,8 @@ class Mamba3Mixer:
             return None
         dims = self._dims(B)
         input = _bf16_dev(input, "mixer input")
-        projected = self.in_proj.apply(input)
+        projected = (self.in_proj.apply(input) if norm is None
+                     else self.in_proj.apply_normed(input, norm))
         gated = torch.empty((B, 1, c.d_inner()), dtype=torch.bfloat16, device=input.device)
         ptr = lambda t: None if t is None else t.data_ptr()
         ang = ptr(st.angle) if rot else None

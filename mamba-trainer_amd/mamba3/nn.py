@@ -167,6 +167,25 @@ class Linear:
             ws.numel(), _stream(x)))
         return y
 
+    def apply_normed(self, x: torch.Tensor, norm: RmsNorm) -> torch.Tensor:
+        """apply(norm.apply(x)): for the few rows of a decode step in one
+        launch (m3_norm_linear_nt), whose operand is rounded to bf16 before the
+        row's factor instead of after it; elsewhere as two calls."""
+        x = _bf16_dev(x, "Linear input")
+        m = x.numel() // max(x.shape[-1], 1)
+        if m <= 4 and x.shape[-1] == self.in_features == norm.dim:
+            y = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=torch.bfloat16,
+                            device=x.device)
+            st = _lib.lib().m3_norm_linear_nt(
+                m, self.in_features, self.out_features, x.data_ptr(),
+                None if norm.weight is None else norm.weight.data_ptr(), C.c_float(norm.eps),
+                self.codes_t.data_ptr(), None if self.scales is None else self.scales.data_ptr(),
+                None, y.data_ptr(), _stream(x))
+            if st != _lib.M3_ERR_UNSUPPORTED:
+                _lib.check(st)
+                return y
+        return self.apply(norm.apply(x))
+
 
 class Embedding:
     """embedding.rs: a [vocab, dim] table (Normal std 0.02), bf16 rows."""

@@ -63,3 +63,55 @@ def test_few_rows_repeat_bit_for_bit():
     assert torch.equal(a, b)
     # a row's result does not depend on the rows beside it
     assert torch.equal(lin.apply(x[2:5].contiguous())[1], lin.apply(x[3:4].contiguous())[0])
+
+
+@pytest.mark.parametrize("m,k,n,int8,gain", [(1, 64, 16, True, True), (1, 1536, 1540, True, True),
+                                             (4, 768, 5400, True, False), (3, 320, 4100, False, True),
+                                             (4, 2560, 516, True, True), (2, 512, 1000, True, True)])
+def test_normed_few_rows_against_f64(m, k, n, int8, gain):
+    """m3_norm_linear_nt: the operand bf16(x gain) is off by 2^-9 of each
+    product, the output by 2^-9 of itself, the f32 sum as above."""
+    from mamba3.nn import Linear, RmsNorm
+    rng = np.random.default_rng(m + k + n)
+    x = mo.bf16(rng.normal(0, 3, (m, k)))
+    x[0, : k // 2] = 0.0
+    g = rng.uniform(-1.5, 1.5, k).astype(np.float32)
+    w = rng.normal(0, 0.02, (k, n)).astype(np.float32)
+    lin = Linear(t_f32(w), int8_weights=int8)
+    norm = RmsNorm(k, torch.device("cuda"), weight=gain)
+    if gain:
+        norm.weight.copy_(t_f32(g))
+    if int8:
+        c, s = mo.quantize_int8_columns(w)
+        w_eff = c.astype(np.float64) * s
+    else:
+        w_eff = mo.bf16(w)
+    normed = mo.rms_norm(x, g if gain else None, 1e-5)
+    ref = normed @ w_eff
+    from mamba3 import _lib
+    before = _lib.lib().m3_launch_count()
+    y = lin.apply_normed(t_bf16(x), norm)
+    torch.cuda.synchronize()
+    assert _lib.lib().m3_launch_count() - before == 1
+    got = host(y)
+    bound = 2.0 ** -8 * np.abs(ref) + (2.0 ** -9 + (k + 4) * 2.0 ** -24) * (np.abs(normed) @ np.abs(w_eff))
+    assert np.all(np.abs(got - ref) <= bound), np.max(np.abs(got - ref) / bound)
+    # no further off than the two calls: both operands hold k independent
+    # roundings, whose norms differ by a few k^-1/2 (shorter rows say nothing)
+    if k < 500:
+        return
+    two = host(lin.apply(norm.apply(t_bf16(x))))
+    err = lambda a: np.linalg.norm(a - ref) / np.linalg.norm(ref)
+    assert err(got) <= 1.2 * err(two) + 1e-4
+
+
+def test_normed_rows_past_the_kernel_run_as_two_calls():
+    from mamba3 import _lib
+    from mamba3.nn import Linear, RmsNorm
+    lin = Linear(t_f32(np.random.default_rng(1).normal(0, 0.02, (128, 64)).astype(np.float32)))
+    norm = RmsNorm(128, torch.device("cuda"))
+    x = torch.randn(5, 1, 128, device="cuda").bfloat16()
+    before = _lib.lib().m3_launch_count()
+    y = lin.apply_normed(x, norm)
+    assert _lib.lib().m3_launch_count() - before == 2 and y.shape == (5, 1, 64)
+    assert torch.equal(y, lin.apply(norm.apply(x)))
