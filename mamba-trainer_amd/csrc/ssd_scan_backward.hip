@@ -145,6 +145,18 @@ __device__ __forceinline__ float clamp_exp(float d) {
     return expf(fminf(fmaxf(d, -60.0f), 0.0f));
 }
 
+// dt A on a 2^-14 grid and what is left of it (with the product's own
+// rounding): prefix sums of the grid part are exact in f32 up to 2^10, and
+// those of the rest some 2^-40 off, so the difference of two prefixes is as
+// exact as the step between them.  One f32 prefix of a long, fast-decaying
+// chunk (about -50 at its end) holds 4e-6, which came out whole in every decay
+// factor of its last rows and in da_log.
+__device__ __forceinline__ void split_decay(float dt, float A, float &hi, float &lo) {
+    const float v = dt * A;
+    hi = rintf(v * 16384.0f) * (1.0f / 16384.0f);
+    lo = (v - hi) + __builtin_fmaf(dt, A, -v);
+}
+
 template <bool PRECISE>
 __device__ __forceinline__ void sincos_any(float x, float &s, float &c) {
     if constexpr (PRECISE) {
@@ -243,11 +255,10 @@ struct Smem {
     static constexpr int AP = NH + 3;
     float acs[QT * AP], asn[QT * AP];
     float phi_end[NH];      // the chunk's angle total per pair
-    float dtv[QT], lamv[QT], acum[QT], gw[QT], ww[QT], eac[QT], ebar[QT], wbar[QT];
+    float dtv[QT], lamv[QT], acum[QT], aclo[QT], gw[QT], ww[QT], eac[QT], ebar[QT], wbar[QT];
     float rin[kRows], cinx[kRows], dwi[kRows], qv[kRows], rcr[kRows];
     float dgv[QT], dal[QT];
-    float red[32];
-    float gs, pdsum;
+    float red[48];
 };
 
 // Per-token scalars, the in-chunk angles, and (X, dY) / (B~, C~) as asked.
@@ -354,8 +365,14 @@ __device__ void stage(const ScanLaunch &a, const BwdArgs &g, S &sm, size_t bh, i
         sm.ww[tid] = lam * dt + (1.0f - lamn) * dtn;    // fused.rs:2496-2498
     }
     if (wave == 0) {
-        const float v = seg_scan<64>(tid < QT ? dt * A : 0.0f);
-        if (lane < QT) sm.acum[lane] = v;
+        float hi, lo;
+        split_decay(tid < QT ? dt : 0.0f, A, hi, lo);
+        hi = seg_scan<64>(hi);
+        lo = seg_scan<64>(lo);
+        if (lane < QT) {
+            sm.acum[lane] = hi;
+            sm.aclo[lane] = lo;
+        }
     }
     __syncthreads();
     if (rot) {
@@ -382,9 +399,9 @@ __device__ void stage(const ScanLaunch &a, const BwdArgs &g, S &sm, size_t bh, i
     }
     __syncthreads();
     if (tid < QT) {
-        const float e = sm.acum[QT - 1];
-        sm.eac[tid] = clamp_exp(sm.acum[tid]);
-        sm.ebar[tid] = clamp_exp(e - sm.acum[tid]);
+        const float hi = sm.acum[tid], lo = sm.aclo[tid];
+        sm.eac[tid] = clamp_exp(hi + lo);
+        sm.ebar[tid] = clamp_exp((sm.acum[QT - 1] - hi) + (sm.aclo[QT - 1] - lo));
         sm.wbar[tid] = sm.ebar[tid] * sm.ww[tid];
     }
     // ---- rotation by the negative in-chunk angle (fused.rs:610-617) into LDS
@@ -438,7 +455,7 @@ struct PassSmem {
     // per chunk parity: cos / sin of the in-chunk angle [token][pair], the
     // token scalars, the decay prefix and the per-token scale
     float acs[2][QT * AP], asn[2][QT * AP];
-    float dtv[2][QT], acum[2][QT], ww[2][QT], scal[2][QT];
+    float dtv[2][QT], acum[2][QT], aclo[2][QT], ww[2][QT], scal[2][QT];
     float phi[16];           // the sequence's angle total per pair (reverse pass)
     float red[16];
 };
@@ -555,8 +572,14 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             sm.ww[sb][tid] = d.lam * d.dt + (1.0f - d.lamn) * d.dtn;
         }
         if (wave == 0) {
-            const float v = seg_scan<64>(tid < QT ? d.dt * A : 0.0f);
-            if (lane < QT) sm.acum[sb][lane] = v;
+            float hi, lo;
+            split_decay(tid < QT ? d.dt : 0.0f, A, hi, lo);
+            hi = seg_scan<64>(hi);
+            lo = seg_scan<64>(lo);
+            if (lane < QT) {
+                sm.acum[sb][lane] = hi;
+                sm.aclo[sb][lane] = lo;
+            }
         }
     };
     // the in-chunk angle of this workgroup's pairs and its cos / sin; per
@@ -578,9 +601,10 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             }
         }
         if (tid < QT) {
-            const float et = sm.acum[sb][QT - 1];
-            sm.scal[sb][tid] = FWD ? clamp_exp(et - sm.acum[sb][tid]) * sm.ww[sb][tid]
-                                   : clamp_exp(sm.acum[sb][tid]);
+            const float hi = sm.acum[sb][tid], lo = sm.aclo[sb][tid];
+            sm.scal[sb][tid] = FWD ? clamp_exp((sm.acum[sb][QT - 1] - hi) + (sm.aclo[sb][QT - 1] - lo)) *
+                                         sm.ww[sb][tid]
+                                   : clamp_exp(hi + lo);
         }
     };
     // rotation by the negative in-chunk angle (fused.rs:610-617) into LDS;
@@ -611,7 +635,7 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             if constexpr (!FWD) v *= sm.scal[sb][t];
             sm.Xs[(pr / R) * LDR + t * R + pr % R] = v;
         }
-        e = clamp_exp(sm.acum[sb][QT - 1]);
+        e = clamp_exp(sm.acum[sb][QT - 1] + sm.aclo[sb][QT - 1]);
     };
     // U^T (V^T) at this lane's (n, p): A(m = n, k = rho), B(k = rho, col = p);
     // the rotation by the chunk's angle totals, the in-chunk angles of its
@@ -972,6 +996,7 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
     // diagonal's dg sums, and off it L = dM o M (row sums, column sums) and
     // the dw sums
     static_assert(kRows == 32 || kRows == 64, "band rows");
+    float asum = 0.0f;   // sum of L (alpha_t - alpha_s), this thread's share
     for (int e0 = 0; e0 < kRows * kRows; e0 += kBT) {
         const int e = e0 + tid, t = e / kRows, s = e % kRows;
         const int tt = t / R, ts = s / R;
@@ -980,7 +1005,8 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
             float m = 0.0f, d = 0.0f;
             if (tt >= ts) {
                 const float cb = sm.Ms[t * LM + s], dm = sm.Ds[t * LM + s];
-                const float E = clamp_exp(sm.acum[tt] - sm.acum[ts]);
+                const float step = (sm.acum[tt] - sm.acum[ts]) + (sm.aclo[tt] - sm.aclo[ts]);
+                const float E = clamp_exp(step);
                 const float K = (tt == ts ? sm.gw[ts] : sm.ww[ts]) * E;
                 m = cb * K;
                 d = dm * K;
@@ -989,6 +1015,7 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
                 } else {
                     lam = dm * m;
                     dwe = dm * cb * E;
+                    asum = __builtin_fmaf(lam, step, asum);
                 }
             }
             sm.Ms[t * LM + s] = m;
@@ -1076,9 +1103,11 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
         }
         gsum = group_sum(gsum, 64);
         dsum = group_sum(dsum, 64);
+        asum = group_sum(asum, 64);
         if (lane == 0) {
             sm.red[wave] = gsum;
             sm.red[16 + wave] = dsum;
+            sm.red[32 + wave] = asum;
         }
     }
     static_assert(kWaves <= 16, "block reduction slots");
@@ -1091,14 +1120,25 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
         if (lane == 0) w.pd[bhk] = ds;
         // the alpha_E terms of the last row: sum over rows of wbar q
         const float e = group_sum(lane < kRows ? sm.qv[lane] * sm.wbar[lane / R] : 0.0f, 64);
-        float d = 0.0f, dw = 0.0f;
+        // da_log's share (a = -e^{a_log} dt, so da_log = sum of a da): every
+        // term weighs the decay it crossed, alpha_t for the carry-in, alpha_E -
+        // alpha_s for the state, alpha_E for what passes through.  The sum of
+        // dt da, whose cumsums cancel most of each row and column sum, was off
+        // by up to 1.3e-5 in chunks of 64 rows.
+        const float alt = tid < QT ? sm.acum[tid] + sm.aclo[tid] : 0.0f;
+        const float ale = sm.acum[QT - 1] + sm.aclo[QT - 1];
+        const float toe = tid < QT ? (sm.acum[QT - 1] - sm.acum[tid]) + (sm.aclo[QT - 1] - sm.aclo[tid]) : 0.0f;
+        float d = 0.0f, dw = 0.0f, pa = 0.0f;
         if (tid < QT) {
             for (int r = 0; r < R; ++r) {
                 const int row = tid * R + r;
+                pa += sm.rcr[row] * alt + sm.qv[row] * sm.wbar[tid] * toe;
                 d += sm.rin[row] - sm.cinx[row] + sm.rcr[row] - sm.qv[row] * sm.wbar[tid];
                 dw += sm.dwi[row] + sm.qv[row] * sm.ebar[tid];
             }
         }
+        pa = group_sum(pa + (lane < kWaves ? sm.red[32 + lane] : 0.0f), 64);
+        if (lane == 0) w.pa[bhk] = pa + w.eda[bhk] * gs * ale;
         if (tid == QT - 1) d += e + w.eda[bhk] * gs;
         if (tid < QT) sm.dal[tid] = d;
         const size_t tg = static_cast<size_t>(ck) * QT + tid;
@@ -1241,10 +1281,6 @@ __global__ void __launch_bounds__(256) bwd_token_kernel(ScanLaunch a, BwdArgs g,
         g.ddt[tkx] = ddt;
         g.dlambda[tkx] = dlam;
     }
-    float asum = tk_live ? dt * da : 0.0f;
-    __shared__ float red[16];
-    asum = block_sum(asum, red);
-    if (threadIdx.x == 0) w.pa[bhk] = asum;
 }
 
 // ---------------------------------------------------------------- per head
@@ -1252,7 +1288,6 @@ __global__ void __launch_bounds__(256) bwd_head_kernel(ScanLaunch a, BwdArgs g, 
     __shared__ float red[16];
     const size_t hh = blockIdx.x;
     const size_t H = a.heads;
-    const float A = 0.0f - expf(a.a_log[hh]);
     float sa = 0.0f, sd = 0.0f;
     const size_t n = a.batch * static_cast<size_t>(nck);
     for (size_t j = threadIdx.x; j < n; j += blockDim.x) {
@@ -1264,7 +1299,7 @@ __global__ void __launch_bounds__(256) bwd_head_kernel(ScanLaunch a, BwdArgs g, 
     sa = block_sum(sa, red);
     sd = block_sum(sd, red + 8);
     if (threadIdx.x == 0) {
-        g.da_log[hh] = A * sa;     // A = -exp(a_log): dA/da_log = A
+        g.da_log[hh] = sa;
         if (g.dd_skip != nullptr) g.dd_skip[hh] = sd;
     }
 }
