@@ -267,8 +267,8 @@ typedef struct m3_scan_grads {
  * m3_scan_backward_workspace_bytes(in) bytes, 256-byte aligned).  The forward
  * chunk states are recomputed; the forward outputs are not needed.  The
  * chunk kernels take head_dim 64, d_state 64/128, rank 1/2/4 with aligned
- * buffers; their partial sums inside a workgroup are accumulated with LDS
- * atomics, so repeated calls agree to f32 rounding, not bit for bit.  Small
+ * buffers; every sum has a fixed order, so repeated calls agree bit for bit.
+ * Small
  * heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens on) run
  * them on zero-padded copies in the workspace.  Other shapes (and alignments) take the reverse mode of the recurrence token by
  * token, one workgroup per sequence with states recomputed from checkpoints

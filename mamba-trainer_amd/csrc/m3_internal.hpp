@@ -135,10 +135,6 @@ hipError_t launch_scan_chunked(const ScanLaunch &a, void *workspace, hipStream_t
 // fused single launch (bf16, rank 1, up to three rounds of its workgroups), 3
 // otherwise.
 int scan_chunked_launches(const ScanLaunch &a);
-// Rows (token, rank) per chunk of the backward: 32, or 64 for bf16 storage
-// with d_state 64 (whose 16-byte staging needs the longer chunk).
-inline int scan_backward_rows(const ScanLaunch &a) { return (a.bf16 && a.d_state == 64) ? 64 : 32; }
-
 // Backward of the scan (mamba3_scan mode, the chunk-parallel shapes): the
 // gradients of the loss given dL/dy (and optionally dL/dh, dL/dangle of the
 // outgoing state).  Outputs in the storage type where the input has it.

@@ -6,8 +6,7 @@
 // forward: head_dim 64, d_state 64/128, rank 1/2/4; f32 or bf16 storage,
 // f32 arithmetic (MFMA f32 16x16x4 over f32 operands in LDS).
 //
-// Chunks of 32 rows (token, rank); 64 for bf16 storage with d_state 64.  In
-// chunk k's own rotating frame, with alpha the in-chunk inclusive cumsum of a = dt A, K_ts = W_ts e^{alpha_t -
+// Chunks of 32 rows (token, rank).  In chunk k's own rotating frame, with alpha the in-chunk inclusive cumsum of a = dt A, K_ts = W_ts e^{alpha_t -
 // alpha_s} (W = g on the token diagonal, w below it), CB = C~ B~^T, M = CB o K,
 // wbar_s = e^{alpha_E - alpha_s} w_s, S_k the state entering the chunk and
 // Gh_k = dL/d(e_k S_k + U_k) = R(-Phi_k) G_{k+1}:
@@ -39,7 +38,8 @@ namespace m3 {
 namespace {
 
 constexpr int kP = 64;
-constexpr int kWaves = 16;
+constexpr int kRows = 32;    // (token, rank) rows of a chunk
+constexpr int kWaves = 8;    // of the chunk kernel
 constexpr int kBT = 64 * kWaves;
 
 struct BwdArgs {
@@ -133,14 +133,6 @@ __device__ __forceinline__ void st4(void *p, size_t i, f32x4 v) {
     }
 }
 
-// (p, n) of element e of a [p-tile][n-tile][lane][4] MFMA D-layout record
-__device__ __forceinline__ void dl_pn(int e, int ntn, int &p, int &n) {
-    const int r = e & 3, lane = (e >> 2) & 63, tile = e >> 8;
-    const int i = tile % ntn, pt = tile / ntn;
-    p = 16 * pt + (lane & 15);
-    n = 16 * i + 4 * (lane >> 4) + r;
-}
-
 __device__ __forceinline__ float clamp_exp(float d) {
     return expf(fminf(fmaxf(d, -60.0f), 0.0f));
 }
@@ -157,64 +149,88 @@ __device__ __forceinline__ void split_decay(float dt, float A, float &hi, float 
     lo = (v - hi) + __builtin_fmaf(dt, A, -v);
 }
 
-template <bool PRECISE>
-__device__ __forceinline__ void sincos_any(float x, float &s, float &c) {
-    if constexpr (PRECISE) {
-        sincosf(x, &s, &c);
+// Four consecutive elements of a row as they are loaded: 8 bytes of bf16
+// storage, 16 of f32.  An address off the 4-byte grid (a bf16 dy the caller
+// placed there) is read element by element.
+template <typename T> struct Raw4 { u32x2 q; };
+template <> struct Raw4<float> { u32x4 q; };
+__device__ __forceinline__ void ld4(Raw4<bf16_t> &d, rsrc_t r, uint32_t off, bool aligned = true) {
+    if (aligned) {
+        d.q = bld8(r, off);
     } else {
-        const float rev = wrap_angle(x) * 0.15915494309189533577f;
-        s = __builtin_amdgcn_sinf(rev);
-        c = __builtin_amdgcn_cosf(rev);
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            h[i] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off + 2 * i, 0, 0));
+        d.q = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    }
+}
+__device__ __forceinline__ void ld4(Raw4<float> &d, rsrc_t r, uint32_t off, bool = true) { d.q = bld16(r, off); }
+__device__ __forceinline__ void un4(const Raw4<bf16_t> &d, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        v[2 * i] = __uint_as_float(d.q[i] << 16);
+        v[2 * i + 1] = __uint_as_float(d.q[i] & 0xFFFF0000u);
+    }
+}
+__device__ __forceinline__ void un4(const Raw4<float> &d, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(d.q[i]);
+}
+// PN consecutive theta values (2 or 4)
+template <typename T, int PN>
+__device__ __forceinline__ void ldth(rsrc_t r, uint32_t off, uint32_t (&q)[PN]) {
+    if constexpr (sizeof(T) == 4) {
+        if constexpr (PN == 4) {
+            const u32x4 v = bld16(r, off);
+            q[0] = v[0]; q[1] = v[1]; q[2] = v[2]; q[3] = v[3];
+        } else {
+            const u32x2 v = bld8(r, off);
+            q[0] = v[0]; q[1] = v[1];
+        }
+    } else if constexpr (PN == 4) {
+        const u32x2 v = bld8(r, off);
+        q[0] = v[0]; q[1] = v[1];
+    } else {
+        q[0] = bld4(r, off);
+    }
+}
+template <typename T, int PN>
+__device__ __forceinline__ void unth(const uint32_t (&q)[PN], float (&v)[PN]) {
+#pragma unroll
+    for (int i = 0; i < PN; ++i)
+        v[i] = sizeof(T) == 4 ? __uint_as_float(q[i])
+                              : __uint_as_float((i & 1) ? (q[i >> 1] & 0xFFFF0000u) : (q[i >> 1] << 16));
+}
+
+// Elements e .. e + 3 (column e / R, rank e % R) of token t into a row-major
+// [row][pitch] tile of (token, rank) rows.
+template <int R>
+__device__ __forceinline__ void put4(float *tile, int pitch, int t, int e, const float (&v)[4]) {
+    if constexpr (R == 1) {
+        *reinterpret_cast<f32x4 *>(tile + t * pitch + e) = f32x4{v[0], v[1], v[2], v[3]};
+    } else if constexpr (R == 2) {
+        *reinterpret_cast<f32x2 *>(tile + (2 * t) * pitch + e / 2) = f32x2{v[0], v[2]};
+        *reinterpret_cast<f32x2 *>(tile + (2 * t + 1) * pitch + e / 2) = f32x2{v[1], v[3]};
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tile[(4 * t + r) * pitch + e / 4] = v[r];
     }
 }
 
-// D(16x16) += A(16 x K) B(K x 16) in f32: A(m, k) = a[m * am + k * ak],
-// B(k, n) = b[k * bk + n * bn]; lane (c, g) supplies A(c, k0+g), B(k0+g, c).
-// The operands of up to sixteen MFMAs are read from LDS together and the
-// MFMAs then issue back to back (one LDS wait per batch, not per MFMA).
-template <int K>
-__device__ __forceinline__ f32x4 mma_f32(const float *a, int am, int ak, const float *b, int bk,
-                                         int bn, f32x4 acc, int c, int g) {
-    static_assert(K % 4 == 0, "K");
-    constexpr int KB = K / 4 < 16 ? K / 4 : 16;
+// Inclusive scans over 32-lane segments of PN values at once.
+template <int PN>
+__device__ __forceinline__ void scan32(float (&v)[PN]) {
+    if constexpr (PN == 4) {
+        seg_scan4<32>(v[0], v[1], v[2], v[3]);
+    } else {
 #pragma unroll
-    for (int k0 = 0; k0 < K; k0 += 4 * KB) {
-        float av[KB], bv[KB];
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-            const int k = k0 + 4 * j + g;
-            av[j] = a[c * am + k * ak];
-            bv[j] = b[k * bk + c * bn];
-        }
-#pragma unroll
-        for (int j = 0; j < KB; ++j) acc = mfma_f32(av[j], bv[j], acc);
+        for (int i = 0; i < PN; ++i) v[i] = seg_scan<32>(v[i]);
     }
-    return acc;
 }
-
-// Two products sharing the B operand: D0 += A0 B, D1 += A1 B.
-template <int K>
-__device__ __forceinline__ void mma2_f32(const float *a0, const float *a1, int am, int ak,
-                                         const float *b, int bk, int bn, f32x4 &d0, f32x4 &d1,
-                                         int c, int g) {
-    static_assert(K % 4 == 0, "K");
-    constexpr int KB = K / 4 < 16 ? K / 4 : 16;
-#pragma unroll
-    for (int k0 = 0; k0 < K; k0 += 4 * KB) {
-        float av[KB], aw[KB], bv[KB];
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-            const int k = k0 + 4 * j + g;
-            av[j] = a0[c * am + k * ak];
-            aw[j] = a1[c * am + k * ak];
-            bv[j] = b[k * bk + c * bn];
-        }
-#pragma unroll
-        for (int j = 0; j < KB; ++j) {
-            d0 = mfma_f32(av[j], bv[j], d0);
-            d1 = mfma_f32(aw[j], bv[j], d1);
-        }
-    }
+// The wave's sum, in every lane (DPP; a shuffle tree is six LDS round trips).
+__device__ __forceinline__ float wave_sum(float v) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(seg_scan<64>(v)), 63));
 }
 
 __device__ __forceinline__ float block_sum(float v, float *red) {
@@ -226,205 +242,6 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
     float s = 0.0f;
     for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) s += red[w];
     return s;
-}
-
-// ---------------------------------------------------------------- staging
-template <int N, int R, int kRows>
-struct Smem {
-    static constexpr int QT = kRows / R, NH = N / 2, NTN = N / 16;
-    // Row pitches = 12 (mod 64 words) where LDS allows: an MFMA operand read
-    // as A(c, k0 + g) = m[c * pitch + k] then touches each bank at most once
-    // (64 banks) or twice (32), and read transposed, m[c + k * pitch], at most
-    // twice (three times).  The 64-row chunk keeps 4 (mod 64) to fit.
-    static constexpr int kPad = kRows == 64 ? 4 : 12;
-    static constexpr int LB = N + kPad;     // B~, C~ rows
-    static constexpr int LX = kP + kPad;    // X, dY rows
-    static constexpr int LM = kRows + kPad; // M, dCB rows
-    static constexpr int LS = N + kPad;     // S, Gh rows
-    // staged element (row rho, column n / p)
-    __device__ static int bi(int rho, int n) { return rho * LB + n; }
-    __device__ static int xi(int rho, int p) { return rho * LX + p; }
-    float Bs[kRows * LB], Cs[kRows * LB];
-    float Xs[kRows * LX], Ys[kRows * LX];
-    float Ms[kRows * LM], Ds[kRows * LM];
-    float Ss[kP * LS], Gs[kP * LS];
-    // per token and pair, rows of AP = NH + 3 words: a row-strided access by
-    // sixteen lanes then spreads over the banks instead of landing on one.
-    // cos and sin of the in-chunk angle; once every reader holds its values
-    // they take the two halves of the angle sums
-    static constexpr int AP = NH + 3;
-    float acs[QT * AP], asn[QT * AP];
-    float phi_end[NH];      // the chunk's angle total per pair
-    float dtv[QT], lamv[QT], acum[QT], aclo[QT], gw[QT], ww[QT], eac[QT], ebar[QT], wbar[QT];
-    float rin[kRows], cinx[kRows], dwi[kRows], qv[kRows], rcr[kRows];
-    float dgv[QT], dal[QT];
-    float red[48];
-};
-
-// Per-token scalars, the in-chunk angles, and (X, dY) / (B~, C~) as asked.
-// Every global load of the chunk is issued before the first use of any of
-// them (NTH threads, the workgroup size): a wave then waits once for its
-// whole share instead of once per staged element.
-template <typename T, int N, int R, int kRows, bool WANT_B, bool WANT_X, int NTH, typename S>
-__device__ void stage(const ScanLaunch &a, const BwdArgs &g, S &sm, size_t bh, int ck) {
-    constexpr int QT = S::QT, NH = S::NH, NW = NTH / 64;
-    constexpr int TI = NH / NW;                 // angle pairs per wave
-    // chunks of at most 32 tokens scan two pairs per wave scan (lanes [0, 32)
-    // and [32, 64)); lane -> token tl of pair wave + (PK j + hl) NW
-    constexpr bool PACK = QT <= 32;
-    constexpr int PK = PACK ? 2 : 1, TS = TI / PK;
-    static_assert(TI % PK == 0, "paired angle scans");
-    constexpr int JB = (QT * NH + NTH - 1) / NTH;   // (token, pair) items per thread
-    constexpr int JX = kRows * kP / NTH;        // (row, p) items per thread
-    static_assert(NH % NW == 0 && (kRows * kP) % NTH == 0, "stage split");
-    constexpr bool kPrecise = true;   // precise sines whatever the storage
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t H = a.heads, L = a.seq;
-    const size_t bb = bh / H, hh = bh % H;
-    const bool rot = a.theta != nullptr;
-    const float A = 0.0f - expf(a.a_log[hh]);
-    const size_t t0 = static_cast<size_t>(ck) * QT;
-
-    // ---- loads
-    float dt = 0.0f, lam = 0.0f, dtn = 0.0f, lamn = 0.0f;
-    if (tid < QT) {
-        const size_t t = t0 + tid;
-        const size_t ix = (bb * L + t) * H + hh;
-        if (t < L) {
-            dt = a.dt[ix];
-            lam = a.lambda[ix];
-        }
-        if (t + 1 < L) {
-            dtn = a.dt[ix + H];
-            lamn = a.lambda[ix + H];
-        }
-    }
-    const int tl = PACK ? (lane & 31) : lane, hl = PACK ? (lane >> 5) : 0;
-    const size_t tgl = t0 + tl;
-    const bool tlive = tl < QT && tgl < L;
-    // Loads are unconditional at clamped (in-bounds) indices and the dead
-    // lanes zeroed afterwards, so no load sits behind a branch (which would
-    // make each one wait for its data before the next is issued).
-    float th[TS];
-    if (rot) {
-        const size_t th0 = ((bb * L + (tlive ? tgl : 0)) * H + hh) * NH;
-#pragma unroll
-        for (int j = 0; j < TS; ++j) {
-            const float v = ldv<T>(a.theta, th0 + wave + (PK * j + hl) * NW);
-            th[j] = tlive ? v : 0.0f;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < TS; ++j) th[j] = 0.0f;
-    }
-    float b1[JB][R], b2[JB][R], c1[JB][R], c2[JB][R];
-#pragma unroll
-    for (int j = 0; j < JB; ++j) {
-        const int e = tid + j * NTH, t = e / NH;
-        const int i = e < QT * NH ? e % NH : 0;
-        const size_t tg = t0 + t;
-        const bool live = e < QT * NH && tg < L;
-        const size_t base = ((bb * L + (live ? tg : 0)) * H + hh) * N * R;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            b1[j][r] = b2[j][r] = 0.0f;
-            if constexpr (WANT_B) {
-                const float u1 = ldv<T>(a.b, base + i * R + r);
-                const float u2 = ldv<T>(a.b, base + (i + NH) * R + r);
-                b1[j][r] = live ? u1 : 0.0f;
-                b2[j][r] = live ? u2 : 0.0f;
-            }
-            const float v1 = ldv<T>(a.c, base + i * R + r);
-            const float v2 = ldv<T>(a.c, base + (i + NH) * R + r);
-            c1[j][r] = live ? v1 : 0.0f;
-            c2[j][r] = live ? v2 : 0.0f;
-        }
-    }
-    float yv[JX], xv[JX];
-#pragma unroll
-    for (int j = 0; j < JX; ++j) {
-        const int e = tid + j * NTH, rho = e / kP, p = e % kP;
-        const int t = rho / R, r = rho % R;
-        const size_t tg = t0 + t;
-        const bool live = tg < L;
-        const size_t ix = (((bb * L + (live ? tg : 0)) * H + hh) * kP + p) * R + r;
-        const float vy = ldv<T>(g.dy, ix);
-        yv[j] = live ? vy : 0.0f;
-        xv[j] = 0.0f;
-        if constexpr (WANT_X) {
-            const float vx = ldv<T>(a.x, ix);
-            xv[j] = live ? vx : 0.0f;
-        }
-    }
-
-    // ---- per-token scalars and the in-chunk prefixes (wave scans, lane = token)
-    if (tid < QT) {
-        sm.dtv[tid] = dt;
-        sm.lamv[tid] = lam;
-        sm.gw[tid] = lam * dt;                          // fused.rs:2494
-        sm.ww[tid] = lam * dt + (1.0f - lamn) * dtn;    // fused.rs:2496-2498
-    }
-    if (wave == 0) {
-        float hi, lo;
-        split_decay(tid < QT ? dt : 0.0f, A, hi, lo);
-        hi = seg_scan<64>(hi);
-        lo = seg_scan<64>(lo);
-        if (lane < QT) {
-            sm.acum[lane] = hi;
-            sm.aclo[lane] = lo;
-        }
-    }
-    __syncthreads();
-    if (rot) {
-        // the in-chunk angle (inclusive cumsum of dt theta) and its cos / sin
-        const float dtl = tlive ? sm.dtv[tl] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < TS; ++j) {
-            const int i = wave + (PK * j + hl) * NW;
-            const float v = PACK ? seg_scan<32>(dtl * th[j]) : seg_scan<64>(dtl * th[j]);
-            if (tl < QT) {
-                float sv, cv;
-                sincos_any<kPrecise>(v, sv, cv);
-                sm.acs[tl * S::AP + i] = cv;
-                sm.asn[tl * S::AP + i] = sv;
-            }
-            if (tl == QT - 1) sm.phi_end[i] = v;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < JX; ++j) {
-        const int e = tid + j * NTH, rho = e / kP, p = e % kP;
-        sm.Ys[S::xi(rho, p)] = yv[j];
-        if constexpr (WANT_X) sm.Xs[S::xi(rho, p)] = xv[j];
-    }
-    __syncthreads();
-    if (tid < QT) {
-        const float hi = sm.acum[tid], lo = sm.aclo[tid];
-        sm.eac[tid] = clamp_exp(hi + lo);
-        sm.ebar[tid] = clamp_exp((sm.acum[QT - 1] - hi) + (sm.aclo[QT - 1] - lo));
-        sm.wbar[tid] = sm.ebar[tid] * sm.ww[tid];
-    }
-    // ---- rotation by the negative in-chunk angle (fused.rs:610-617) into LDS
-#pragma unroll
-    for (int j = 0; j < JB; ++j) {
-        const int e = tid + j * NTH, t = e / NH, i = e % NH;
-        if (e >= QT * NH) break;
-        float sn = 0.0f, cs = 1.0f;
-        if (rot) {
-            cs = sm.acs[t * S::AP + i];
-            sn = sm.asn[t * S::AP + i];
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int rho = t * R + r;
-            if constexpr (WANT_B) {
-                sm.Bs[S::bi(rho, i)] = b1[j][r] * cs + b2[j][r] * sn;
-                sm.Bs[S::bi(rho, i + NH)] = -b1[j][r] * sn + b2[j][r] * cs;
-            }
-            sm.Cs[S::bi(rho, i)] = c1[j][r] * cs + c2[j][r] * sn;
-            sm.Cs[S::bi(rho, i + NH)] = -c1[j][r] * sn + c2[j][r] * cs;
-        }
-    }
 }
 
 // ---------------------------------------------------------------- state passes
@@ -439,42 +256,42 @@ __device__ void stage(const ScanLaunch &a, const BwdArgs &g, S &sm, size_t bh, i
 //     sum_rho C~[rho][n] e^{alpha} dY[rho][p], the chunk's direct share of
 //     dL/dS_k (the carry-in product y += e^alpha C~ S, scan.rs:253-263); then
 //     dh0, dlast_u0 and the gradient of (1 - lambda_0) dt_0.
-// One workgroup per (batch, head, 16 rotation pairs) and direction; thread =
-// (p, four pairs): the state's 32 columns of those pairs stay in registers.
-// Per chunk the workgroup stages the token scalars and its pairs' in-chunk
-// angles (the scans of the chunk kernel's stage, so every value is the
-// same), rotates its 32 columns of B (or C) into LDS scaled by wbar (or not),
-// stages X (or e^alpha dY), and forms U^T (or V^T) by f32 MFMA directly in the
-// state's lane layout.  The raw inputs of the next chunks are loaded ahead
-// into registers; no per-chunk record but S_k (Gh_k) leaves the workgroup.
-template <int R, int kRows>
+// One workgroup per (batch, head, 16 rotation pairs) and direction; the
+// state's 32 columns of those pairs, for all 64 p, stay in registers in the
+// MFMA D layout (lane (c, g) of wave pt: column n = 16 i1 + c and its partner,
+// p = 16 pt + 4 g + r), which is also how the chunk kernel's operands read the
+// records.  Per chunk the workgroup stages the token scalars and its pairs'
+// in-chunk angles (the scans of the chunk kernel, so every value is the same),
+// rotates its 32 columns of B (or C) into LDS scaled by wbar (or not), stages
+// X (or e^alpha dY) as rows, and forms U (or V) by f32 MFMA.  The raw inputs
+// of the next chunks are loaded ahead into registers, four elements a load; no
+// per-chunk record but S_k (Gh_k) leaves the workgroup.  At batch 8 x 2048, 12
+// heads, d_state 128 the two passes take 204 us (226 with an element a load and
+// X transposed in LDS, whose writes fell on a quarter of the banks).
+template <int R>
 struct PassSmem {
-    static constexpr int QT = kRows / R, LDR = kRows + 4, AP = 17;
+    static constexpr int QT = kRows / R, LDR = kRows + 4, LX = kP + 4, AP = 17;
     float As[32 * LDR];      // rotated columns: [column][rho], lo pairs then hi
-    float Xs[kP * LDR];      // X or e^alpha dY: [p][rho]
+    float Xs[kRows * LX];    // X or e^alpha dY: [rho][p]
     // per chunk parity: cos / sin of the in-chunk angle [token][pair], the
     // token scalars, the decay prefix and the per-token scale
     float acs[2][QT * AP], asn[2][QT * AP];
-    float dtv[2][QT], acum[2][QT], aclo[2][QT], ww[2][QT], scal[2][QT];
+    float acum[2][QT], aclo[2][QT], ww[2][QT], scal[2][QT];
     float phi[16];           // the sequence's angle total per pair (reverse pass)
     float red[16];
 };
 
-template <typename T, int N, int R, int kRows, bool FWD>
+template <typename T, int N, int R, bool FWD>
 __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w, int nck,
-                           size_t blk, PassSmem<R, kRows> &sm) {
-    using S = PassSmem<R, kRows>;
-    constexpr int NTN = N / 16, HT = NTN / 2, NH = N / 2, QT = S::QT, LDR = S::LDR, AP = S::AP;
-    constexpr int NW = 4;                       // waves
-    constexpr int TI = 16 / NW;                 // pairs per wave in the angle scans
-    constexpr bool PACK = QT <= 32;             // two 32-token scans per wave
-    constexpr int PK = PACK ? 2 : 1, TS = TI / PK;
-    constexpr int JB = 16 * kRows / 256;        // (row, pair) items per thread
-    constexpr int JX = kP * kRows / 256;        // (row, p) items per thread
-    constexpr int D = kRows == 32 ? 3 : 2;      // chunks loaded ahead
-    static_assert(TI % PK == 0 && JB >= 1 && JX >= 1, "pass split");
-    const int tid = threadIdx.x, lane = tid & 63, pt = tid >> 6;
-    const int wave = __builtin_amdgcn_readfirstlane(pt);
+                           size_t blk, PassSmem<R> &sm) {
+    using S = PassSmem<R>;
+    constexpr int NTN = N / 16, HT = NTN / 2, NH = N / 2, QT = S::QT, LDR = S::LDR, LX = S::LX, AP = S::AP;
+    constexpr int PN = 2;                       // pairs a half-wave scans
+    constexpr int NB = QT * 4 * R;              // four-element items of B (or C): 128
+    constexpr int JX = 2;                       // ... of X (or dY) per thread: 512
+    constexpr int D = 3;                        // chunks loaded ahead
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int pt = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, gq = lane >> 4;
     const int i1 = static_cast<int>(blk % HT);
     const size_t bh = blk / HT;
@@ -482,54 +299,53 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     const size_t bb = bh / H, hh = bh % H;
     const bool rot = a.theta != nullptr;
     const float A = 0.0f - expf(a.a_log[hh]);
-    const int p = 16 * pt + c, nlo = 16 * i1 + 4 * gq;
-    const size_t sbase = bh * kP * N + static_cast<size_t>(p) * N;
-    const int tl = PACK ? (lane & 31) : lane, hl = PACK ? (lane >> 5) : 0;
-    auto rot4 = [](f32x4 &lo, f32x4 &hi, f32x4 cs, f32x4 sn) {
+    const int p0 = 16 * pt + 4 * gq, nlo = 16 * i1 + c;
+    const size_t sbase = bh * kP * N + static_cast<size_t>(p0) * N + nlo;   // state (p0, nlo)
+    const int tl = lane & 31, hl = lane >> 5;   // the angle scans: lane -> token, pairs ip ..
+    const int ip = 4 * pt + PN * hl;
+    auto rot4 = [](f32x4 &lo, f32x4 &hi, float cs, float sn) {
         const f32x4 l = lo;
         lo = l * cs - hi * sn;
         hi = l * sn + hi * cs;
     };
-    auto sincos4 = [](f32x4 t, f32x4 &sn, f32x4 &cs) {
+    auto ld_state = [&](const float *p, f32x4 &lo, f32x4 &hi) {
+#pragma unroll
         for (int r = 0; r < 4; ++r) {
-            float s, cc;
-            sincosf(t[r], &s, &cc);
-            sn[r] = s;
-            cs[r] = cc;
+            lo[r] = p[sbase + r * N];
+            hi[r] = p[sbase + r * N + NH];
+        }
+    };
+    auto st_state = [&](float *p, f32x4 lo, f32x4 hi) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            p[sbase + r * N] = lo[r];
+            p[sbase + r * N + NH] = hi[r];
         }
     };
 
     struct In {
-        float dt, lam, dtn, lamn;
-        float th[TS];
-        float b1[JB], b2[JB];
-        float xv[JX];
+        float dt, lam, dtn, lamn, dtl;
+        uint32_t th[PN];
+        Raw4<T> b1, b2, x[JX];
     };
     // Chunk k's raw inputs, by buffer loads over this sequence's tokens: a
-    // token at or past the sequence end reads as zero, as the chunk kernel's
-    // stage zeroes it.  A thread's items sit at fixed byte offsets from its
-    // chunk-0 offsets (256 threads cover whole tokens of every array).
+    // token at or past the sequence end reads as zero.  A thread's items sit
+    // at fixed byte offsets from its chunk-0 offsets.
     constexpr uint32_t SZ = sizeof(T);
     const scan::SeqBufs rs = scan::seq_bufs<T, N, kP, R>(a, bb, hh);
     const rsrc_t rbc = FWD ? rs.b : rs.c;
     const rsrc_t rxy = FWD ? rs.x
                            : make_rsrc(static_cast<const char *>(g.dy) + (bb * L * H + hh) * kP * R * SZ,
                                        static_cast<uint32_t>((L * H - hh) * kP * R * SZ));
-    auto ld = [](rsrc_t r, uint32_t off) -> float {
-        if constexpr (sizeof(T) == 4)
-            return bldf(r, off);
-        else
-            return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)) << 16);
-    };
-    const int ts = tid < QT ? tid : 0;
-    const uint32_t o_s = ts * rs.tok_s;
-    const uint32_t o_th = tl * rs.tok_th + (16 * i1) * SZ;
-    const int tb = tid / (16 * R), qr = tid % (16 * R);
-    const uint32_t o_bc = tb * rs.tok_bc + (16 * i1 * R + qr) * SZ;
-    const uint32_t bc_j = (16 / R) * rs.tok_bc;
-    const int tx = tid / (kP * R), pr = tid % (kP * R);
-    const uint32_t o_xy = tx * rs.tok_x + pr * SZ;
-    const uint32_t xy_j = (256 / (kP * R)) * rs.tok_x;
+    const bool xal = FWD || (reinterpret_cast<uintptr_t>(g.dy) & 3u) == 0;
+    const uint32_t o_s = (tid < QT ? tid : 0) * rs.tok_s;
+    const uint32_t o_tl = (tl < QT ? tl : 0) * rs.tok_s;
+    const uint32_t o_th = (tl < QT ? tl : 0) * rs.tok_th + (16 * i1 + ip) * SZ;
+    const int tb = tid / (4 * R), eb = (tid % (4 * R)) * 4;      // items tid < NB
+    const uint32_t o_bc = tb * rs.tok_bc + (16 * i1 * R + eb) * SZ;
+    const int tx = tid / (16 * R), ex = (tid % (16 * R)) * 4;    // items tid + 256 j
+    const uint32_t o_xy = tx * rs.tok_x + ex * SZ;
+    const uint32_t xy_j = (256 / (16 * R)) * rs.tok_x;
     auto load = [&](int k, In &d) {
         const int kk = k < 0 ? 0 : (k < nck ? k : nck - 1);   // outside: re-read, unused
         const uint32_t t0 = static_cast<uint32_t>(kk) * QT;
@@ -538,28 +354,16 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         d.dtn = bldf(rs.s0, o_s + (t0 + 1) * rs.tok_s);
         d.lamn = bldf(rs.s1, o_s + (t0 + 1) * rs.tok_s);
         if (rot) {
-            const uint32_t o = o_th + t0 * rs.tok_th;
-#pragma unroll
-            for (int j = 0; j < TS; ++j) {
-                const float v = ld(rs.th, o + (wave + (PK * j + hl) * NW) * SZ);
-                d.th[j] = tl < QT ? v : 0.0f;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < TS; ++j) d.th[j] = 0.0f;
+            d.dtl = bldf(rs.s0, o_tl + t0 * rs.tok_s);
+            ldth<T, PN>(rs.th, o_th + t0 * rs.tok_th, d.th);
         }
-        const uint32_t ob = o_bc + t0 * rs.tok_bc;
-#pragma unroll
-        for (int j = 0; j < JB; ++j) {
-            d.b1[j] = ld(rbc, ob + j * bc_j);
-            d.b2[j] = ld(rbc, ob + j * bc_j + NH * R * SZ);
+        if (tid < NB) {
+            ld4(d.b1, rbc, o_bc + t0 * rs.tok_bc);
+            ld4(d.b2, rbc, o_bc + t0 * rs.tok_bc + NH * R * SZ);
         }
-        const uint32_t ox = o_xy + t0 * rs.tok_x;
 #pragma unroll
-        for (int j = 0; j < JX; ++j) d.xv[j] = ld(rxy, ox + j * xy_j);
+        for (int j = 0; j < JX; ++j) ld4(d.x[j], rxy, o_xy + t0 * rs.tok_x + j * xy_j, xal);
     };
-    // Chunk k's term of this lane's state columns (acc), its decay e and the
-    // rotation by its angle totals (pc, ps).
     // The chunk's work in four pieces, software-pipelined over two sets of
     // the per-chunk tables (sb = chunk parity): the scalars and decay prefix
     // (p1) and the angles (p2) of chunk k + 1 run in the same two barrier
@@ -568,14 +372,13 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     // token scalars, the decay prefix (fused.rs:2494-2498)
     auto p1 = [&](const In &d, int sb) {
         if (tid < QT) {
-            sm.dtv[sb][tid] = d.dt;
             sm.ww[sb][tid] = d.lam * d.dt + (1.0f - d.lamn) * d.dtn;
         }
-        if (wave == 0) {
+        if (pt == 0) {
             float hi, lo;
             split_decay(tid < QT ? d.dt : 0.0f, A, hi, lo);
-            hi = seg_scan<64>(hi);
-            lo = seg_scan<64>(lo);
+            hi = seg_scan<32>(hi);
+            lo = seg_scan<32>(lo);
             if (lane < QT) {
                 sm.acum[sb][lane] = hi;
                 sm.aclo[sb][lane] = lo;
@@ -584,19 +387,20 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     };
     // the in-chunk angle of this workgroup's pairs and its cos / sin; per
     // token wbar (B~'s scale) or e^alpha (dY's)
-    auto p2 = [&](int k, const In &d, int sb) {
+    auto p2 = [&](const In &d, int sb) {
         if (rot) {
-            const size_t t0 = static_cast<size_t>(k) * QT;
-            const float dtl = (tl < QT && t0 + tl < L) ? sm.dtv[sb][tl] : 0.0f;
+            float v[PN];
+            unth<T, PN>(d.th, v);
 #pragma unroll
-            for (int j = 0; j < TS; ++j) {
-                const int i = wave + (PK * j + hl) * NW;
-                const float v = PACK ? seg_scan<32>(dtl * d.th[j]) : seg_scan<64>(dtl * d.th[j]);
-                if (tl < QT) {
+            for (int j = 0; j < PN; ++j) v[j] = tl < QT ? d.dtl * v[j] : 0.0f;
+            scan32<PN>(v);
+            if (tl < QT) {
+#pragma unroll
+                for (int j = 0; j < PN; ++j) {
                     float sv, cv;
-                    sincos_any<true>(v, sv, cv);
-                    sm.acs[sb][tl * AP + i] = cv;
-                    sm.asn[sb][tl * AP + i] = sv;
+                    sincosf(v[j], &sv, &cv);
+                    sm.acs[sb][tl * AP + ip + j] = cv;
+                    sm.asn[sb][tl * AP + ip + j] = sv;
                 }
             }
         }
@@ -610,53 +414,61 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     // rotation by the negative in-chunk angle (fused.rs:610-617) into LDS;
     // the chunk decay
     auto p3 = [&](const In &d, int sb, float &e) {
+        if (tid < NB) {
+            float b1[4], b2[4];
+            un4(d.b1, b1);
+            un4(d.b2, b2);
+            const float sc = FWD ? sm.scal[sb][tb] : 1.0f;
 #pragma unroll
-        for (int j = 0; j < JB; ++j) {
-            const int ee = tid + 256 * j, t = ee / (16 * R), qr = ee % (16 * R);
-            const int q = qr / R, rho = t * R + qr % R;
-            float sn = 0.0f, cs = 1.0f;
-            if (rot) {
-                cs = sm.acs[sb][t * AP + q];
-                sn = sm.asn[sb][t * AP + q];
+            for (int j = 0; j < 4; ++j) {
+                const int q = (eb + j) / R, rho = tb * R + (eb + j) % R;
+                float sn = 0.0f, cs = 1.0f;
+                if (rot) {
+                    cs = sm.acs[sb][tb * AP + q];
+                    sn = sm.asn[sb][tb * AP + q];
+                }
+                sm.As[q * LDR + rho] = (b1[j] * cs + b2[j] * sn) * sc;
+                sm.As[(16 + q) * LDR + rho] = (-b1[j] * sn + b2[j] * cs) * sc;
             }
-            float lo = d.b1[j] * cs + d.b2[j] * sn;
-            float hi = -d.b1[j] * sn + d.b2[j] * cs;
-            if constexpr (FWD) {
-                lo *= sm.scal[sb][t];
-                hi *= sm.scal[sb][t];
-            }
-            sm.As[q * LDR + rho] = lo;
-            sm.As[(16 + q) * LDR + rho] = hi;
         }
 #pragma unroll
         for (int j = 0; j < JX; ++j) {
-            const int ee = tid + 256 * j, t = ee / (kP * R), pr = ee % (kP * R);
-            float v = d.xv[j];
-            if constexpr (!FWD) v *= sm.scal[sb][t];
-            sm.Xs[(pr / R) * LDR + t * R + pr % R] = v;
+            const int t = tx + j * (256 / (16 * R));
+            float v[4];
+            un4(d.x[j], v);
+            if constexpr (!FWD) {
+                const float sc = sm.scal[sb][t];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] *= sc;
+            }
+            put4<R>(sm.Xs, LX, t, ex, v);
         }
         e = clamp_exp(sm.acum[sb][QT - 1] + sm.aclo[sb][QT - 1]);
     };
-    // U^T (V^T) at this lane's (n, p): A(m = n, k = rho), B(k = rho, col = p);
-    // the rotation by the chunk's angle totals, the in-chunk angles of its
-    // last row
-    auto p4 = [&](int sb, f32x4 &alo, f32x4 &ahi, f32x4 &pc, f32x4 &ps) {
+    // U (V) at this lane's (p, n): A(m = p, k = rho), B(k = rho, col = n), with
+    // k slot 4 g + r of a block of 16 the rho of MFMA r's lane group g; the
+    // rotation by the chunk's angle totals, the in-chunk angles of its last row
+    auto p4 = [&](int sb, f32x4 &alo, f32x4 &ahi, float &pc, float &ps) {
         alo = f32x4{0.f, 0.f, 0.f, 0.f};
         ahi = alo;
-        const float *br = sm.Xs + p * LDR;
 #pragma unroll
         for (int kb = 0; kb < kRows / 16; ++kb) {
-            alo = scan::mma_kb(sm.As + c * LDR + 16 * kb, br + 16 * kb, alo, gq);
-            ahi = scan::mma_kb(sm.As + (16 + c) * LDR + 16 * kb, br + 16 * kb, ahi, gq);
-        }
-        pc = f32x4{1.f, 1.f, 1.f, 1.f};
-        ps = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (rot) {
+            const f32x4 bl = *reinterpret_cast<const f32x4 *>(sm.As + c * LDR + 16 * kb + 4 * gq);
+            const f32x4 bhv = *reinterpret_cast<const f32x4 *>(sm.As + (16 + c) * LDR + 16 * kb + 4 * gq);
+            float av[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) av[r] = sm.Xs[(16 * kb + 4 * gq + r) * LX + 16 * pt + c];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                pc[r] = sm.acs[sb][(QT - 1) * AP + 4 * gq + r];
-                ps[r] = sm.asn[sb][(QT - 1) * AP + 4 * gq + r];
+                alo = mfma_f32(av[r], bl[r], alo);
+                ahi = mfma_f32(av[r], bhv[r], ahi);
             }
+        }
+        pc = 1.0f;
+        ps = 0.0f;
+        if (rot) {
+            pc = sm.acs[sb][(QT - 1) * AP + c];
+            ps = sm.asn[sb][(QT - 1) * AP + c];
         }
     };
     auto offs = [&](int k, size_t &o, size_t &oh) {
@@ -668,18 +480,19 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
     if constexpr (FWD) {
         if (a.h0 != nullptr) {
-            lo = *reinterpret_cast<const f32x4 *>(a.h0 + sbase + nlo);
-            hi = *reinterpret_cast<const f32x4 *>(a.h0 + sbase + nlo + NH);
+            ld_state(a.h0, lo, hi);
             if (a.last_u0 != nullptr) {
                 const size_t i0 = (bb * L) * H + hh;
                 const float first = (1.0f - a.lambda[i0]) * a.dt[i0];
-                lo += *reinterpret_cast<const f32x4 *>(a.last_u0 + sbase + nlo) * first;
-                hi += *reinterpret_cast<const f32x4 *>(a.last_u0 + sbase + nlo + NH) * first;
+                f32x4 ul, uh;
+                ld_state(a.last_u0, ul, uh);
+                lo += ul * first;
+                hi += uh * first;
             }
         }
         if (rot && a.angle0 != nullptr) {
-            f32x4 sn, cs;
-            sincos4(*reinterpret_cast<const f32x4 *>(a.angle0 + bh * NH + nlo), sn, cs);
+            float sn, cs;
+            sincosf(a.angle0[bh * NH + nlo], &sn, &cs);
             rot4(lo, hi, cs, sn);
         }
         In d[D];
@@ -687,7 +500,7 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         for (int j = 0; j < D; ++j) load(j, d[j]);
         p1(d[0], 0);
         __syncthreads();
-        p2(0, d[0], 0);
+        p2(d[0], 0);
         __syncthreads();
         for (int k = 0; k < nck; k += D) {
 #pragma unroll
@@ -696,13 +509,13 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                 if (kc < nck) {
                     const int sb = kc & 1;
                     const bool more = kc + 1 < nck;
-                    float e;
+                    float e, pc, ps;
                     p3(d[j], sb, e);
                     if (more) p1(d[(j + 1) % D], sb ^ 1);
                     __syncthreads();
-                    f32x4 ulo, uhi, pc, ps;
+                    f32x4 ulo, uhi;
                     p4(sb, ulo, uhi, pc, ps);
-                    if (more) p2(kc + 1, d[(j + 1) % D], sb ^ 1);
+                    if (more) p2(d[(j + 1) % D], sb ^ 1);
                     size_t o, oh;
                     offs(kc, o, oh);
                     *reinterpret_cast<f32x4 *>(w.s + o) = lo;
@@ -718,30 +531,20 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         }
     } else {
         if (g.dh_out != nullptr) {
-            lo = *reinterpret_cast<const f32x4 *>(g.dh_out + sbase + nlo);
-            hi = *reinterpret_cast<const f32x4 *>(g.dh_out + sbase + nlo + NH);
+            ld_state(g.dh_out, lo, hi);
             if (rot) {
                 // phi_end = angle0 + sum_k Phi_k: the final frame, S_C = R(phi_end) h_out.
                 // Each Phi_k is the in-chunk scan's last value, summed in chunk order.
                 constexpr int DT = 8;
-                float ph[TS], dq[DT], tq[DT][TS];
+                float ph[PN], dq[DT];
+                uint32_t tq[DT][PN];
 #pragma unroll
-                for (int j = 0; j < TS; ++j) {
-                    const int i = wave + (PK * j + hl) * NW;
-                    ph[j] = a.angle0 != nullptr ? a.angle0[bh * NH + 16 * i1 + i] : 0.0f;
-                }
-                auto tload = [&](int k, float &dv, float (&tv)[TS]) {
-                    const int kk = k < nck ? k : nck - 1;
-                    const size_t tg = static_cast<size_t>(kk) * QT + tl;
-                    const bool tlive = tl < QT && tg < L;
-                    const size_t row = (bb * L + (tlive ? tg : 0)) * H + hh;
-                    const float v = a.dt[row];
-                    dv = tlive ? v : 0.0f;
-#pragma unroll
-                    for (int j = 0; j < TS; ++j) {
-                        const float u = ldv<T>(a.theta, row * NH + 16 * i1 + wave + (PK * j + hl) * NW);
-                        tv[j] = tlive ? u : 0.0f;
-                    }
+                for (int j = 0; j < PN; ++j)
+                    ph[j] = a.angle0 != nullptr ? a.angle0[bh * NH + 16 * i1 + ip + j] : 0.0f;
+                auto tload = [&](int k, float &dv, uint32_t (&tv)[PN]) {
+                    const uint32_t t0 = static_cast<uint32_t>(k < nck ? k : nck - 1) * QT;
+                    dv = bldf(rs.s0, o_tl + t0 * rs.tok_s);
+                    ldth<T, PN>(rs.th, o_th + t0 * rs.tok_th, tv);
                 };
 #pragma unroll
                 for (int q = 0; q < DT; ++q) tload(q, dq[q], tq[q]);
@@ -749,27 +552,26 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
 #pragma unroll
                     for (int q = 0; q < DT; ++q) {
                         if (k + q < nck) {
+                            float v[PN];
+                            unth<T, PN>(tq[q], v);
 #pragma unroll
-                            for (int j = 0; j < TS; ++j) {
-                                const float v = PACK ? seg_scan<32>(dq[q] * tq[q][j])
-                                                     : seg_scan<64>(dq[q] * tq[q][j]);
-                                ph[j] += v;
-                            }
+                            for (int j = 0; j < PN; ++j) v[j] = tl < QT ? dq[q] * v[j] : 0.0f;
+                            scan32<PN>(v);
+#pragma unroll
+                            for (int j = 0; j < PN; ++j) ph[j] += v[j];
                         }
                         tload(k + DT + q, dq[q], tq[q]);
                     }
                 }
                 if (tl == QT - 1) {
 #pragma unroll
-                    for (int j = 0; j < TS; ++j) sm.phi[wave + (PK * j + hl) * NW] = ph[j];
+                    for (int j = 0; j < PN; ++j) sm.phi[ip + j] = ph[j];
                 }
                 __syncthreads();
-                f32x4 pe;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) pe[r] = sm.phi[4 * gq + r];
+                const float pe = sm.phi[c];
                 __syncthreads();
-                f32x4 sn, cs;
-                sincos4(pe, sn, cs);
+                float sn, cs;
+                sincosf(pe, &sn, &cs);
                 rot4(lo, hi, cs, sn);
             }
         }
@@ -778,7 +580,7 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         for (int j = 0; j < D; ++j) load(nck - 1 - j, d[j]);
         p1(d[0], (nck - 1) & 1);
         __syncthreads();
-        p2(nck - 1, d[0], (nck - 1) & 1);
+        p2(d[0], (nck - 1) & 1);
         __syncthreads();
         for (int k = nck - 1; k >= 0; k -= D) {
 #pragma unroll
@@ -787,13 +589,13 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                 if (kc >= 0) {
                     const int sb = kc & 1;
                     const bool more = kc > 0;
-                    float e;
+                    float e, pc, ps;
                     p3(d[j], sb, e);
                     if (more) p1(d[(j + 1) % D], sb ^ 1);
                     __syncthreads();
-                    f32x4 vlo, vhi, pc, ps;
+                    f32x4 vlo, vhi;
                     p4(sb, vlo, vhi, pc, ps);
-                    if (more) p2(kc - 1, d[(j + 1) % D], sb ^ 1);
+                    if (more) p2(d[(j + 1) % D], sb ^ 1);
                     if (rot) rot4(lo, hi, pc, -ps);   // R(-Phi_k)
                     size_t o, oh;
                     offs(kc, o, oh);
@@ -808,26 +610,20 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         }
         // into the global frame: dZ0 = R(-angle0) G_0
         if (rot && a.angle0 != nullptr) {
-            f32x4 sn, cs;
-            sincos4(*reinterpret_cast<const f32x4 *>(a.angle0 + bh * NH + nlo), sn, cs);
+            float sn, cs;
+            sincosf(a.angle0[bh * NH + nlo], &sn, &cs);
             rot4(lo, hi, cs, -sn);
         }
         float dfirst = 0.0f;
         if (a.h0 != nullptr) {
-            if (g.dh0 != nullptr) {
-                *reinterpret_cast<f32x4 *>(g.dh0 + sbase + nlo) = lo;
-                *reinterpret_cast<f32x4 *>(g.dh0 + sbase + nlo + NH) = hi;
-            }
+            if (g.dh0 != nullptr) st_state(g.dh0, lo, hi);
             if (a.last_u0 != nullptr) {
                 const size_t i0 = (bb * L) * H + hh;
                 const float first = (1.0f - a.lambda[i0]) * a.dt[i0];
-                const f32x4 ul = *reinterpret_cast<const f32x4 *>(a.last_u0 + sbase + nlo);
-                const f32x4 uh = *reinterpret_cast<const f32x4 *>(a.last_u0 + sbase + nlo + NH);
+                f32x4 ul, uh;
+                ld_state(a.last_u0, ul, uh);
                 for (int r = 0; r < 4; ++r) dfirst += lo[r] * ul[r] + hi[r] * uh[r];
-                if (g.dlast_u0 != nullptr) {
-                    *reinterpret_cast<f32x4 *>(g.dlast_u0 + sbase + nlo) = lo * first;
-                    *reinterpret_cast<f32x4 *>(g.dlast_u0 + sbase + nlo + NH) = hi * first;
-                }
+                if (g.dlast_u0 != nullptr) st_state(g.dlast_u0, lo * first, hi * first);
             }
         }
         dfirst = block_sum(dfirst, sm.red);
@@ -837,172 +633,338 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
 
 // Both sequential passes in one launch (they are independent): workgroups
 // [0, nb) run the forward recurrence, [nb, 2 nb) the reverse one.
-template <typename T, int N, int R, int kRows>
-__global__ void __launch_bounds__(256) bwd_passes_kernel(ScanLaunch a, BwdArgs g, BwdWs w,
-                                                         int nck) {
-    __shared__ __attribute__((aligned(16))) PassSmem<R, kRows> sm;
+template <typename T, int N, int R>
+__global__ void __launch_bounds__(256) bwd_passes_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
+    __shared__ __attribute__((aligned(16))) PassSmem<R> sm;
     const size_t nb = a.batch * a.heads * (N / 32);
     if (blockIdx.x < nb)
-        state_pass<T, N, R, kRows, true>(a, g, w, nck, blockIdx.x, sm);
+        state_pass<T, N, R, true>(a, g, w, nck, blockIdx.x, sm);
     else
-        state_pass<T, N, R, kRows, false>(a, g, w, nck, blockIdx.x - nb, sm);
+        state_pass<T, N, R, false>(a, g, w, nck, blockIdx.x - nb, sm);
 }
 
 // ---------------------------------------------------------------- chunk gradients
-template <typename T, int N, int R, int kRows>
-__global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs g, BwdWs w,
-                                                           int nck) {
-    using S = Smem<N, R, kRows>;
-    constexpr int NT = kRows / 16;
-    constexpr int QT = S::QT, NH = S::NH, NTN = N / 16;
-    constexpr int LB = S::LB, LX = S::LX, LM = S::LM, LS = S::LS;
+// One workgroup of eight waves per chunk, two to a CU (80 KB of LDS and 128
+// VGPRs each): a chunk is a chain of six barriers, so one workgroup leaves
+// every unit idle most of the time, and the other fills in.  Measured at batch 8
+// x 2048, 12 heads, d_state 128, bf16 storage: sixteen waves with everything in
+// 158 KB of LDS, one to a CU, operands read by words, 445 us (MFMA busy 23 % of
+// the time, LDS 44 %); this form 297 us, against some 140 us for its 700 MB at
+// the rate of a large copy and 106 us of f32 MFMA.  What keeps it in 80 KB: the state S entering the chunk and Gh never go through LDS.  Their
+// records' lane layout (column n = 16 i + c, p = 16 pt + 4 g + r) is the MFMA
+// operand of the dC~ and dB~ products as it stands (k = p, 16 bytes a lane);
+// the Gh B~^T product reads Gh's record by words.  Operand rows in LDS are read
+// 16 bytes a lane, k slot 4 g + r of a block of 16 being lane group g's of MFMA
+// r, and read transposed in the same order, whose four lane groups then sit 4
+// rows apart, on banks of their own.
+template <int N, int R>
+struct Smem {
+    static constexpr int QT = kRows / R, NH = N / 2, NTN = N / 16, PT = NTN / 2;
+    static constexpr int LB = N + 12;       // B~, C~ rows
+    static constexpr int LX = kP + 4;       // X, dY rows
+    static constexpr int LM = kRows + 4;    // M, dCB rows
+    static constexpr int AP = NH + 1;
+    float Bs[kRows * LB], Cs[kRows * LB];
+    float Xs[kRows * LX], Ys[kRows * LX];   // Xs: the band's column sums once X has been used
+    float Ms[kRows * LM], Ds[kRows * LM];
+    // per token and pair: cos and sin of the in-chunk angle; once every reader
+    // holds its values, the two halves of the angle sums
+    float acs[QT * AP], asn[QT * AP];
+    float acum[QT], aclo[QT], gw[QT], ww[QT], eac[QT], ebar[QT], wbar[QT];
+    float rin[kRows], dgr[kRows];
+    float rcr[PT][kRows], qv[PT][kRows];    // per pair tile: rows' S and Gh sums
+    float red[3][kWaves];
+};
+
+template <typename T, int N, int R>
+__global__ void __launch_bounds__(kBT, 4) bwd_chunk_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
+    using S = Smem<N, R>;
+    constexpr int QT = S::QT, NH = S::NH, NTN = S::NTN, PT = S::PT;
+    constexpr int LB = S::LB, LX = S::LX, LM = S::LM, AP = S::AP;
+    constexpr uint32_t SZ = sizeof(T);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     S &sm = *reinterpret_cast<S *>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, gq = lane >> 4;
     const size_t bhk = blockIdx.x;
     const int ck = static_cast<int>(bhk % nck);
     const size_t bh = bhk / nck;
     const size_t H = a.heads, L = a.seq;
     const size_t bb = bh / H, hh = bh % H;
+    const bool rot = a.theta != nullptr;
     const float D = a.d_skip ? a.d_skip[hh] : 0.0f;
+    const float A = 0.0f - expf(a.a_log[hh]);
+    const uint32_t t0 = static_cast<uint32_t>(ck) * QT;
 
-    stage<T, N, R, kRows, true, true, kBT>(a, g, sm, bh, ck);
-    // the state entering the chunk and Gh, [p][n]: four consecutive n per
-    // 16-byte record piece, all loads in flight together
+    // ---- loads, all in flight together: tokens past the end read as zeros
+    const scan::SeqBufs rs = scan::seq_bufs<T, N, kP, R>(a, bb, hh);
+    const rsrc_t rdy = make_rsrc(static_cast<const char *>(g.dy) + (bb * L * H + hh) * kP * R * SZ,
+                                 static_cast<uint32_t>((L * H - hh) * kP * R * SZ));
+    const bool yal = (reinterpret_cast<uintptr_t>(g.dy) & 3u) == 0;
+    // the angle scans: lane -> token tl, pairs i0 ..
+    constexpr int PN = NH / 16;
+    const int tl = lane & 31, hl = lane >> 5;
+    const int i0 = (NH / kWaves) * wave + PN * hl;
+    float dtl = 0.0f;
+    uint32_t thq[PN];
+    if (rot) {
+        const uint32_t t = t0 + (tl < QT ? tl : 0);
+        dtl = bldf(rs.s0, t * rs.tok_s);
+        ldth<T, PN>(rs.th, t * rs.tok_th + i0 * SZ, thq);
+    }
+    float dt = 0.0f, lam = 0.0f, dtn = 0.0f, lamn = 0.0f;
+    if (tid < QT) {
+        dt = bldf(rs.s0, (t0 + tid) * rs.tok_s);
+        lam = bldf(rs.s1, (t0 + tid) * rs.tok_s);
+        dtn = bldf(rs.s0, (t0 + tid + 1) * rs.tok_s);
+        lamn = bldf(rs.s1, (t0 + tid + 1) * rs.tok_s);
+    }
+    // four elements of each half row of B and C, of a row of X and dY
+    constexpr int IB = NH * R / 4, IX = kP * R / 4;   // items per token
+    static_assert(QT * IX == kBT && QT * IB <= kBT, "one item a thread");
+    const bool has_b = tid < QT * IB;
+    const int tb = tid / IB, eb = (tid % IB) * 4, tx = tid / IX, ex = (tid % IX) * 4;
+    Raw4<T> b1, b2, c1, c2, xq, yq;
+    ld4(xq, rs.x, (t0 + tx) * rs.tok_x + ex * SZ);
+    ld4(yq, rdy, (t0 + tx) * rs.tok_x + ex * SZ, yal);
+    if (has_b) {
+        const uint32_t o = (t0 + tb) * rs.tok_bc + eb * SZ;
+        ld4(b1, rs.b, o);
+        ld4(b2, rs.b, o + NH * R * SZ);
+        ld4(c1, rs.c, o);
+        ld4(c2, rs.c, o + NH * R * SZ);
+    }
+    // The wave's dC~ (waves 0-3) or dB~ job: pair tile ji, JR row tiles from rt0
+    // on; S or Gh of its columns
+    constexpr int JR = PT == 4 ? 2 : 1;
+    static_assert(2 * PT * (2 / JR) == kWaves, "one job a wave");
+    const bool isb = wave >= kWaves / 2;
+    const int ji = wave % PT, rt0 = PT == 4 ? 0 : (wave / PT) & 1;
+    const size_t rec = bhk * kP * N;
+    const float eda = w.eda[bhk];
+    f32x4 fl[4], fh[4];
     {
-        constexpr int JS = kP * N / 4 / kBT;
-        static_assert(JS * 4 * kBT == kP * N, "state copy split");
-        f32x4 sv[JS], gv[JS];
-        const f32x4 *s4 = reinterpret_cast<const f32x4 *>(w.s +
-                                                          bhk * kP * N);
-        const f32x4 *g4 = reinterpret_cast<const f32x4 *>(w.gh + bhk * kP * N);
+        const f32x4 *r4 = reinterpret_cast<const f32x4 *>((isb ? w.gh : w.s) + rec) + lane;
 #pragma unroll
-        for (int j = 0; j < JS; ++j) {
-            sv[j] = s4[tid + j * kBT];
-            gv[j] = g4[tid + j * kBT];
+        for (int q = 0; q < 4; ++q) {
+            fl[q] = r4[(q * NTN + ji) * 64];
+            fh[q] = r4[(q * NTN + ji + PT) * 64];
         }
+    }
+
+    // ---- per-token scalars, the decay prefix, the in-chunk angles (inclusive
+    // cumsums of dt theta) and their cos / sin; X and dY
+    if (tid < QT) {
+        sm.gw[tid] = lam * dt;                          // fused.rs:2494
+        sm.ww[tid] = lam * dt + (1.0f - lamn) * dtn;    // fused.rs:2496-2498
+    }
+    if (wave == 0) {
+        float hi, lo;
+        split_decay(dt, A, hi, lo);
+        hi = seg_scan<32>(hi);
+        lo = seg_scan<32>(lo);
+        if (lane < QT) {
+            sm.acum[lane] = hi;
+            sm.aclo[lane] = lo;
+        }
+    }
+    if (rot) {
+        float v[PN];
+        unth<T, PN>(thq, v);
 #pragma unroll
-        for (int j = 0; j < JS; ++j) {
-            int p, n;
-            dl_pn(4 * (tid + j * kBT), NTN, p, n);
+        for (int j = 0; j < PN; ++j) v[j] = tl < QT ? dtl * v[j] : 0.0f;
+        scan32<PN>(v);
+        if (tl < QT) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                sm.Ss[p * LS + n + r] = sv[j][r];
-                sm.Gs[p * LS + n + r] = gv[j][r];
+            for (int j = 0; j < PN; ++j) {
+                float sv, cv;
+                sincosf(v[j], &sv, &cv);
+                sm.acs[tl * AP + i0 + j] = cv;
+                sm.asn[tl * AP + i0 + j] = sv;
             }
         }
     }
-    if (tid < kRows) {
-        sm.rin[tid] = sm.cinx[tid] = sm.dwi[tid] = sm.qv[tid] = sm.rcr[tid] = 0.0f;
+    float dsum = 0.0f, gsum = 0.0f, asum = 0.0f;
+    {
+        float xv[4], yv[4];
+        un4(xq, xv);
+        un4(yq, yv);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dsum = __builtin_fmaf(xv[j], yv[j], dsum);
+        put4<R>(sm.Xs, LX, tx, ex, xv);
+        put4<R>(sm.Ys, LX, tx, ex, yv);
     }
-    if (tid < QT) sm.dgv[tid] = 0.0f;
+    __syncthreads();
+    if (tid < QT) {
+        const float hi = sm.acum[tid], lo = sm.aclo[tid];
+        sm.eac[tid] = clamp_exp(hi + lo);
+        sm.ebar[tid] = clamp_exp((sm.acum[QT - 1] - hi) + (sm.aclo[QT - 1] - lo));
+        sm.wbar[tid] = sm.ebar[tid] * sm.ww[tid];
+    }
+    // rotation by the negative in-chunk angle (fused.rs:610-617) into LDS
+    if (has_b) {
+        float u1[4], u2[4], v1[4], v2[4], cs[4], sn[4];
+        un4(b1, u1);
+        un4(b2, u2);
+        un4(c1, v1);
+        un4(c2, v2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            cs[j] = rot ? sm.acs[tb * AP + (eb + j) / R] : 1.0f;
+            sn[j] = rot ? sm.asn[tb * AP + (eb + j) / R] : 0.0f;
+        }
+        float lo[4], hi[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            lo[j] = u1[j] * cs[j] + u2[j] * sn[j];
+            hi[j] = -u1[j] * sn[j] + u2[j] * cs[j];
+        }
+        put4<R>(sm.Bs, LB, tb, eb, lo);
+        put4<R>(sm.Bs + NH, LB, tb, eb, hi);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            lo[j] = v1[j] * cs[j] + v2[j] * sn[j];
+            hi[j] = -v1[j] * sn[j] + v2[j] * cs[j];
+        }
+        put4<R>(sm.Cs, LB, tb, eb, lo);
+        put4<R>(sm.Cs + NH, LB, tb, eb, hi);
+    }
     __syncthreads();
 
     // Three phases.  Phase 1 is everything that does not need the band: the
     // band products themselves, the Gh B~^T half of dX, the S dY / Gh X half of
     // each dC~ / dB~ job with its row sums, and the jobs' sines.  Phase 2 is
     // the band, elementwise.  Phase 3 finishes dX and the jobs with M and dCB.
-    // Work per wave: at most one dX tile and one job (accumulators stay in
-    // registers across the barriers); band products go to the waves from
-    // kWaves / 2 on first, which carry no dX tile.
-    constexpr int NB = NT * (NT + 1) / 2;
-    constexpr int PT = NTN / 2, NJ = NT * PT;
-    static_assert(2 * NJ <= kWaves && 4 * NT <= kWaves, "one job and one dX tile per wave");
-    const bool rot = a.theta != nullptr;
 
-    // ---- phase 1a: band products, raw: CB[t][s] = sum_n C~[t][n] B~[s][n]
-    // into Ms and dM[t][s] = sum_p dY[t][p] X[s][p] into Ds, for the tiles on
-    // and below the diagonal (the tiles above lie above the token diagonal)
-    for (int job = (wave + kWaves / 2) % kWaves; job < 2 * NB; job += kWaves) {
-        int q = job >> 1, tj = 0;
-        while (q > tj) {
-            q -= tj + 1;
-            ++tj;
+    // ---- phase 1a: dX^T[p][s] = sum_n Gh[p][n] B~[s][n] (x wbar_s, + phase 3),
+    // one 16 x 16 tile a wave: A(p = c, k): word c & 3 of the record's lane of
+    // (n, p >> 2), the four lane groups at n = 16 i + 4 j + g
+    const int xpt = wave & 3, xst = wave >> 2;
+    f32x4 xacc = {0.f, 0.f, 0.f, 0.f};
+    {
+        const float *gr = w.gh + rec + (xpt * NTN * 64 + gq + 16 * (c >> 2)) * 4 + (c & 3);
+        const float *br = sm.Bs + (16 * xst + c) * LB + gq;
+        constexpr int HB = NTN / 2;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            float av[HB][4];
+#pragma unroll
+            for (int i = 0; i < HB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) av[i][j] = gr[((half * HB + i) * 64 + 4 * j) * 4];
+#pragma unroll
+            for (int i = 0; i < HB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    xacc = mfma_f32(av[i][j], br[16 * (half * HB + i) + 4 * j], xacc);
         }
-        const int si = q;
+    }
+    // ---- phase 1b: dC~ and dB~ as [n][row] tiles
+    f32x4 lo[JR], hi[JR];
+    float cs[JR][4], sn[JR][4];
+    const int n0 = 16 * ji + 4 * gq;
+    // the job's own rotated operand (C~ for dC~, B~ for dB~) at its elements
+    const float *own = isb ? sm.Bs : sm.Cs;
+    {
+        const float *xr = isb ? sm.Xs : sm.Ys;
+#pragma unroll
+        for (int jr = 0; jr < JR; ++jr) {
+            lo[jr] = f32x4{0.f, 0.f, 0.f, 0.f};
+            hi[jr] = lo[jr];
+        }
+        // dC~^T[n][t] = e^{alpha_t} sum_p S[p][n] dY[t][p], dB~^T[n][s] = wbar_s
+        // sum_p Gh[p][n] X[s][p] (+ phase 3)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int jr = 0; jr < JR; ++jr) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(xr + (16 * (rt0 + jr) + c) * LX + 16 * q + 4 * gq);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    lo[jr] = mfma_f32(fl[q][r], v[r], lo[jr]);
+                    hi[jr] = mfma_f32(fh[q][r], v[r], hi[jr]);
+                }
+            }
+        if (!isb && rt0 == 0) {
+            // <Gh, S> over the job's columns
+            const f32x4 *r4 = reinterpret_cast<const f32x4 *>(w.gh + rec) + lane;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 ga = r4[(q * NTN + ji) * 64], gb = r4[(q * NTN + ji + PT) * 64];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    gsum = __builtin_fmaf(ga[r], fl[q][r], gsum);
+                    gsum = __builtin_fmaf(gb[r], fh[q][r], gsum);
+                }
+            }
+        }
+#pragma unroll
+        for (int jr = 0; jr < JR; ++jr) {
+            const int row = 16 * (rt0 + jr) + c, tr = row / R;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                cs[jr][r] = rot ? sm.acs[tr * AP + n0 + r] : 1.0f;
+                sn[jr][r] = rot ? sm.asn[tr * AP + n0 + r] : 0.0f;
+            }
+            if (!isb) {
+                const float ea = sm.eac[tr];
+                lo[jr] = lo[jr] * ea;
+                hi[jr] = hi[jr] * ea;
+            }
+            // row . (S or Gh part): the e^alpha dy.(S C~) and x.(Gh B~) terms
+            const f32x4 o1 = *reinterpret_cast<const f32x4 *>(own + row * LB + n0);
+            const f32x4 o2 = *reinterpret_cast<const f32x4 *>(own + row * LB + n0 + NH);
+            float q = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) q += lo[jr][r] * o1[r] + hi[jr][r] * o2[r];
+            q += __shfl_xor(q, 16, 64);
+            q += __shfl_xor(q, 32, 64);
+            if (gq == 0) (isb ? sm.qv : sm.rcr)[ji][row] = q;
+            if (isb) {
+                const float wb = sm.wbar[tr];
+                lo[jr] = lo[jr] * wb;
+                hi[jr] = hi[jr] * wb;
+            }
+        }
+    }
+    // ---- phase 1c: band products, raw: CB[t][s] = sum_n C~[t][n] B~[s][n]
+    // into Ms and dM[t][s] = sum_p dY[t][p] X[s][p] into Ds, for the three
+    // tiles on and below the diagonal (the tile above lies above the token
+    // diagonal)
+    if (wave < 6) {
+        const int q = wave % 3, tj = q > 0, si = q > 1;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         float *dst;
-        if ((job & 1) == 0) {
-            acc = mma_f32<N>(sm.Cs + 16 * tj * LB, LB, 1, sm.Bs + 16 * si * LB, 1, LB, acc, c, gq);
+        if (wave < 3) {
+#pragma unroll
+            for (int kb = 0; kb < N / 16; ++kb)
+                acc = scan::mma_kb(sm.Cs + (16 * tj + c) * LB + 16 * kb, sm.Bs + (16 * si + c) * LB + 16 * kb, acc, gq);
             dst = sm.Ms;
         } else {
-            acc = mma_f32<kP>(sm.Ys + 16 * tj * LX, LX, 1, sm.Xs + 16 * si * LX, 1, LX, acc, c, gq);
+#pragma unroll
+            for (int kb = 0; kb < kP / 16; ++kb)
+                acc = scan::mma_kb(sm.Ys + (16 * tj + c) * LX + 16 * kb, sm.Xs + (16 * si + c) * LX + 16 * kb, acc, gq);
             dst = sm.Ds;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) dst[(16 * tj + 4 * gq + r) * LM + 16 * si + c] = acc[r];
     }
-
-    // ---- phase 1b: dX^T[p][s] = wbar_s sum_n Gh[p][n] B~[s][n] (+ phase 3)
-    const bool has_dx = wave < 4 * NT;
-    const int xpt = wave & 3, xst = wave >> 2;
-    f32x4 xacc = {0.f, 0.f, 0.f, 0.f};
-    if (has_dx)
-        xacc = mma_f32<N>(sm.Gs + 16 * xpt * LS, LS, 1, sm.Bs + 16 * xst * LB, 1, LB, xacc, c, gq);
-
-    // ---- phase 1c: dC~ and dB~ as [n][row] tiles; job = (which, pair tile i,
-    // row tile); a job writes the gradient of C (which = 0) or B
-    const bool has_job = wave < 2 * NJ, isb = wave >= NJ;
-    const int jj = isb ? wave - NJ : wave;
-    const int ji = jj % PT, rt = jj / PT;
-    const int row = 16 * rt + c, tr = row / R, rr = row % R;
-    const int n0 = 16 * ji + 4 * gq;
-    // the job's own rotated operand (C~ for dC~, B~ for dB~) at its elements
-    const float *own = isb ? sm.Bs : sm.Cs;
-    float sn[4], cs[4], o1[4], o2[4];
-    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
-    if (has_job) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            sn[r] = 0.0f;
-            cs[r] = 1.0f;
-            if (rot) {
-                cs[r] = sm.acs[tr * S::AP + n0 + r];
-                sn[r] = sm.asn[tr * S::AP + n0 + r];
-            }
-            o1[r] = own[row * LB + n0 + r];
-            o2[r] = own[row * LB + n0 + r + NH];
-        }
-        if (!isb) {
-            // dC~^T[n][t] = e^{alpha_t} sum_p S[p][n] dY[t][p] + (phase 3)
-            mma2_f32<kP>(sm.Ss + 16 * ji, sm.Ss + 16 * (ji + PT), 1, LS, sm.Ys + 16 * rt * LX, 1,
-                         LX, lo, hi, c, gq);
-            const float ea = sm.eac[tr];
-            lo = lo * ea;
-            hi = hi * ea;
-        } else {
-            // dB~^T[n][s] = wbar_s sum_p Gh[p][n] X[s][p] + (phase 3)
-            mma2_f32<kP>(sm.Gs + 16 * ji, sm.Gs + 16 * (ji + PT), 1, LS, sm.Xs + 16 * rt * LX, 1,
-                         LX, lo, hi, c, gq);
-        }
-        // row . (S or Gh part): the e^alpha dy.(S C~) and wbar x.(Gh B~) terms
-        float q = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) q += lo[r] * o1[r] + hi[r] * o2[r];
-        q += __shfl_xor(q, 16, 64);
-        q += __shfl_xor(q, 32, 64);
-        if (gq == 0) atomicAdd(isb ? &sm.qv[row] : &sm.rcr[row], q);
-        if (isb) {
-            const float wb = sm.wbar[tr];
-            lo = lo * wb;
-            hi = hi * wb;
-        }
-    }
     __syncthreads();
 
-    // ---- phase 2: the band, elementwise (one (t, s) per thread in turn, s
-    // fastest): K = W e^{alpha_t - alpha_s}, M = CB o K, dCB = dM o K; the
-    // diagonal's dg sums, and off it L = dM o M (row sums, column sums) and
-    // the dw sums
-    static_assert(kRows == 32 || kRows == 64, "band rows");
-    float asum = 0.0f;   // sum of L (alpha_t - alpha_s), this thread's share
-    for (int e0 = 0; e0 < kRows * kRows; e0 += kBT) {
-        const int e = e0 + tid, t = e / kRows, s = e % kRows;
-        const int tt = t / R, ts = s / R;
-        float lam = 0.0f, dwe = 0.0f;
-        if (e < kRows * kRows) {
-            float m = 0.0f, d = 0.0f;
+    // ---- phase 2: the band, elementwise (two (t, s) a thread, s fastest): K =
+    // W e^{alpha_t - alpha_s}, M = CB o K, dCB = dM o K; the diagonal's dg
+    // sums, and off it L = dM o M (row sums, column sums), the dw sums and the
+    // sum of L (alpha_t - alpha_s).  Sums are stored, not added atomically, and
+    // added in a fixed order: the gradients repeat bit for bit.
+    float *const cpl = sm.Xs, *const cpw = sm.Xs + 2 * kWaves * kRows;   // [16][32] column sums
+    {
+        float cl = 0.0f, cw = 0.0f;
+#pragma unroll
+        for (int it = 0; it < kRows * kRows / kBT; ++it) {
+            const int e = tid + it * kBT, t = e / kRows, s = e % kRows;
+            const int tt = t / R, ts = s / R;
+            float m = 0.0f, d = 0.0f, lm = 0.0f, dgd = 0.0f;
             if (tt >= ts) {
                 const float cb = sm.Ms[t * LM + s], dm = sm.Ds[t * LM + s];
                 const float step = (sm.acum[tt] - sm.acum[ts]) + (sm.aclo[tt] - sm.aclo[ts]);
@@ -1011,45 +973,51 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
                 m = cb * K;
                 d = dm * K;
                 if (tt == ts) {
-                    atomicAdd(&sm.dgv[ts], dm * cb);
+                    dgd = dm * cb;
                 } else {
-                    lam = dm * m;
-                    dwe = dm * cb * E;
-                    asum = __builtin_fmaf(lam, step, asum);
+                    lm = dm * m;
+                    cw += dm * cb * E;
+                    asum = __builtin_fmaf(lm, step, asum);
                 }
             }
             sm.Ms[t * LM + s] = m;
             sm.Ds[t * LM + s] = d;
+            cl += lm;
+            // row sums: a row is 32 consecutive lanes of a wave
+            const float row = seg_scan<32>(lm);
+            if ((lane & 31) == 31) sm.rin[t] = row;
+            if constexpr (R >= 2) dgd += __shfl_xor(dgd, 1, 64);
+            if constexpr (R >= 4) dgd += __shfl_xor(dgd, 2, 64);
+            if (tt == ts && s % R == 0) sm.dgr[t] = dgd;
         }
-        // row sums: a row is kRows consecutive lanes of one wave
-        float rs = lam;
-        for (int off = 1; off < kRows; off <<= 1) rs += __shfl_xor(rs, off, 64);
-        if (s == 0 && e < kRows * kRows) sm.rin[t] = rs;
-        // column sums: add the wave's rows first, then one atomic per column
-        float cl = lam, cw = dwe;
-        if constexpr (kRows == 32) {
-            cl += __shfl_xor(cl, 32, 64);
-            cw += __shfl_xor(cw, 32, 64);
-        }
-        if (lane < kRows && e < kRows * kRows) {
-            atomicAdd(&sm.cinx[s], cl);
-            atomicAdd(&sm.dwi[s], cw);
-        }
+        cpl[(2 * wave + hl) * kRows + tl] = cl;
+        cpw[(2 * wave + hl) * kRows + tl] = cw;
     }
     __syncthreads();
 
     // ---- phase 3a: dX^T[p][s] += sum_t dY[t][p] M[t][s] + D dY[s][p]
-    if (has_dx) {
-        const int s = 16 * xst + c, ts = s / R, rs = s % R;
+    {
+        const int s = 16 * xst + c, ts = s / R, rr = s % R;
         f32x4 acc = xacc * sm.wbar[ts];
-        acc = mma_f32<kRows>(sm.Ys + 16 * xpt, 1, LX, sm.Ms + 16 * xst, LM, 1, acc, c, gq);
-        const size_t tg = static_cast<size_t>(ck) * QT + ts;
+#pragma unroll
+        for (int kb = 0; kb < kRows / 16; ++kb) {
+            float av[4], bv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * kb + 4 * gq + r;
+                av[r] = sm.Ys[t * LX + 16 * xpt + c];
+                bv[r] = sm.Ms[t * LM + s];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc = mfma_f32(av[r], bv[r], acc);
+        }
+        const size_t tg = t0 + ts;
         if (tg < L) {
             const size_t base = ((bb * L + tg) * H + hh) * kP * R;
             const int p0 = 16 * xpt + 4 * gq;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] += D * sm.Ys[s * LX + p0 + r];
-            st4<T, R>(g.dx, base + p0 * R + rs, acc);
+            const f32x4 yv = *reinterpret_cast<const f32x4 *>(sm.Ys + s * LX + p0);
+            acc += yv * D;
+            st4<T, R>(g.dx, base + p0 * R + rr, acc);
         }
     }
     // ---- phase 3b: the band halves of dC~ and dB~
@@ -1057,124 +1025,157 @@ __global__ void __launch_bounds__(kBT, 1) bwd_chunk_kernel(ScanLaunch a, BwdArgs
     // then the angle sums (every cos / sin was read in phase 1: asn receives
     // the dB~ half, acs the dC~ half, one lane per (token, pair)) and the
     // rotation back, d = R(psi) d~ (the transpose of fused.rs:610-617)
-    if (has_job) {
-        if (!isb)
-            mma2_f32<kRows>(sm.Bs + 16 * ji, sm.Bs + 16 * (ji + PT), 1, LB, sm.Ds + 16 * rt * LM,
-                            1, LM, lo, hi, c, gq);
-        else
-            mma2_f32<kRows>(sm.Cs + 16 * ji, sm.Cs + 16 * (ji + PT), 1, LB, sm.Ds + 16 * rt, LM, 1,
-                            lo, hi, c, gq);
-        if (rot) {
-            float *half = isb ? sm.asn : sm.acs;
+    {
+        const float *ar = isb ? sm.Cs : sm.Bs;
+#pragma unroll
+        for (int kb = 0; kb < kRows / 16; ++kb) {
+            float al[4], ah[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float cr = lo[r] * o2[r] - hi[r] * o1[r];
-                // the R rows of a token sit in adjacent lanes
-                if constexpr (R >= 2) cr += __shfl_xor(cr, 1, 64);
-                if constexpr (R >= 4) cr += __shfl_xor(cr, 2, 64);
-                if (rr == 0) half[tr * S::AP + n0 + r] = cr;
+                const float *x = ar + (16 * kb + 4 * gq + r) * LB + 16 * ji + c;
+                al[r] = x[0];
+                ah[r] = x[NH];
+            }
+#pragma unroll
+            for (int jr = 0; jr < JR; ++jr) {
+                const int rt = 16 * (rt0 + jr) + c;
+                f32x4 bv;
+                if (isb) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bv[r] = sm.Ds[(16 * kb + 4 * gq + r) * LM + rt];
+                } else {
+                    bv = *reinterpret_cast<const f32x4 *>(sm.Ds + rt * LM + 16 * kb + 4 * gq);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    lo[jr] = mfma_f32(al[r], bv[r], lo[jr]);
+                    hi[jr] = mfma_f32(ah[r], bv[r], hi[jr]);
+                }
             }
         }
-        f32x4 v1, v2;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            v1[r] = lo[r] * cs[r] - hi[r] * sn[r];
-            v2[r] = lo[r] * sn[r] + hi[r] * cs[r];
-        }
-        const size_t tg = static_cast<size_t>(ck) * QT + tr;
-        if (tg < L) {
-            void *dst = isb ? g.db : g.dc;
-            const size_t base = ((bb * L + tg) * H + hh) * N * R;
-            st4<T, R>(dst, base + n0 * R + rr, v1);
-            st4<T, R>(dst, base + (n0 + NH) * R + rr, v2);
-        }
-    }
-
-    // ---- <Gh, S> and the skip's sum dY . X, one block reduction for both
-    {
-        float gsum = 0.0f, dsum = 0.0f;
-        for (int e = tid; e < kP * N; e += kBT) {
-            const int p = e / N, n = e % N;
-            gsum += sm.Gs[p * LS + n] * sm.Ss[p * LS + n];
-        }
-        for (int e = tid; e < kRows * kP; e += kBT) {
-            const int rho = e / kP, p = e % kP;
-            dsum += sm.Ys[rho * LX + p] * sm.Xs[rho * LX + p];
-        }
-        gsum = group_sum(gsum, 64);
-        dsum = group_sum(dsum, 64);
-        asum = group_sum(asum, 64);
-        if (lane == 0) {
-            sm.red[wave] = gsum;
-            sm.red[16 + wave] = dsum;
-            sm.red[32 + wave] = asum;
+        for (int jr = 0; jr < JR; ++jr) {
+            const int row = 16 * (rt0 + jr) + c, tr = row / R, rr = row % R;
+            if (rot) {
+                float *half = isb ? sm.asn : sm.acs;
+                const f32x4 o1 = *reinterpret_cast<const f32x4 *>(own + row * LB + n0);
+                const f32x4 o2 = *reinterpret_cast<const f32x4 *>(own + row * LB + n0 + NH);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float cr = lo[jr][r] * o2[r] - hi[jr][r] * o1[r];
+                    // the R rows of a token sit in adjacent lanes
+                    if constexpr (R >= 2) cr += __shfl_xor(cr, 1, 64);
+                    if constexpr (R >= 4) cr += __shfl_xor(cr, 2, 64);
+                    if (rr == 0) half[tr * AP + n0 + r] = cr;
+                }
+            }
+            f32x4 v1, v2;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v1[r] = lo[jr][r] * cs[jr][r] - hi[jr][r] * sn[jr][r];
+                v2[r] = lo[jr][r] * sn[jr][r] + hi[jr][r] * cs[jr][r];
+            }
+            const size_t tg = t0 + tr;
+            if (tg < L) {
+                void *dst = isb ? g.db : g.dc;
+                const size_t base = ((bb * L + tg) * H + hh) * N * R;
+                st4<T, R>(dst, base + n0 * R + rr, v1);
+                st4<T, R>(dst, base + (n0 + NH) * R + rr, v2);
+            }
         }
     }
-    static_assert(kWaves <= 16, "block reduction slots");
+    // ---- <Gh, S>, the skip's sum dY . X and the band's share of da_log
+    gsum = wave_sum(gsum);
+    dsum = wave_sum(dsum);
+    asum = wave_sum(asum);
+    if (lane == 0) {
+        sm.red[0][wave] = gsum;
+        sm.red[1][wave] = dsum;
+        sm.red[2][wave] = asum;
+    }
     __syncthreads();
 
-    // ---- per-token scalars: dalpha, then da = in-chunk reverse cumsum
+    // ---- in-chunk reverse cumsums of the angle sums, over lanes in reverse
+    // token order (lane tl holds token QT - 1 - tl), four (two) pairs at once
+    if (rot) {
+        const int t = QT - 1 - tl;
+        float v[PN];
+#pragma unroll
+        for (int j = 0; j < PN; ++j)
+            v[j] = tl < QT ? sm.acs[t * AP + i0 + j] + sm.asn[t * AP + i0 + j] : 0.0f;
+        scan32<PN>(v);
+        const size_t tg = t0 + t;
+        if (tl < QT && tg < L) {
+            float *dst = w.cin + (bh * L + tg) * NH + i0;
+            if constexpr (PN == 4)
+                *reinterpret_cast<f32x4 *>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+            else
+                *reinterpret_cast<f32x2 *>(dst) = f32x2{v[0], v[1]};
+        }
+        if (tl == QT - 1) {
+#pragma unroll
+            for (int j = 0; j < PN; ++j) w.ctot[bhk * NH + i0 + j] = v[j];
+        }
+    }
+    // ---- per-token scalars (lane = row, then the row's token at lane t R)
     if (wave == 0) {
-        const float gs = group_sum(lane < kWaves ? sm.red[lane] : 0.0f, 64);
-        const float ds = group_sum(lane < kWaves ? sm.red[16 + lane] : 0.0f, 64);
-        if (lane == 0) w.pd[bhk] = ds;
-        // the alpha_E terms of the last row: sum over rows of wbar q
-        const float e = group_sum(lane < kRows ? sm.qv[lane] * sm.wbar[lane / R] : 0.0f, 64);
+        float gs = 0.0f, ds = 0.0f, pa = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kWaves; ++q) {
+            gs += sm.red[0][q];
+            ds += sm.red[1][q];
+            pa += sm.red[2][q];
+        }
+        // lanes 0-31 the column sums of L, lanes 32-63 those of dw
+        const float *cp = hl ? cpw : cpl;
+        float col = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 2 * kWaves; ++q) col += cp[q * kRows + tl];
+        const float dwi = __shfl(col, tl + 32, 64);
+        float rc = 0.0f, qv = 0.0f;
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+            rc += sm.rcr[q][tl];
+            qv += sm.qv[q][tl];
+        }
+        const int t = tl / R;   // both halves of the wave form the rows; the first keeps them
+        const float wb = sm.wbar[t];
         // da_log's share (a = -e^{a_log} dt, so da_log = sum of a da): every
         // term weighs the decay it crossed, alpha_t for the carry-in, alpha_E -
         // alpha_s for the state, alpha_E for what passes through.  The sum of
         // dt da, whose cumsums cancel most of each row and column sum, was off
-        // by up to 1.3e-5 in chunks of 64 rows.
-        const float alt = tid < QT ? sm.acum[tid] + sm.aclo[tid] : 0.0f;
+        // by up to 1.3e-5.
+        const float alt = sm.acum[t] + sm.aclo[t];
         const float ale = sm.acum[QT - 1] + sm.aclo[QT - 1];
-        const float toe = tid < QT ? (sm.acum[QT - 1] - sm.acum[tid]) + (sm.aclo[QT - 1] - sm.aclo[tid]) : 0.0f;
-        float d = 0.0f, dw = 0.0f, pa = 0.0f;
-        if (tid < QT) {
-            for (int r = 0; r < R; ++r) {
-                const int row = tid * R + r;
-                pa += sm.rcr[row] * alt + sm.qv[row] * sm.wbar[tid] * toe;
-                d += sm.rin[row] - sm.cinx[row] + sm.rcr[row] - sm.qv[row] * sm.wbar[tid];
-                dw += sm.dwi[row] + sm.qv[row] * sm.ebar[tid];
-            }
+        const float toe = (sm.acum[QT - 1] - sm.acum[t]) + (sm.aclo[QT - 1] - sm.aclo[t]);
+        const float egs = eda * gs;
+        pa += wave_sum(hl ? 0.0f : rc * alt + qv * wb * toe) + egs * ale;
+        const float et = wave_sum(hl ? 0.0f : qv * wb);
+        float d = sm.rin[tl] - col + rc - qv * wb;
+        float dw = dwi + qv * sm.ebar[t], dg = sm.dgr[tl];
+        if constexpr (R >= 2) {
+            d += __shfl_xor(d, 1, 64);
+            dw += __shfl_xor(dw, 1, 64);
+            dg += __shfl_xor(dg, 1, 64);
         }
-        pa = group_sum(pa + (lane < kWaves ? sm.red[32 + lane] : 0.0f), 64);
-        if (lane == 0) w.pa[bhk] = pa + w.eda[bhk] * gs * ale;
-        if (tid == QT - 1) d += e + w.eda[bhk] * gs;
-        if (tid < QT) sm.dal[tid] = d;
-        const size_t tg = static_cast<size_t>(ck) * QT + tid;
-        if (tid < QT && tg < L) {
-            w.dg[bh * L + tg] = sm.dgv[tid];
-            w.dw[bh * L + tg] = dw;
+        if constexpr (R >= 4) {
+            d += __shfl_xor(d, 2, 64);
+            dw += __shfl_xor(dw, 2, 64);
+            dg += __shfl_xor(dg, 2, 64);
         }
-    }
-    __syncthreads();
-    // in-chunk reverse cumsums as wave scans over lanes in reverse token order
-    // (lane l holds token QT-1-l): da from dalpha (wave 0), and per rotation
-    // pair the angle sums (pairs spread over the waves, written back to acs)
-    {
-        const int t = QT - 1 - lane;
-        const size_t tg = static_cast<size_t>(ck) * QT + t;
-        const bool live = lane < QT && tg < L;
-        if (wave == 0) {
-            const float v = seg_scan<64>(lane < QT ? sm.dal[t] : 0.0f);
-            if (live) w.da[bh * L + tg] = v;
+        // the alpha_E terms of the last token; da its reverse cumsum
+        if (t == QT - 1) d += et + egs;
+        const int rt = QT - 1 - tl;
+        float da = __shfl(d, (rt < 0 ? 0 : rt) * R, 64);
+        da = seg_scan<32>(tl < QT ? da : 0.0f);
+        if (lane == 0) {
+            w.pd[bhk] = ds;
+            w.pa[bhk] = pa;
         }
-        if (a.theta != nullptr) {
-            for (int i = wave; i < NH; i += kWaves) {
-                const float v = seg_scan<64>(
-                    lane < QT ? sm.acs[t * S::AP + i] + sm.asn[t * S::AP + i] : 0.0f);
-                if (lane < QT) sm.acs[t * S::AP + i] = v;
-                if (lane == QT - 1) w.ctot[bhk * NH + i] = v;
-            }
-        }
-    }
-    if (a.theta != nullptr) {
-        __syncthreads();
-        // token-major rows of pairs, stored whole
-        for (int e = tid; e < QT * NH; e += kBT) {
-            const int t = e / NH, i = e % NH;
-            const size_t tg = static_cast<size_t>(ck) * QT + t;
-            if (tg < L) w.cin[(bh * L + tg) * NH + i] = sm.acs[t * S::AP + i];
+        if (lane < QT && t0 + rt < L) w.da[bh * L + t0 + rt] = da;
+        if (lane < kRows && tl % R == 0 && t0 + t < L) {
+            w.dg[bh * L + t0 + t] = dg;
+            w.dw[bh * L + t0 + t] = dw;
         }
     }
 }
@@ -1208,7 +1209,7 @@ __global__ void bwd_angle_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
 // dlambda_t = dt_t (dg_t + dw_t) - dt_t dw_{t-1}    (trapezoid_weights_backward,
 // fused.rs:2513-2549), plus the carried-in boundary term at t = 0.
 // One workgroup per chunk, one wave per token, lane = rotation pair.
-template <typename T, int N, int R, int kRows>
+template <typename T, int N, int R>
 __global__ void __launch_bounds__(256) bwd_token_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
     constexpr int NH = N / 2, QT = kRows / R;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1407,9 +1408,10 @@ hipError_t set_lds(K kern, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
 
-template <typename T, int N, int R, int RW>
+template <typename T, int N, int R>
 hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStream_t s) {
-    const int nck = static_cast<int>((a.seq + RW / R - 1) / (RW / R));
+    constexpr int QT = kRows / R;
+    const int nck = static_cast<int>((a.seq + QT - 1) / QT);
     const size_t bh = a.batch * a.heads, bhk = bh * nck;
     const BwdLayout l = bwd_layout(bh, nck, a.seq, N, R);
     BwdWs w;
@@ -1430,9 +1432,9 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
     w.lux = f(l.lux);
     w.lub = f(l.lub);
 
-    static_assert(sizeof(Smem<N, R, RW>) <= 160 * 1024, "chunk kernel LDS over 160 KB");
-    const size_t lds = sizeof(Smem<N, R, RW>);
-    static const hipError_t a2 = set_lds(bwd_chunk_kernel<T, N, R, RW>, lds);
+    static_assert(sizeof(Smem<N, R>) <= 80 * 1024, "two chunk workgroups a CU");
+    const size_t lds = sizeof(Smem<N, R>);
+    static const hipError_t a2 = set_lds(bwd_chunk_kernel<T, N, R>, lds);
     if (a2 != hipSuccess) return a2;
     hipError_t e;
     BwdArgs gm = g;
@@ -1443,16 +1445,16 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
         if (a.theta != nullptr) gm.dangle_out = w.seed;
     }
     const BwdArgs &g2 = gm;
-    hipLaunchKernelGGL((bwd_passes_kernel<T, N, R, RW>), dim3(2 * bh * (N / 32)), dim3(256), 0, s, a, g2, w,
+    hipLaunchKernelGGL((bwd_passes_kernel<T, N, R>), dim3(2 * bh * (N / 32)), dim3(256), 0, s, a, g2, w,
                        nck);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((bwd_chunk_kernel<T, N, R, RW>), dim3(bhk), dim3(kBT), lds, s, a, g2, w, nck);
+    hipLaunchKernelGGL((bwd_chunk_kernel<T, N, R>), dim3(bhk), dim3(kBT), lds, s, a, g2, w, nck);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (a.theta != nullptr) {
         hipLaunchKernelGGL((bwd_angle_kernel<N>), dim3(bh), dim3(64), 0, s, a, g2, w, nck);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((bwd_token_kernel<T, N, R, RW>), dim3(bhk), dim3(256), 0, s, a, g2, w, nck);
+    hipLaunchKernelGGL((bwd_token_kernel<T, N, R>), dim3(bhk), dim3(256), 0, s, a, g2, w, nck);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(bwd_head_kernel, dim3(a.heads), dim3(256), 0, s, a, g2, w, nck);
     if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -1463,17 +1465,17 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
     return hipSuccess;
 }
 
-template <typename T, int N64ROWS>
+template <typename T>
 hipError_t launch_bwd_t(const ScanLaunch &a, const BwdArgs &g, char *ws, hipStream_t s) {
     const size_t n = a.d_state, r = a.rank;
     if (n == 128) {
-        if (r == 1) return launch_bwd<T, 128, 1, 32>(a, g, ws, s);
-        if (r == 2) return launch_bwd<T, 128, 2, 32>(a, g, ws, s);
-        if (r == 4) return launch_bwd<T, 128, 4, 32>(a, g, ws, s);
+        if (r == 1) return launch_bwd<T, 128, 1>(a, g, ws, s);
+        if (r == 2) return launch_bwd<T, 128, 2>(a, g, ws, s);
+        if (r == 4) return launch_bwd<T, 128, 4>(a, g, ws, s);
     } else if (n == 64) {
-        if (r == 1) return launch_bwd<T, 64, 1, N64ROWS>(a, g, ws, s);
-        if (r == 2) return launch_bwd<T, 64, 2, N64ROWS>(a, g, ws, s);
-        if (r == 4) return launch_bwd<T, 64, 4, N64ROWS>(a, g, ws, s);
+        if (r == 1) return launch_bwd<T, 64, 1>(a, g, ws, s);
+        if (r == 2) return launch_bwd<T, 64, 2>(a, g, ws, s);
+        if (r == 4) return launch_bwd<T, 64, 4>(a, g, ws, s);
     }
     return hipErrorNotSupported;
 }
@@ -1486,7 +1488,7 @@ bool scan_backward_supported(const ScanLaunch &a) {
 
 size_t scan_backward_workspace(const ScanLaunch &a) {
     if (!scan_backward_supported(a)) return 0;
-    const size_t qt = static_cast<size_t>(scan_backward_rows(a)) / a.rank;
+    const size_t qt = kRows / a.rank;
     const size_t nck = (a.seq + qt - 1) / qt;
     return bwd_layout(a.batch * a.heads, nck, a.seq, a.d_state, a.rank).total;
 }
@@ -1511,8 +1513,8 @@ hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *
     g.dlast_u0 = gr.dlast_u0;
     g.dangle0 = gr.dangle0;
     char *ws = static_cast<char *>(workspace);
-    if (a.bf16) return launch_bwd_t<bf16_t, 64>(a, g, ws, stream);
-    return launch_bwd_t<float, 32>(a, g, ws, stream);
+    if (a.bf16) return launch_bwd_t<bf16_t>(a, g, ws, stream);
+    return launch_bwd_t<float>(a, g, ws, stream);
 }
 
 }  // namespace m3
