@@ -154,8 +154,12 @@ __device__ __forceinline__ void split_decay(float dt, float A, float &hi, float 
 // fused multiply-adds, good while the multiple is an exact f32 integer and the
 // last part's error stays below the result's: |x| < 2^13 here, past which the
 // library's sincosf takes over), then the Taylor polynomials to r^9 and r^10
-// on |r| <= pi / 4 and the quadrant's swap and signs.  About a quarter of
-// sincosf's instructions, and the backward forms three per (token, pair).
+// on |r| <= pi / 4 and the quadrant's swap and signs: within 6.9e-8 of f64 (an
+// exact result rounded: 3.0e-8).  34 instructions where sincosf compiles to 147,
+// both its paths counted, and the backward forms three per (token, pair): a
+// forward and backward of 2 x 4096 tokens, 8 heads, d_state 64, bf16 storage,
+// 318 -> 305 us, of 1 x 1154, 8 heads, 128, rank 4, f32, 434 -> 418; no change
+// where the chip is full (8 x 2048, 12 heads).
 __device__ __forceinline__ void sincos_turn(float x, float &sn, float &cs) {
     const float k = rintf(x * 0.63661977236758134f);                 // 2 / pi
     float r = __builtin_fmaf(k, -1.5707963267948966f, x);            // pi / 2 rounded to f32,
@@ -293,20 +297,28 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 // in-chunk angles (the scans of the chunk kernel, so every value is the same),
 // rotates its 32 columns of B (or C) into LDS scaled by wbar (or not), stages
 // X (or e^alpha dY) as rows, and forms U (or V) by f32 MFMA.  The raw inputs
-// of the next chunks are loaded ahead into registers, four elements a load; no
-// per-chunk record but S_k (Gh_k) leaves the workgroup.  At batch 8 x 2048, 12
-// heads, d_state 128 the two passes take 204 us (226 with an element a load and
-// X transposed in LDS, whose writes fell on a quarter of the banks).
+// are loaded ahead into registers, four elements a load; no per-chunk record
+// but S_k (Gh_k) leaves the workgroup.
+//
+// The recurrence is serial over the chunks, so with few sequences the time is
+// the chain of one step (barriers, scans, sine, products): a step is two
+// chunks, whose chains run side by side between the same two barriers.  A
+// forward and backward against one chunk a step: 2 x 4096 tokens, 8 heads,
+// d_state 64, bf16 storage, 305 -> 261 us; 1 x 1154, 8 heads, 128, rank 4, f32,
+// 418 -> 361; 2 x 1777, 12 heads, 128, f32, 243 -> 229.  With the chip full it
+// is bandwidth and issue that bound them: batch 8 x 2048, 12 heads, d_state 128,
+// 205 us either way, for 500 MB (100 us at the rate of a large copy).
 template <int R>
 struct PassSmem {
     static constexpr int QT = kRows / R, LDR = kRows + 4, LX = kP + 4, AP = 17;
-    float As[32 * LDR];      // rotated columns: [column][rho], lo pairs then hi
-    float Xs[kRows * LX];    // X or e^alpha dY: [rho][p]
-    // per chunk parity: cos / sin of the in-chunk angle [token][pair], the
-    // token scalars, the decay prefix and the per-token scale
-    float acs[2][QT * AP], asn[2][QT * AP];
-    float acum[2][QT], aclo[2][QT], ww[2][QT], scal[2][QT];
-    float phi[16];           // the sequence's angle total per pair (reverse pass)
+    // per chunk of the step
+    float As[2][32 * LDR];      // rotated columns: [column][rho], lo pairs then hi
+    float Xs[2][kRows * LX];    // X or e^alpha dY: [rho][p]
+    // per step parity and chunk: cos / sin of the in-chunk angle [token][pair],
+    // the decay prefix, the token and per-token scales
+    float acs[2][2][QT * AP], asn[2][2][QT * AP];
+    float acum[2][2][QT], aclo[2][2][QT], ww[2][2][QT], scal[2][2][QT];
+    float phi[2][16];           // the sequence's angle total per pair (reverse pass)
     float red[16];
 };
 
@@ -315,10 +327,8 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                            size_t blk, PassSmem<R> &sm) {
     using S = PassSmem<R>;
     constexpr int NTN = N / 16, HT = NTN / 2, NH = N / 2, QT = S::QT, LDR = S::LDR, LX = S::LX, AP = S::AP;
-    constexpr int PN = 2;                       // pairs a half-wave scans
-    constexpr int NB = QT * 4 * R;              // four-element items of B (or C): 128
-    constexpr int JX = 2;                       // ... of X (or dY) per thread: 512
-    constexpr int D = 3;                        // chunks loaded ahead
+    constexpr int PN = 4;                       // pairs a half-wave scans
+    constexpr int JX = 2;                       // four-element items of X (dY) per thread and chunk
     const int tid = threadIdx.x, lane = tid & 63;
     const int pt = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, gq = lane >> 4;
@@ -330,8 +340,8 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
     const float A = 0.0f - expf(a.a_log[hh]);
     const int p0 = 16 * pt + 4 * gq, nlo = 16 * i1 + c;
     const size_t sbase = bh * kP * N + static_cast<size_t>(p0) * N + nlo;   // state (p0, nlo)
-    const int tl = lane & 31, hl = lane >> 5;   // the angle scans: lane -> token, pairs ip ..
-    const int ip = 4 * pt + PN * hl;
+    const int tl = lane & 31, hl = lane >> 5;   // the scans: lane -> token tl of the step's chunk hl
+    const int ip = PN * pt;                     // and pairs ip ..
     auto rot4 = [](f32x4 &lo, f32x4 &hi, float cs, float sn) {
         const f32x4 l = lo;
         lo = l * cs - hi * sn;
@@ -352,14 +362,18 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
         }
     };
 
+    // Steps of two chunks: half the barriers, and the chains of one chunk
+    // (scan, sine, products) beside the other's.  A second chunk past the
+    // sequence's end is all zeros: decay one, no angle, nothing added.
+    const int ns = (nck + 1) / 2;
     struct In {
         float dt, lam, dtn, lamn, dtl;
         uint32_t th[PN];
-        Raw4<T> b1, b2, x[JX];
+        Raw4<T> b1, b2, x[2 * JX];
     };
-    // Chunk k's raw inputs, by buffer loads over this sequence's tokens: a
+    // Step s's raw inputs, by buffer loads over this sequence's tokens: a
     // token at or past the sequence end reads as zero.  A thread's items sit
-    // at fixed byte offsets from its chunk-0 offsets.
+    // at fixed byte offsets from its step-0 offsets.
     constexpr uint32_t SZ = sizeof(T);
     const scan::SeqBufs rs = scan::seq_bufs<T, N, kP, R>(a, bb, hh);
     const rsrc_t rbc = FWD ? rs.b : rs.c;
@@ -367,50 +381,47 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                            : make_rsrc(static_cast<const char *>(g.dy) + (bb * L * H + hh) * kP * R * SZ,
                                        static_cast<uint32_t>((L * H - hh) * kP * R * SZ));
     const bool xal = FWD || (reinterpret_cast<uintptr_t>(g.dy) & 3u) == 0;
-    const uint32_t o_s = (tid < QT ? tid : 0) * rs.tok_s;
-    const uint32_t o_tl = (tl < QT ? tl : 0) * rs.tok_s;
-    const uint32_t o_th = (tl < QT ? tl : 0) * rs.tok_th + (16 * i1 + ip) * SZ;
-    const int tb = tid / (4 * R), eb = (tid % (4 * R)) * 4;      // items tid < NB
-    const uint32_t o_bc = tb * rs.tok_bc + (16 * i1 * R + eb) * SZ;
-    const int tx = tid / (16 * R), ex = (tid % (16 * R)) * 4;    // items tid + 256 j
+    const int tk = hl * QT + (tl < QT ? tl : 0);                 // this lane's token of the step
+    const uint32_t o_s = tk * rs.tok_s;
+    const uint32_t o_th = tk * rs.tok_th + (16 * i1 + ip) * SZ;
+    // B (C) items: 128 a chunk, one a thread; X (dY): 512 a chunk
+    const int tb = tid / (4 * R) % QT, sb_ = tid >> 7, eb = (tid % (4 * R)) * 4;
+    const uint32_t o_bc = (sb_ * QT + tb) * rs.tok_bc + (16 * i1 * R + eb) * SZ;
+    const int tx = tid / (16 * R), ex = (tid % (16 * R)) * 4;    // item tid + 256 j: token tx + j XJ
+    constexpr int XJ = 256 / (16 * R);
     const uint32_t o_xy = tx * rs.tok_x + ex * SZ;
-    const uint32_t xy_j = (256 / (16 * R)) * rs.tok_x;
-    auto load = [&](int k, In &d) {
-        const int kk = k < 0 ? 0 : (k < nck ? k : nck - 1);   // outside: re-read, unused
-        const uint32_t t0 = static_cast<uint32_t>(kk) * QT;
-        d.dt = bldf(rs.s0, o_s + t0 * rs.tok_s);
-        d.lam = bldf(rs.s1, o_s + t0 * rs.tok_s);
-        d.dtn = bldf(rs.s0, o_s + (t0 + 1) * rs.tok_s);
-        d.lamn = bldf(rs.s1, o_s + (t0 + 1) * rs.tok_s);
-        if (rot) {
-            d.dtl = bldf(rs.s0, o_tl + t0 * rs.tok_s);
-            ldth<T, PN>(rs.th, o_th + t0 * rs.tok_th, d.th);
+    auto load = [&](int st, In &d) {
+        const int ss = st < 0 ? 0 : (st < ns ? st : ns - 1);   // outside: re-read, unused
+        const uint32_t t0 = static_cast<uint32_t>(ss) * (2 * QT);
+        d.dtl = bldf(rs.s0, o_s + t0 * rs.tok_s);
+        if (pt == 0) {
+            d.lam = bldf(rs.s1, o_s + t0 * rs.tok_s);
+            d.dtn = bldf(rs.s0, o_s + (t0 + 1) * rs.tok_s);
+            d.lamn = bldf(rs.s1, o_s + (t0 + 1) * rs.tok_s);
         }
-        if (tid < NB) {
-            ld4(d.b1, rbc, o_bc + t0 * rs.tok_bc);
-            ld4(d.b2, rbc, o_bc + t0 * rs.tok_bc + NH * R * SZ);
-        }
+        if (rot) ldth<T, PN>(rs.th, o_th + t0 * rs.tok_th, d.th);
+        ld4(d.b1, rbc, o_bc + t0 * rs.tok_bc);
+        ld4(d.b2, rbc, o_bc + t0 * rs.tok_bc + NH * R * SZ);
 #pragma unroll
-        for (int j = 0; j < JX; ++j) ld4(d.x[j], rxy, o_xy + t0 * rs.tok_x + j * xy_j, xal);
+        for (int j = 0; j < 2 * JX; ++j) ld4(d.x[j], rxy, o_xy + (t0 + j * XJ) * rs.tok_x, xal);
     };
-    // The chunk's work in four pieces, software-pipelined over two sets of
-    // the per-chunk tables (sb = chunk parity): the scalars and decay prefix
-    // (p1) and the angles (p2) of chunk k + 1 run in the same two barrier
-    // phases as the staging (p3) and the products (p4) of chunk k.
-    //   phase X: p3(k), p1(k + 1);  barrier;  phase Y: p4(k), p2(k + 1);  barrier
+    // The step's work in four pieces, software-pipelined over two sets of the
+    // per-step tables (sb = step parity): the scalars and decay prefixes (p1)
+    // and the angles (p2) of the next step run in the same two barrier phases
+    // as the staging (p3) and the products (p4) of this one.
+    //   phase X: p3(s), p1(s + 1);  barrier;  phase Y: p4(s), p2(s + 1);  barrier
     // token scalars, the decay prefix (fused.rs:2494-2498)
     auto p1 = [&](const In &d, int sb) {
-        if (tid < QT) {
-            sm.ww[sb][tid] = d.lam * d.dt + (1.0f - d.lamn) * d.dtn;
-        }
         if (pt == 0) {
+            const float dt = tl < QT ? d.dtl : 0.0f;
             float hi, lo;
-            split_decay(tid < QT ? d.dt : 0.0f, A, hi, lo);
+            split_decay(dt, A, hi, lo);
             hi = seg_scan<32>(hi);
             lo = seg_scan<32>(lo);
-            if (lane < QT) {
-                sm.acum[sb][lane] = hi;
-                sm.aclo[sb][lane] = lo;
+            if (tl < QT) {
+                sm.ww[sb][hl][tl] = d.lam * dt + (1.0f - d.lamn) * d.dtn;
+                sm.acum[sb][hl][tl] = hi;
+                sm.aclo[sb][hl][tl] = lo;
             }
         }
     };
@@ -428,85 +439,94 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                 for (int j = 0; j < PN; ++j) {
                     float sv, cv;
                     sincos_turn(v[j], sv, cv);
-                    sm.acs[sb][tl * AP + ip + j] = cv;
-                    sm.asn[sb][tl * AP + ip + j] = sv;
+                    sm.acs[sb][hl][tl * AP + ip + j] = cv;
+                    sm.asn[sb][hl][tl * AP + ip + j] = sv;
                 }
             }
         }
-        if (tid < QT) {
-            const float hi = sm.acum[sb][tid], lo = sm.aclo[sb][tid];
-            sm.scal[sb][tid] = FWD ? clamp_exp((sm.acum[sb][QT - 1] - hi) + (sm.aclo[sb][QT - 1] - lo)) *
-                                         sm.ww[sb][tid]
-                                   : clamp_exp(hi + lo);
+        if (pt == 0 && tl < QT) {
+            const float hi = sm.acum[sb][hl][tl], lo = sm.aclo[sb][hl][tl];
+            sm.scal[sb][hl][tl] = FWD ? clamp_exp((sm.acum[sb][hl][QT - 1] - hi) + (sm.aclo[sb][hl][QT - 1] - lo)) *
+                                            sm.ww[sb][hl][tl]
+                                      : clamp_exp(hi + lo);
         }
     };
     // rotation by the negative in-chunk angle (fused.rs:610-617) into LDS;
-    // the chunk decay
-    auto p3 = [&](const In &d, int sb, float &e) {
-        if (tid < NB) {
+    // the chunks' decays
+    auto p3 = [&](const In &d, int sb, float (&e)[2]) {
+        {
             float b1[4], b2[4];
             un4(d.b1, b1);
             un4(d.b2, b2);
-            const float sc = FWD ? sm.scal[sb][tb] : 1.0f;
+            const float sc = FWD ? sm.scal[sb][sb_][tb] : 1.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int q = (eb + j) / R, rho = tb * R + (eb + j) % R;
                 float sn = 0.0f, cs = 1.0f;
                 if (rot) {
-                    cs = sm.acs[sb][tb * AP + q];
-                    sn = sm.asn[sb][tb * AP + q];
+                    cs = sm.acs[sb][sb_][tb * AP + q];
+                    sn = sm.asn[sb][sb_][tb * AP + q];
                 }
-                sm.As[q * LDR + rho] = (b1[j] * cs + b2[j] * sn) * sc;
-                sm.As[(16 + q) * LDR + rho] = (-b1[j] * sn + b2[j] * cs) * sc;
+                sm.As[sb_][q * LDR + rho] = (b1[j] * cs + b2[j] * sn) * sc;
+                sm.As[sb_][(16 + q) * LDR + rho] = (-b1[j] * sn + b2[j] * cs) * sc;
             }
         }
 #pragma unroll
-        for (int j = 0; j < JX; ++j) {
-            const int t = tx + j * (256 / (16 * R));
+        for (int j = 0; j < 2 * JX; ++j) {
+            const int u = j / JX, t = tx + (j % JX) * XJ;
             float v[4];
             un4(d.x[j], v);
             if constexpr (!FWD) {
-                const float sc = sm.scal[sb][t];
+                const float sc = sm.scal[sb][u][t];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] *= sc;
             }
-            put4<R>(sm.Xs, LX, t, ex, v);
+            put4<R>(sm.Xs[u], LX, t, ex, v);
         }
-        e = clamp_exp(sm.acum[sb][QT - 1] + sm.aclo[sb][QT - 1]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) e[u] = clamp_exp(sm.acum[sb][u][QT - 1] + sm.aclo[sb][u][QT - 1]);
     };
-    // U (V) at this lane's (p, n): A(m = p, k = rho), B(k = rho, col = n), with
-    // k slot 4 g + r of a block of 16 the rho of MFMA r's lane group g; the
-    // rotation by the chunk's angle totals, the in-chunk angles of its last row
-    auto p4 = [&](int sb, f32x4 &alo, f32x4 &ahi, float &pc, float &ps) {
-        alo = f32x4{0.f, 0.f, 0.f, 0.f};
-        ahi = alo;
+    // U (V) of the two chunks at this lane's (p, n): A(m = p, k = rho), B(k =
+    // rho, col = n), with k slot 4 g + r of a block of 16 the rho of MFMA r's
+    // lane group g; the rotations by the chunks' angle totals, the in-chunk
+    // angles of their last rows
+    auto p4 = [&](int sb, f32x4 (&alo)[2], f32x4 (&ahi)[2], float (&pc)[2], float (&ps)[2]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) alo[u] = ahi[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < kRows / 16; ++kb) {
-            const f32x4 bl = *reinterpret_cast<const f32x4 *>(sm.As + c * LDR + 16 * kb + 4 * gq);
-            const f32x4 bhv = *reinterpret_cast<const f32x4 *>(sm.As + (16 + c) * LDR + 16 * kb + 4 * gq);
-            float av[4];
+            f32x4 bl[2], bhv[2];
+            float av[2][4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) av[r] = sm.Xs[(16 * kb + 4 * gq + r) * LX + 16 * pt + c];
+            for (int u = 0; u < 2; ++u) {
+                bl[u] = *reinterpret_cast<const f32x4 *>(sm.As[u] + c * LDR + 16 * kb + 4 * gq);
+                bhv[u] = *reinterpret_cast<const f32x4 *>(sm.As[u] + (16 + c) * LDR + 16 * kb + 4 * gq);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                alo = mfma_f32(av[r], bl[r], alo);
-                ahi = mfma_f32(av[r], bhv[r], ahi);
+                for (int r = 0; r < 4; ++r) av[u][r] = sm.Xs[u][(16 * kb + 4 * gq + r) * LX + 16 * pt + c];
             }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    alo[u] = mfma_f32(av[u][r], bl[u][r], alo[u]);
+                    ahi[u] = mfma_f32(av[u][r], bhv[u][r], ahi[u]);
+                }
         }
-        pc = 1.0f;
-        ps = 0.0f;
-        if (rot) {
-            pc = sm.acs[sb][(QT - 1) * AP + c];
-            ps = sm.asn[sb][(QT - 1) * AP + c];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            pc[u] = rot ? sm.acs[sb][u][(QT - 1) * AP + c] : 1.0f;
+            ps[u] = rot ? sm.asn[sb][u][(QT - 1) * AP + c] : 0.0f;
         }
     };
-    auto offs = [&](int k, size_t &o, size_t &oh) {
-        const size_t bhk = bh * nck + k;
-        o = bhk * kP * N + ((pt * NTN + i1) * 64 + lane) * 4;
-        oh = bhk * kP * N + ((pt * NTN + i1 + HT) * 64 + lane) * 4;
+    auto put_record = [&](float *base, int k, f32x4 lo, f32x4 hi) {
+        if (k >= nck) return;
+        float *o = base + (bh * nck + k) * kP * N + ((pt * NTN + i1) * 64 + lane) * 4;
+        *reinterpret_cast<f32x4 *>(o) = lo;
+        *reinterpret_cast<f32x4 *>(o + HT * 256) = hi;
     };
 
     f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+    In d[2];
     if constexpr (FWD) {
         if (a.h0 != nullptr) {
             ld_state(a.h0, lo, hi);
@@ -524,38 +544,35 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             sincosf(a.angle0[bh * NH + nlo], &sn, &cs);
             rot4(lo, hi, cs, sn);
         }
-        In d[D];
-#pragma unroll
-        for (int j = 0; j < D; ++j) load(j, d[j]);
+        load(0, d[0]);
+        load(1, d[1]);
         p1(d[0], 0);
         __syncthreads();
         p2(d[0], 0);
         __syncthreads();
-        for (int k = 0; k < nck; k += D) {
+        for (int k = 0; k < ns; k += 2) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) {
-                const int kc = k + j;
-                if (kc < nck) {
-                    const int sb = kc & 1;
-                    const bool more = kc + 1 < nck;
-                    float e, pc, ps;
-                    p3(d[j], sb, e);
-                    if (more) p1(d[(j + 1) % D], sb ^ 1);
+            for (int sb = 0; sb < 2; ++sb) {
+                const int st = k + sb;
+                if (st < ns) {
+                    float e[2], pc[2], ps[2];
+                    p3(d[sb], sb, e);
+                    p1(d[sb ^ 1], sb ^ 1);
+                    load(st + 2, d[sb]);
                     __syncthreads();
-                    f32x4 ulo, uhi;
+                    f32x4 ulo[2], uhi[2];
                     p4(sb, ulo, uhi, pc, ps);
-                    if (more) p2(d[(j + 1) % D], sb ^ 1);
-                    size_t o, oh;
-                    offs(kc, o, oh);
-                    *reinterpret_cast<f32x4 *>(w.s + o) = lo;
-                    *reinterpret_cast<f32x4 *>(w.s + oh) = hi;
-                    lo = lo * e + ulo;
-                    hi = hi * e + uhi;
-                    if (rot) rot4(lo, hi, pc, ps);   // R(Phi_k)
-                    if (i1 == 0 && tid == 0) w.eda[bh * nck + kc] = e;
+                    p2(d[sb ^ 1], sb ^ 1);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        put_record(w.s, 2 * st + u, lo, hi);
+                        lo = lo * e[u] + ulo[u];
+                        hi = hi * e[u] + uhi[u];
+                        if (rot && 2 * st + u < nck) rot4(lo, hi, pc[u], ps[u]);   // R(Phi_k)
+                        if (i1 == 0 && tid == 0 && 2 * st + u < nck) w.eda[bh * nck + 2 * st + u] = e[u];
+                    }
                     __syncthreads();
                 }
-                load(kc + D, d[j]);
             }
         }
     } else {
@@ -563,24 +580,24 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             ld_state(g.dh_out, lo, hi);
             if (rot) {
                 // phi_end = angle0 + sum_k Phi_k: the final frame, S_C = R(phi_end) h_out.
-                // Each Phi_k is the in-chunk scan's last value, summed in chunk order.
-                constexpr int DT = 8;
+                // Each Phi_k is the in-chunk scan's last value; a half-wave sums
+                // every second chunk.
+                constexpr int DT = 4;
                 float ph[PN], dq[DT];
                 uint32_t tq[DT][PN];
 #pragma unroll
-                for (int j = 0; j < PN; ++j)
-                    ph[j] = a.angle0 != nullptr ? a.angle0[bh * NH + 16 * i1 + ip + j] : 0.0f;
-                auto tload = [&](int k, float &dv, uint32_t (&tv)[PN]) {
-                    const uint32_t t0 = static_cast<uint32_t>(k < nck ? k : nck - 1) * QT;
-                    dv = bldf(rs.s0, o_tl + t0 * rs.tok_s);
+                for (int j = 0; j < PN; ++j) ph[j] = 0.0f;
+                auto tload = [&](int st, float &dv, uint32_t (&tv)[PN]) {
+                    const uint32_t t0 = static_cast<uint32_t>(st < ns ? st : ns - 1) * (2 * QT);
+                    dv = bldf(rs.s0, o_s + t0 * rs.tok_s);
                     ldth<T, PN>(rs.th, o_th + t0 * rs.tok_th, tv);
                 };
 #pragma unroll
                 for (int q = 0; q < DT; ++q) tload(q, dq[q], tq[q]);
-                for (int k = 0; k < nck; k += DT) {
+                for (int k = 0; k < ns; k += DT) {
 #pragma unroll
                     for (int q = 0; q < DT; ++q) {
-                        if (k + q < nck) {
+                        if (k + q < ns) {
                             float v[PN];
                             unth<T, PN>(tq[q], v);
 #pragma unroll
@@ -594,47 +611,44 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                 }
                 if (tl == QT - 1) {
 #pragma unroll
-                    for (int j = 0; j < PN; ++j) sm.phi[ip + j] = ph[j];
+                    for (int j = 0; j < PN; ++j) sm.phi[hl][ip + j] = ph[j];
                 }
                 __syncthreads();
-                const float pe = sm.phi[c];
-                __syncthreads();
+                const float pe = (a.angle0 != nullptr ? a.angle0[bh * NH + nlo] : 0.0f) + sm.phi[0][c] + sm.phi[1][c];
                 float sn, cs;
                 sincosf(pe, &sn, &cs);
                 rot4(lo, hi, cs, sn);
             }
         }
-        In d[D];
-#pragma unroll
-        for (int j = 0; j < D; ++j) load(nck - 1 - j, d[j]);
-        p1(d[0], (nck - 1) & 1);
+        const int top = (ns - 1) | 1;   // the odd step of the last two; past the end if ns is odd
+        load(top < ns ? top : top - 2, d[1]);
+        load(top - 1, d[0]);
+        if (top < ns) p1(d[1], 1); else p1(d[0], 0);
         __syncthreads();
-        p2(d[0], (nck - 1) & 1);
+        if (top < ns) p2(d[1], 1); else p2(d[0], 0);
         __syncthreads();
-        for (int k = nck - 1; k >= 0; k -= D) {
+        for (int k = top; k >= 0; k -= 2) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) {
-                const int kc = k - j;
-                if (kc >= 0) {
-                    const int sb = kc & 1;
-                    const bool more = kc > 0;
-                    float e, pc, ps;
-                    p3(d[j], sb, e);
-                    if (more) p1(d[(j + 1) % D], sb ^ 1);
+            for (int q = 0; q < 2; ++q) {
+                const int sb = 1 - q, st = k - q;
+                if (st < ns) {
+                    float e[2], pc[2], ps[2];
+                    p3(d[sb], sb, e);
+                    p1(d[sb ^ 1], sb ^ 1);
+                    load(st - 2, d[sb]);
                     __syncthreads();
-                    f32x4 vlo, vhi;
+                    f32x4 vlo[2], vhi[2];
                     p4(sb, vlo, vhi, pc, ps);
-                    if (more) p2(d[(j + 1) % D], sb ^ 1);
-                    if (rot) rot4(lo, hi, pc, -ps);   // R(-Phi_k)
-                    size_t o, oh;
-                    offs(kc, o, oh);
-                    *reinterpret_cast<f32x4 *>(w.gh + o) = lo;
-                    *reinterpret_cast<f32x4 *>(w.gh + oh) = hi;
-                    lo = lo * e + vlo;
-                    hi = hi * e + vhi;
+                    p2(d[sb ^ 1], sb ^ 1);
+#pragma unroll
+                    for (int u = 1; u >= 0; --u) {
+                        if (rot && 2 * st + u < nck) rot4(lo, hi, pc[u], -ps[u]);   // R(-Phi_k)
+                        put_record(w.gh, 2 * st + u, lo, hi);
+                        lo = lo * e[u] + vlo[u];
+                        hi = hi * e[u] + vhi[u];
+                    }
                     __syncthreads();
                 }
-                load(kc - D, d[j]);
             }
         }
         // into the global frame: dZ0 = R(-angle0) G_0

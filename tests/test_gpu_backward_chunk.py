@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 EDGES = [(2, T, 3, 64, N, R, True, True, True, dt)
          for N, R in ((64, 1), (64, 2), (64, 4), (128, 1), (128, 2), (128, 4))
-         for T, dt in ((32 // R, "f32"), (32 // R + 1, "bf16"), (3 * 32 // R - 1, "f32"))]
+         for T, dt in ((32 // R, "f32"), (32 // R + 1, "bf16"), (3 * 32 // R - 1, "f32"),
+                       (4 * 32 // R + 1, "f32"), (5 * 32 // R + 3, "bf16"))]
 
 
 @pytest.mark.parametrize("case", EDGES, ids=[repr(c[1:]) for c in EDGES])
