@@ -2476,6 +2476,8 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t H = a.heads, L = a.seq;
     const size_t bb = bh / H, hh = bh % H;
+    const bool last_seg = seg == nseg - 1;
+    const bool agg = seg > 0 && !last_seg;   // nothing reads the first's aggregate, or the last's records
     // ---- the segment's aggregate: U (rounded to bf16, the record's values),
     //      its decay, and per pair its wrapped angle total with cos and sin
     const int lg = lane >> 4, lc = lane & 15;
@@ -2489,7 +2491,7 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
             q[r] = static_cast<__bf16>(sacc[f][0][r]);
             q[4 + r] = static_cast<__bf16>(sacc[f][1][r]);
         }
-        if (seg > 0)
+        if (agg)
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, q), ru,
                                                    static_cast<uint32_t>((urec + rec_off<NTN>(f, lane)) * 2), 0, kCoh);
     }
@@ -2501,19 +2503,20 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
         sm.ang[tid] = tot;
         sm.cph[tid] = tc;
         sm.sph[tid] = ts;
-        if (seg > 0) {
+        if (agg) {
             __hip_atomic_store(&ws.phi[bhs * NH + tid], tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ws.cph[bhs * NH + tid], tc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ws.sph[bhs * NH + tid], ts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    if (seg > 0 && tid == 0)
-        __hip_atomic_store(&ws.eda[bhs], eacc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());   // the record's stores are done
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (agg) {
+        if (tid == 0) __hip_atomic_store(&ws.eda[bhs], eacc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());   // the record's stores are done
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    }
     __syncthreads();
-    if (seg > 0 && tid == 0)
+    if (agg && tid == 0)
         __hip_atomic_store(&ws.flag[bhs], (epoch << 2) | kFlagAgg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // ---- the state entering the segment, S_j (in its frame), and the angle
@@ -2525,6 +2528,7 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
         return static_cast<uint32_t>(((((rec * 4 + wave) * NF + f) * 2 + q) * 64 + lane) * 16);
     };
     const int p = 16 * wave + lc;
+    float *const csn = reinterpret_cast<float *>(sm.band);   // [cos, sin x NH]: the band is dead
     if (seg == 0) {
         // S_0 = R(angle0) (h0 + (1 - lambda_0) dt_0 last_u0)   (scan.rs:521-535)
         const float *h0 = a.mode_raw ? a.h0 : a.init_state;
@@ -2534,6 +2538,13 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
             const size_t i0s = (bb * L) * H + hh;
             first = (1.0f - a.lambda[i0s]) * a.dt[i0s];
         }
+        const bool turned = a.theta != nullptr && a.angle0 != nullptr;
+        if (tid < NH) {
+            const float ph = turned ? a.angle0[bh * NH + tid] : 0.0f;
+            sm.phc[tid] = ph;
+            if (turned) sincosf(ph, &csn[NH + tid], &csn[tid]);
+        }
+        __syncthreads();
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             const int nlo = 16 * f + 4 * lg;
@@ -2547,25 +2558,16 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
                     hi += *reinterpret_cast<const f32x4 *>(l0 + sb + nlo + NH) * first;
                 }
             }
-            if (a.theta != nullptr && a.angle0 != nullptr) {
-                const f32x4 ph = *reinterpret_cast<const f32x4 *>(a.angle0 + bh * NH + nlo);
-                f32x4 cs, sn;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float s1, c1;
-                    sincosf(ph[r], &s1, &c1);
-                    sn[r] = s1;
-                    cs[r] = c1;
-                }
+            if (turned) {
+                const f32x4 cs = *reinterpret_cast<const f32x4 *>(csn + nlo);
+                const f32x4 sn = *reinterpret_cast<const f32x4 *>(csn + NH + nlo);
                 const f32x4 z = {0.f, 0.f, 0.f, 0.f};
                 chain_step(lo, hi, 1.0f, z, z, cs, sn);
             }
             slo[f] = lo;
             shi[f] = hi;
         }
-        if (tid < NH)
-            sm.phc[tid] = (a.theta != nullptr && a.angle0 != nullptr) ? a.angle0[bh * NH + tid] : 0.0f;
-        __syncthreads();
+        __syncthreads();   // csn is read
     } else {
         if (wave == 0) {
             // the look-back, all at once: lane l reads the flag of segment
@@ -2624,62 +2626,74 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
                 phc = __hip_atomic_load(&ws.incphi[(seq0 + kinc) * NH + tid], __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT);
             // fold forward through the aggregates of segments kinc + 1 .. seg
-            // - 1, two at a time: their scalars through LDS (the band region,
-            // dead by now), every load of a pair of steps issued before its use
-            float *fsc = reinterpret_cast<float *>(sm.band);   // [2][e | phi, cos, sin x NH]
-            constexpr int FS = 1 + 3 * NH;
-            for (int m0 = kinc + 1; m0 < seg; m0 += 2) {
-                const int nm = min(2, seg - m0);
-                __syncthreads();   // the previous pair's scalars are read
-                for (int i = tid; i < nm * FS; i += kThreads) {
-                    const int st = i / FS, w = i % FS;
-                    const size_t rec = seq0 + m0 + st;
-                    float v;
-                    if (w == 0)
-                        v = __hip_atomic_load(&ws.eda[rec], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    else if (w <= NH)
-                        v = __hip_atomic_load(&ws.phi[rec * NH + (w - 1)], __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-                    else if (w <= 2 * NH)
-                        v = __hip_atomic_load(&ws.cph[rec * NH + (w - 1 - NH)], __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-                    else
-                        v = __hip_atomic_load(&ws.sph[rec * NH + (w - 1 - 2 * NH)], __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-                    fsc[i] = v;
+            // - 1.  Every lane loads what its four pairs need of a record
+            // straight into registers, kAhead records ahead, so the walk is
+            // loads in flight and FMAs, with no barrier and no LDS.  Two records at a time
+            // with their scalars through LDS (two barriers and two round trips
+            // to memory a step) took 57.6 us for 8 sequences of 4096 tokens at
+            // d_state 128 and this form 40.4; 16 of 2048 at 64 27.1 and 22.6; 24
+            // of 1024 31.8 and 26.1; 96 of 2048, three rounds of workgroups whose
+            // walks are short, 80.0 and 77.2.
+            // Three records ahead at d_state 128 spill (256 VGPRs).
+            constexpr int kAhead = N == 64 ? 3 : 2;
+            struct Rec {
+                bf16x8 u[NF];
+                f32x4 cs[NF], sn[NF];
+                float e, ph;
+            } q[kAhead];
+            const rsrc_t rph = make_rsrc(ws.phi, static_cast<uint32_t>(ws.u_bytes / 64));
+            const rsrc_t rcs = make_rsrc(ws.cph, static_cast<uint32_t>(ws.u_bytes / 64));
+            const rsrc_t rsn = make_rsrc(ws.sph, static_cast<uint32_t>(ws.u_bytes / 64));
+            const rsrc_t red = make_rsrc(ws.eda, static_cast<uint32_t>(ws.u_bytes / (32 * N)));
+            auto fetch = [&](int m, Rec &d) {
+                const size_t rec = seq0 + m;
+                const uint32_t po = static_cast<uint32_t>(rec) * (NH * 4);
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const uint32_t uo =
+                        static_cast<uint32_t>(((rec * 4 + wave) * NTN * 256 + rec_off<NTN>(f, lane)) * 2);
+                    d.u[f] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ru, uo, 0, kCoh));
+                    d.cs[f] = cld16f(rcs, po + (16 * f + 4 * lg) * 4);
+                    d.sn[f] = cld16f(rsn, po + (16 * f + 4 * lg) * 4);
                 }
-                bf16x8 uq[2][NF];
+                d.e = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(red, static_cast<uint32_t>(rec) * 4, 0, kCoh));
+                d.ph = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rph, po + (tid & (NH - 1)) * 4, 0, kCoh));
+            };
+            auto step = [&](const Rec &d) {
 #pragma unroll
-                for (int st = 0; st < 2; ++st)
-                    if (st < nm) {
-                        const size_t rec = seq0 + m0 + st;
+                for (int f = 0; f < NF; ++f) {
+                    f32x4 ul, uh;
 #pragma unroll
-                        for (int f = 0; f < NF; ++f) {
-                            const uint32_t uo =
-                                static_cast<uint32_t>(((rec * 4 + wave) * NTN * 256 + rec_off<NTN>(f, lane)) * 2);
-                            uq[st][f] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ru, uo, 0, kCoh));
-                        }
+                    for (int r = 0; r < 4; ++r) {
+                        ul[r] = static_cast<float>(d.u[f][r]);
+                        uh[r] = static_cast<float>(d.u[f][4 + r]);
                     }
-                __syncthreads();   // the pair's scalars are in LDS
+                    chain_step(slo[f], shi[f], d.e, ul, uh, d.cs[f], d.sn[f]);
+                }
+                phc = wrap_angle(phc + d.ph);
+            };
+            int m = kinc + 1;
 #pragma unroll
-                for (int st = 0; st < 2; ++st)
-                    if (st < nm) {
-                        const float *sc = fsc + st * FS;
+            for (int i = 0; i < kAhead; ++i)
+                if (m + i < seg) fetch(m + i, q[i]);
+            // no condition between a load and its use here, so that the waits
+            // leave the later records' loads in flight
+            for (; m + 2 * kAhead <= seg; m += kAhead) {
 #pragma unroll
-                        for (int f = 0; f < NF; ++f) {
-                            f32x4 ul, uh, cs, sn;
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                ul[r] = static_cast<float>(uq[st][f][r]);
-                                uh[r] = static_cast<float>(uq[st][f][4 + r]);
-                                cs[r] = sc[1 + NH + 16 * f + 4 * lg + r];
-                                sn[r] = sc[1 + 2 * NH + 16 * f + 4 * lg + r];
-                            }
-                            chain_step(slo[f], shi[f], sc[0], ul, uh, cs, sn);
-                        }
-                        if (tid < NH) phc = wrap_angle(phc + sc[1 + tid]);
-                    }
+                for (int i = 0; i < kAhead; ++i) {
+                    step(q[i]);
+                    fetch(m + i + kAhead, q[i]);
+                }
             }
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+                if (m + i < seg) {
+                    step(q[i]);
+                    if (m + i + kAhead < seg) fetch(m + i + kAhead, q[i]);
+                }
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+                if (m + i + kAhead < seg) step(q[i]);
             if (tid < NH) sm.phc[tid] = phc;
         }
         __syncthreads();
@@ -2691,12 +2705,16 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
     float phe = 0.0f;   // the angle after the segment (pair tid)
     if (tid < NH) {
         phe = wrap_angle(sm.phc[tid] + sm.ang[tid]);
-        __hip_atomic_store(&ws.incphi[bhs * NH + tid], phe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!last_seg)
+            __hip_atomic_store(&ws.incphi[bhs * NH + tid], phe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const bool last_seg = seg == nseg - 1;
     if (last_seg) {
-        __syncthreads();   // every pair's angle entering the segment is read
-        if (tid < NH) sm.phc[tid] = phe;
+        if (tid < NH) {
+            float s1 = 0.0f, c1 = 1.0f;
+            if (a.theta != nullptr) sincosf(phe, &s1, &c1);
+            csn[tid] = c1;
+            csn[NH + tid] = s1;
+        }
         __syncthreads();
     }
 #pragma unroll
@@ -2710,24 +2728,14 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
             sn[r] = sm.sph[16 * f + 4 * lg + r];
         }
         chain_step(olo, ohi, eacc, ul, uh, cs, sn);
-        cst16f(rinc, inc_off(bhs, f, 0), olo);
-        cst16f(rinc, inc_off(bhs, f, 1), ohi);
-        if (last_seg) {
+        if (!last_seg) {
+            cst16f(rinc, inc_off(bhs, f, 0), olo);
+            cst16f(rinc, inc_off(bhs, f, 1), ohi);
+        } else {
             const size_t sb = (bh * P + p) * N;
             const int nlo = 16 * f + 4 * lg;
-            f32x4 ce, se;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (a.theta != nullptr) {
-                    float s1, c1;
-                    sincosf(sm.phc[nlo + r], &s1, &c1);
-                    se[r] = s1;
-                    ce[r] = c1;
-                } else {
-                    se[r] = 0.0f;
-                    ce[r] = 1.0f;
-                }
-            }
+            const f32x4 ce = *reinterpret_cast<const f32x4 *>(csn + nlo);
+            const f32x4 se = *reinterpret_cast<const f32x4 *>(csn + NH + nlo);
             if (a.h_out != nullptr) {
                 f32x4 hl, hh2;   // R(-phi_end) S
 #pragma unroll
@@ -2757,12 +2765,14 @@ __device__ __forceinline__ void fused_tail(const ScanLaunch &a, const FusedWs &w
         }
     }
     if (last_seg && a.angle_out != nullptr && tid < NH) a.angle_out[bh * NH + tid] = phe;
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __syncthreads();
-    if (tid == 0)
-        __hip_atomic_store(&ws.flag[bhs], (epoch << 2) | kFlagInc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!last_seg) {
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __syncthreads();
+        if (tid == 0)
+            __hip_atomic_store(&ws.flag[bhs], (epoch << 2) | kFlagInc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 
     // ---- y = y_local + decay(t) C~_t . S_j, stored (or gated) once
     {
@@ -3326,14 +3336,23 @@ hipError_t launch_three(const ScanLaunch &a, char *base, hipStream_t s) {
 }
 
 // Segments of the fused launch: two sub-chunks each (the C~ of both stay in
-// LDS for the entering state's part of y).
+// LDS for the entering state's part of y), or one while every sub-chunk's
+// workgroup is resident at once (two a CU) and the walk over the segments
+// before stays short: the local pass is half as long, each further segment
+// costs the walk some 0.6 us.  Measured, two against one (us, d_state 128 unless
+// said): 12 sequences of 128 tokens 17.7 / 16.3, 24 of 509 22.4 / 20.0, 48 of 256
+// 21.5 / 18.0, 12 of 640 23.6 / 21.0, 12 of 640 at d_state 64 17.0 / 15.5, 48 of 384
+// 22.6 / 20.0, 128 of 256 at 64 18.2 / 16.8, 48 of 512 24.1 / 23.5.  Past ten
+// sub-chunks the walk eats it: 12 of 768 23.4 / 22.2, 12 of 1024 25.0 / 25.1, 12 of
+// 1280 25.8 / 27.5, 24 of 1024 25.6 / 28.6.
 struct FusedPlan {
     int nsub, kseg, nseg;
 };
 FusedPlan fused_plan(const ScanLaunch &a) {
     FusedPlan p;
     p.nsub = static_cast<int>((a.seq + 63) / 64);
-    p.kseg = p.nsub > 1 ? 2 : 1;
+    const bool one = p.nsub <= 10 && a.batch * a.heads * static_cast<size_t>(p.nsub) <= 2 * device_cus();
+    p.kseg = one ? 1 : 2;
     p.nseg = (p.nsub + p.kseg - 1) / p.kseg;
     return p;
 }
@@ -3342,7 +3361,7 @@ FusedPlan fused_plan(const ScanLaunch &a) {
 // and is taken while its grid fits three rounds of two workgroups per CU.
 // Each round ends in a look-back, while the three launches' cost grows with
 // the sequences alone; measured on MI355X (us per call, fused vs three
-// launches): config 1, 96 sequences of 2048 tokens (3 rounds), 81.5 vs 83.3
+// launches): config 1, 96 sequences of 2048 tokens (3 rounds), 77.2 vs 83.3
 // summed over the kernels; the config-4 prefill's 192 sequences (6 rounds),
 // 17.22 vs 16.94 ms per 24-layer prefill.
 bool fused_covered(const ScanLaunch &a) {
