@@ -7,6 +7,8 @@ from __future__ import annotations
 import ctypes as C
 import os
 
+import torch
+
 from .error import (ArgumentError, ConfigError, DeviceError, IoError, JsonError, Mamba3Error,
                     RankError, ShapeError, StateDictError, UnsupportedError)
 
@@ -187,6 +189,16 @@ _ERRORS = {
     M3_ERR_IO: IoError,
     M3_ERR_JSON: JsonError,
 }
+
+
+def stream_of(t):
+    """The current stream of a device tensor's GPU, as the C calls take it.
+    torch.cuda.current_stream builds a Stream object for it, 2.7 us a call of
+    which a four-layer prefill makes 23; the raw handle is 0.3 us."""
+    i = t.get_device()
+    if i < 0:   # not a device tensor: current_stream's error
+        return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(i))
 
 
 def check(status: int):

@@ -15,11 +15,8 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._lib import stream_of as _stream
 from .error import ArgumentError, ShapeError, UnsupportedError
-
-
-def _stream(t: torch.Tensor):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
 def _bf16_dev(t: torch.Tensor, what: str) -> torch.Tensor:
