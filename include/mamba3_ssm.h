@@ -135,11 +135,11 @@ typedef struct m3_scan_inputs {
     const void *theta;        /* [B, T, H, N/2] or NULL (real dynamics) */
     const float *d_skip;      /* [H] or NULL */
     const m3_ssm_state *state;/* carried-in state or NULL */
-    size_t chunk_size;        /* > 0; the three-launch chunk-parallel form passes
-                               * the state between segments of at least this many
-                               * tokens (tiles inside a segment are the kernel's
-                               * own); the fused single launch always uses
-                               * segments of 128 tokens */
+    size_t chunk_size;        /* > 0; past 64, the three-launch chunk-parallel form
+                               * passes the state between segments of at least this
+                               * many tokens (tiles inside a segment are the
+                               * kernel's own); the fused single launch uses
+                               * segments of 128 tokens, 64 in short windows */
     int32_t want_state;       /* ScanInputs::want_state */
     /* Device scratch for the chunk-parallel scan (no reference counterpart:
      * the reference allocates its intermediates per call): 256-byte aligned,

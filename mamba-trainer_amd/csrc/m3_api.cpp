@@ -479,7 +479,11 @@ static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
                     "d_state 64 or 128, rank 1, 2 or 4, 16-byte aligned buffers and rows of whole "
                     "16-byte pieces", a.theta_stride);
     hipError_t e;
-    const size_t need = m3::scan_chunked_workspace(a);
+    size_t need = m3::scan_chunked_workspace(a);
+    if (need > 0 && in->workspace != nullptr && in->workspace_bytes < need) {
+        a.path |= 2;   // the caller's workspace may hold the records of longer segments
+        need = m3::scan_chunked_workspace(a);
+    }
     const bool ws_aligned = (reinterpret_cast<uintptr_t>(in->workspace) & 255u) == 0;
     const bool chunked =
         need > 0 && in->workspace != nullptr && in->workspace_bytes >= need && ws_aligned;
@@ -648,12 +652,14 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
     local.workspace_bytes = 0;
     int path = g_scan_path.load(std::memory_order_relaxed);
     size_t need = workspace_bytes_for(&local, path, false);
-    if (need > kNoAllocScratchBytes && path == 0) {
-        // the fused launch's records do not fit: the three launches' may
-        const size_t three = workspace_bytes_for(&local, 1, false);
-        if (three <= kNoAllocScratchBytes) {
-            path = 1;
-            need = three;
+    // where the records do not fit: those of longer segments, or the three
+    // launches' in place of the fused launch's, or both
+    for (const int p : {path | 2, 1, 3}) {
+        if (need <= kNoAllocScratchBytes) break;
+        const size_t other = workspace_bytes_for(&local, p, false);
+        if (other <= kNoAllocScratchBytes) {
+            path = p;
+            need = other;
         }
     }
     if (need > kNoAllocScratchBytes)

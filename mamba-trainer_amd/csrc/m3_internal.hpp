@@ -110,11 +110,12 @@ struct ScanLaunch {
     const void *gate_z;
     size_t gate_stride;
     float *h_out, *last_u_out, *angle_out;  // null when not wanted
-    // the caller's chunk_size (tokens; 0 = 64): the chunk-parallel path passes
+    // the caller's chunk_size (tokens; 0 = 64): past 64, the three launches pass
     // the state between segments of at least this many tokens
     size_t chunk_size;
     // chunk-parallel form: 0 the fused single launch where it covers the
-    // shape (bf16, rank 1), 1 the three launches
+    // shape (bf16, rank 1), 1 the three launches; plus 2: no segments shorter
+    // than 128 tokens (fused) or 64 (three launches), whose records are fewer
     int path;
     // the fused launch's look-back: lb_mode 1 gives up at once (tests);
     // lb_spin polls of one flag before giving up (0: the default)

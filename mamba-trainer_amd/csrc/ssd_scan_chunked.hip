@@ -37,6 +37,7 @@
 // over every segment of every sequence; the sequential pass is a few FMAs per
 // element and streams U from HBM.  Segments of several sub-chunks keep the U
 // and S records (and the state pass) small while still filling the chip.
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <type_traits>
@@ -3261,7 +3262,23 @@ SegPlan seg_plan(const ScanLaunch &a) {
     const size_t qt = static_cast<size_t>(rows_for(a)) / a.rank;
     const size_t nsub = (a.seq + qt - 1) / qt;
     const size_t q = a.chunk_size ? a.chunk_size : 64;
-    const size_t kmin = (q + qt - 1) / qt;
+    size_t kmin = (q + qt - 1) / qt;
+    // A segment is a serial walk over its sub-chunks in both heavy kernels (7 to
+    // 11 us a sub-chunk of f32), each further segment a step of the state pass
+    // (0.4 us): the least sum is near k = sqrt(nsub / 18), taken as the power of
+    // two 1, 2, 4 .. up to 32, 128, 512 .. sub-chunks, where a chunk_size of at
+    // most 64 tokens does not ask for longer ones.  Segments of 64 tokens against
+    // these, us a call: f32, 8 sequences of 512 tokens, d_state 64 25.8 / 22.1;
+    // 12 of 128, 128 33.1 / 22.6; 24 of 1024, 128 52.0 / 48.8; 4 of 4096, 64 45.6 /
+    // 45.5; rank 2, 8 of 300, 64 40.6 / 24.7; rank 4, 8 of 1000, 128 124.7 / 74.7,
+    // 8 of 2000, 64 94.2 / 77.5; bf16, rank 2, 12 of 300, 128 32.2 / 25.0; rank 4,
+    // 12 of 300, 128 32.8 / 23.8; one sub-chunk a segment all the way, f32, 4 of
+    // 4096, 64 61.5.
+    if (q <= 64 && (a.path & 2) == 0) {
+        size_t k2 = 1;
+        while (k2 * k2 * 32 < nsub) k2 *= 2;
+        kmin = std::min(kmin, k2);
+    }
     // rounds of resident chunk_scan workgroups: one at rank 1, six for MIMO
     // (measured on MI355X, rotated inputs, us per call: config 1 with the
     // direct-to-LDS staging at 1 / 2 rounds 96.4-97.8 / 100.2-102.8, before it
@@ -3351,7 +3368,8 @@ struct FusedPlan {
 FusedPlan fused_plan(const ScanLaunch &a) {
     FusedPlan p;
     p.nsub = static_cast<int>((a.seq + 63) / 64);
-    const bool one = p.nsub <= 10 && a.batch * a.heads * static_cast<size_t>(p.nsub) <= 2 * device_cus();
+    const bool one = p.nsub <= 10 && (a.path & 2) == 0 &&
+                     a.batch * a.heads * static_cast<size_t>(p.nsub) <= 2 * device_cus();
     p.kseg = one ? 1 : 2;
     p.nseg = (p.nsub + p.kseg - 1) / p.kseg;
     return p;
@@ -3365,7 +3383,7 @@ FusedPlan fused_plan(const ScanLaunch &a) {
 // summed over the kernels; the config-4 prefill's 192 sequences (6 rounds),
 // 17.22 vs 16.94 ms per 24-layer prefill.
 bool fused_covered(const ScanLaunch &a) {
-    if (!(a.bf16 && a.rank == 1 && (a.d_state == 64 || a.d_state == 128) && a.path == 0)) return false;
+    if (!(a.bf16 && a.rank == 1 && (a.d_state == 64 || a.d_state == 128) && (a.path & 1) == 0)) return false;
     const size_t segs = a.batch * a.heads * static_cast<size_t>(fused_plan(a).nseg);
     return segs <= 3 * 2 * device_cus();
 }
