@@ -268,10 +268,10 @@ typedef struct m3_scan_grads {
  * chunk states are recomputed; the forward outputs are not needed.  The
  * chunk kernels take head_dim 64, d_state 64/128, rank 1/2/4 with aligned
  * buffers; every sum has a fixed order, so repeated calls agree bit for bit.
- * Small
- * heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens on) run
- * them on zero-padded copies in the workspace.  Other shapes (and alignments) take the reverse mode of the recurrence token by
- * token, one workgroup per sequence with states recomputed from checkpoints
+ * Small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens
+ * on) run them on zero-padded copies in the workspace.  Other shapes (and
+ * alignments) take the reverse mode of the recurrence token by token, one
+ * workgroup per sequence with states recomputed from checkpoints
  * every 32 tokens (deterministic, and slow: a fallback), up to per-token
  * vectors of 64 KB (2 head_dim rank + 4 d_state rank + 3 d_state/2 floats;
  * beyond that M3_ERR_UNSUPPORTED, before any device work). */
