@@ -10,7 +10,7 @@
 // bounds them is that serial chain, not work: at batch 4 x 512, 4 heads of 16,
 // d_state 16, f32, 16 of the 256 CUs are busy for 233 us (forward) and
 // 5613 us (backward).  Padded, the 16 sequences are cut in chunks that run side by
-// side: 41 and 73 us, 38 and 50 of them launches and their gaps.
+// side: 33 and 59 us, for the most part launches and their gaps.
 #include <algorithm>
 
 #include "m3_device.hpp"
@@ -269,12 +269,13 @@ hipError_t launch_pads(const Pads &p, bool out, hipStream_t s) {
 }  // namespace
 
 // Measured on MI355X (f32, head_dim and d_state 16, us per call, one workgroup
-// per sequence against padded): 8 sequences of 64 / 96 tokens 38 / 51 against
-// 38 / 53, of 128 (bf16) 65 against 43; 4 of 33 at rank 4 54 against 56; 16 of
-// 512 233 against 43; 64 of 400 (heads of 32) 153 against 50; 512 of 512 340
-// against 220; 1024 of 512 344 against 403; 4096 of 64 160 against 268: short
-// windows end before the extra launches do, and a thousand sequences fill the
-// chip as they are.
+// per sequence against padded): 8 sequences of 128 tokens 65 against 24; 16 of
+// 512 233 against 33; 64 of 400 (heads of 32) 153 against 50; 512 of 512 340
+// against 211; 1024 of 512 344 against 403, for a thousand sequences fill the
+// chip as they are.  The line at 128 rows is where the two met (8 of 64 / 96
+// 38 / 51 against 38 / 53) before the padded windows were cut into as many
+// segments as they are now; 4 of 33 at rank 4 were 54 against 56, 4096 of 64 160
+// against 268.
 bool scan_pad_wanted(const ScanLaunch &a) {
     return a.seq * a.rank >= 128 && a.batch * a.heads <= 512 && pad_shape(a, false);
 }
@@ -313,9 +314,10 @@ hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t str
 }
 
 // The token walk against padded (f32, head_dim and d_state 16, us per call): 2
-// sequences of 1 / 4 / 8 / 64 tokens 31 / 52 / 98 / 701 against 48 / 49 / 50 /
-// 47; 16 of 512 5613 against 73; 1024 of 512 8507 against 1483; 8192 of 32
-// 4471 against 990.  Heads over 32, states over 64 and other ranks keep the
+// sequences of 8 / 64 tokens 98 / 701 against 32 / 33; 16 of 512 5613 against 59;
+// 1024 of 512 8507 against 1160; 8192 of 32 4471 against 815; 2 of 1 token 20 by
+// the walk.  The line at 8 tokens was drawn with the chunk kernels at 50 us, which
+// met the walk at 4 (52).  Heads over 32, states over 64 and other ranks keep the
 // walk's two launches.
 bool scan_backward_pad_wanted(const ScanLaunch &a) { return a.seq >= 8 && pad_shape(a, true); }
 
