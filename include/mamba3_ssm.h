@@ -232,7 +232,9 @@ size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
  * with an event.  Calls captured into a HIP graph, and the graph's replays,
  * are not tracked: overlapping them races and gives wrong results.  The
  * scratch needs no clearing: the chunk-parallel kernels write every byte they
- * later read within one call.  It calls no hipMalloc, hipFree or allocating
+ * later read within one call (a call captured into a graph adds a kernel that
+ * clears the fused launch's flags, so that a replay does not take the records
+ * of the one before for its own).  It calls no hipMalloc, hipFree or allocating
  * library routine (the guard's event is created once per device). */
 m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, void *stream);
 

@@ -497,18 +497,17 @@ static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
         a.gate_stride = gate_stride;
     }
     const size_t pad_need = need > 0 || !ws_aligned ? 0 : m3::scan_pad_workspace(a);
+    int launches = 0;
     if (pad_need > 0 && in->workspace != nullptr && in->workspace_bytes >= pad_need) {
-        e = m3::launch_scan_pad(a, in->workspace, s);
-        if (e == hipSuccess) g_launches.fetch_add(m3::scan_pad_launches(a), std::memory_order_relaxed);
+        e = m3::launch_scan_pad(a, in->workspace, s, launches);
     } else if (chunked) {
-        e = m3::launch_scan_chunked(a, in->workspace, s);
-        if (e == hipSuccess)
-            g_launches.fetch_add(m3::scan_chunked_launches(a), std::memory_order_relaxed);
+        e = m3::launch_scan_chunked(a, in->workspace, s, launches);
     } else {
         e = m3::launch_scan(a, s);
-        if (e == hipSuccess) g_launches.fetch_add(1, std::memory_order_relaxed);
+        launches = 1;
     }
     if (e != hipSuccess) return hip_fail(e, "scan launch");
+    g_launches.fetch_add(launches, std::memory_order_relaxed);
     if (gate_z != nullptr && !fuse_gate) {
         e = m3::launch_mixer_gate(B * in->seq, H * P * in->rank, out->y, gate_z, gate_stride,
                                   nullptr, 0.0f, out->y, s);

@@ -129,13 +129,11 @@ hipError_t launch_scan_fast(const ScanLaunch &a, hipStream_t stream);
 // The chunk-parallel form of the same shapes (chunk states, an elementwise
 // state pass, chunk outputs: three launches over a 256-byte aligned caller
 // workspace): the workspace bytes it needs (0 when the shape is not covered),
-// and the launch.
+// and the launch.  `launches` grows by the kernels launched: 1 for the fused
+// single launch (bf16, rank 1, up to three rounds of its workgroups; 2 under
+// stream capture), 3 otherwise.
 size_t scan_chunked_workspace(const ScanLaunch &a);
-hipError_t launch_scan_chunked(const ScanLaunch &a, void *workspace, hipStream_t stream);
-// Kernel launches the chunk-parallel form makes for these inputs: 1 for the
-// fused single launch (bf16, rank 1, up to three rounds of its workgroups), 3
-// otherwise.
-int scan_chunked_launches(const ScanLaunch &a);
+hipError_t launch_scan_chunked(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches);
 // Backward of the scan (mamba3_scan mode, the chunk-parallel shapes): the
 // gradients of the loss given dL/dy (and optionally dL/dh, dL/dangle of the
 // outgoing state).  Outputs in the storage type where the input has it.
@@ -166,12 +164,11 @@ hipError_t launch_scan_backward_generic(const ScanLaunch &a, const ScanGrads &g,
 
 // The heads of small models (head_dim up to 32, d_state up to 64, rank 1, 2 or
 // 4) on zero-padded copies through the kernels above (scan_pad.hip): whether
-// that is the faster form, the workspace it takes (0 where it is not), its
-// kernel launches and the launch.
+// that is the faster form, the workspace it takes (0 where it is not) and the
+// launch, which adds its kernels to `launches`.
 bool scan_pad_wanted(const ScanLaunch &a);
 size_t scan_pad_workspace(const ScanLaunch &a);
-int scan_pad_launches(const ScanLaunch &a);
-hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream);
+hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches);
 bool scan_backward_pad_wanted(const ScanLaunch &a);
 size_t scan_backward_pad_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,

@@ -285,12 +285,7 @@ size_t scan_pad_workspace(const ScanLaunch &a) {
     return pad_layout(a, false).total + scan_chunked_workspace(padded_shape(a, false));
 }
 
-int scan_pad_launches(const ScanLaunch &a) {
-    const ScanLaunch p = padded_shape(a, false);
-    return 2 + (scan_chunked_workspace(p) > 0 ? scan_chunked_launches(p) : 1);
-}
-
-hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream) {
+hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches) {
     const PadLayout l = pad_layout(a, false);
     const PadShapes s(a, false);
     char *base = static_cast<char *>(workspace);
@@ -307,9 +302,14 @@ hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t str
     p.angle_out = static_cast<float *>(get(s.angle, a.angle_out, l.angout));
     hipError_t e = launch_pads(in, false, stream);
     if (e != hipSuccess) return e;
-    e = scan_chunked_workspace(p) > 0 ? launch_scan_chunked(p, base + l.total, stream)
-                                      : launch_scan(p, stream);
+    if (scan_chunked_workspace(p) > 0) {
+        e = launch_scan_chunked(p, base + l.total, stream, launches);
+    } else {
+        e = launch_scan(p, stream);
+        ++launches;
+    }
     if (e != hipSuccess) return e;
+    launches += 2;
     return launch_pads(out, true, stream);
 }
 

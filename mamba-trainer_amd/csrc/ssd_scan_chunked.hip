@@ -3389,7 +3389,8 @@ bool fused_covered(const ScanLaunch &a) {
 }
 
 // Each call gets a fresh epoch, so flags left in a reused workspace by an
-// earlier call never read as published (62 bits, seeded from the clock).
+// earlier call never read as published (62 bits, seeded from the clock); a
+// captured launch, whose replays share one, clears its flags (launch_fused).
 std::atomic<uint64_t> g_epoch{0};
 uint64_t next_epoch() {
     uint64_t e = g_epoch.fetch_add(1, std::memory_order_relaxed);
@@ -3404,13 +3405,38 @@ uint64_t next_epoch() {
     return e & ((uint64_t(1) << 62) - 1);
 }
 
+// The flags of a captured launch.  A graph's replays all carry the epoch they
+// were captured with, so the flags the replay before left would read as
+// published, and its records as this replay's: a kernel of the graph's own
+// clears them first.  An eager call's epoch is its own and needs none of it.
+__global__ void __launch_bounds__(kThreads) clear_flags_kernel(unsigned long long *flag, uint32_t n) {
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < n) __hip_atomic_store(&flag[i], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // the default stream beside another's capture: the launch reports it
+    return false;
+}
+
 template <int N>
-hipError_t launch_fused(const ScanLaunch &a, char *base, hipStream_t s) {
+hipError_t launch_fused(const ScanLaunch &a, char *base, hipStream_t s, int &launches) {
     const FusedPlan fp = fused_plan(a);
     const size_t bh = a.batch * a.heads;
     const size_t segs = bh * fp.nseg;
     const FusedWs ws = fused_ws(base, fused_layout(segs, N), segs, N);
     const uint64_t epoch = next_epoch();
+    if (capturing(s)) {
+        const uint32_t n = static_cast<uint32_t>(segs);
+        hipLaunchKernelGGL(clear_flags_kernel, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, s,
+                           ws.flag, n);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        ++launches;
+    }
+    ++launches;
     // polls of one flag before a look-back gives up (each poll sleeps ~128
     // cycles and waits a memory round trip: about a second in all)
     const int spin = a.lb_spin > 0 ? a.lb_spin : (1 << 20);
@@ -3450,15 +3476,14 @@ size_t scan_chunked_workspace(const ScanLaunch &a) {
     return chunked_layout(seqs * seg_plan(a).nseg, a.d_state, a.bf16 != 0).total;
 }
 
-int scan_chunked_launches(const ScanLaunch &a) { return fused_covered(a) ? 1 : 3; }
-
-hipError_t launch_scan_chunked(const ScanLaunch &a, void *workspace, hipStream_t stream) {
+hipError_t launch_scan_chunked(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches) {
     if (!scan_fast_supported(a) || a.seq == 0) return hipErrorNotSupported;
     char *ws = static_cast<char *>(workspace);
     if (fused_covered(a)) {
-        if (a.d_state == 128) return launch_fused<128>(a, ws, stream);
-        return launch_fused<64>(a, ws, stream);
+        if (a.d_state == 128) return launch_fused<128>(a, ws, stream, launches);
+        return launch_fused<64>(a, ws, stream, launches);
     }
+    launches += 3;
     if (a.bf16) return launch_t<bf16_t, 64>(a, ws, stream);
     return launch_t<float, 32>(a, ws, stream);
 }
