@@ -587,8 +587,9 @@ namespace {
 // process ends.  In host code `scratch` names a host-side stand-in, never the
 // device memory: kernels get the address hipGetSymbolAddress returns for the
 // current device, looked up once per device and kept in g_scratch.
-constexpr size_t kNoAllocScratchBytes = size_t(M3_NO_ALLOC_SCRATCH_MIB) << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[m3::kNoAllocScratchBytes];
+using m3::kNoAllocScratchBytes;
+static_assert(kNoAllocScratchBytes == size_t(M3_NO_ALLOC_SCRATCH_MIB) << 20);
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -651,14 +652,12 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
     local.workspace_bytes = 0;
     int path = g_scan_path.load(std::memory_order_relaxed);
     size_t need = workspace_bytes_for(&local, path, false);
-    // where the records do not fit: those of longer segments, or the three
-    // launches' in place of the fused launch's, or both
-    for (const int p : {path | 2, 1, 3}) {
-        if (need <= kNoAllocScratchBytes) break;
-        const size_t other = workspace_bytes_for(&local, p, false);
-        if (other <= kNoAllocScratchBytes) {
-            path = p;
-            need = other;
+    if (need > kNoAllocScratchBytes && path == 0) {
+        // the fused launch's records do not fit: the three launches' may
+        const size_t three = workspace_bytes_for(&local, 1, false);
+        if (three <= kNoAllocScratchBytes) {
+            path = 1;
+            need = three;
         }
     }
     if (need > kNoAllocScratchBytes)

@@ -115,7 +115,8 @@ struct ScanLaunch {
     size_t chunk_size;
     // chunk-parallel form: 0 the fused single launch where it covers the
     // shape (bf16, rank 1), 1 the three launches; plus 2: no segments shorter
-    // than 128 tokens (fused) or 64 (three launches), whose records are fewer
+    // than 128 tokens (fused) or 64 (three launches), whose records are fewer,
+    // for a workspace that holds no more
     int path;
     // the fused launch's look-back: lb_mode 1 gives up at once (tests);
     // lb_spin polls of one flag before giving up (0: the default)
@@ -173,6 +174,9 @@ bool scan_backward_pad_wanted(const ScanLaunch &a);
 size_t scan_backward_pad_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,
                                     hipStream_t stream);
+
+// The static scratch of m3_scan_no_alloc (M3_NO_ALLOC_SCRATCH_MIB).
+constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
 
 // Largest head_dim / d_state the scan kernels are instantiated for.
 constexpr size_t kScanMaxHeadDim = 128;

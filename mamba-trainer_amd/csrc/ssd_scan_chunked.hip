@@ -3263,22 +3263,6 @@ SegPlan seg_plan(const ScanLaunch &a) {
     const size_t nsub = (a.seq + qt - 1) / qt;
     const size_t q = a.chunk_size ? a.chunk_size : 64;
     size_t kmin = (q + qt - 1) / qt;
-    // A segment is a serial walk over its sub-chunks in both heavy kernels (7 to
-    // 11 us a sub-chunk of f32), each further segment a step of the state pass
-    // (0.4 us): the least sum is near k = sqrt(nsub / 18), taken as the power of
-    // two 1, 2, 4 .. up to 32, 128, 512 .. sub-chunks, where a chunk_size of at
-    // most 64 tokens does not ask for longer ones.  Segments of 64 tokens against
-    // these, us a call: f32, 8 sequences of 512 tokens, d_state 64 25.8 / 22.1;
-    // 12 of 128, 128 33.1 / 22.6; 24 of 1024, 128 52.0 / 48.8; 4 of 4096, 64 45.6 /
-    // 45.5; rank 2, 8 of 300, 64 40.6 / 24.7; rank 4, 8 of 1000, 128 124.7 / 74.7,
-    // 8 of 2000, 64 94.2 / 77.5; bf16, rank 2, 12 of 300, 128 32.2 / 25.0; rank 4,
-    // 12 of 300, 128 32.8 / 23.8; one sub-chunk a segment all the way, f32, 4 of
-    // 4096, 64 61.5.
-    if (q <= 64 && (a.path & 2) == 0) {
-        size_t k2 = 1;
-        while (k2 * k2 * 32 < nsub) k2 *= 2;
-        kmin = std::min(kmin, k2);
-    }
     // rounds of resident chunk_scan workgroups: one at rank 1, six for MIMO
     // (measured on MI355X, rotated inputs, us per call: config 1 with the
     // direct-to-LDS staging at 1 / 2 rounds 96.4-97.8 / 100.2-102.8, before it
@@ -3298,6 +3282,31 @@ SegPlan seg_plan(const ScanLaunch &a) {
     const size_t bh = a.batch * a.heads;
     const size_t fill = bh < rounds * slots ? rounds * slots / bh : 1;
     size_t k = (nsub + fill - 1) / fill;
+    // A segment is a serial walk over its sub-chunks in both heavy kernels (7 to
+    // 11 us a sub-chunk of f32), each further segment a step of the state pass
+    // (0.4 us): the least sum is near k = sqrt(nsub / 18), taken as the power of
+    // two 1, 2, 4 .. up to 32, 128, 512 .. sub-chunks, where a chunk_size of at
+    // most 64 tokens does not ask for longer ones, and the next powers up to 64
+    // tokens where its records are more than the static scratch of
+    // m3_scan_no_alloc holds: both calls then cut alike and agree bit for bit,
+    // and past those 32 MiB the grid is full and short segments lose (rank 2, 32
+    // sequences of 1000 tokens, d_state 128, 68 MB of f32 records 83.5 us against
+    // 79.9, 34 MB of bf16 ones 49.1 against 46.0; rank 4, 48 of 2000, 64, 100 MB
+    // of f32 263 against 243).  Segments of 64 tokens against these, us a call:
+    // f32, 8 sequences of 512 tokens, d_state 64 25.8 / 22.1; 12 of 128, 128
+    // 33.1 / 22.6; 4 of 4096, 64 45.6 / 45.5; rank 2, 8 of 300, 64 40.6 / 24.7;
+    // rank 4, 8 of 1000, 128 119 / 73, 8 of 2000, 64 94.2 / 77.5; bf16, rank 2,
+    // 12 of 300, 128 32.2 / 25.0; rank 4, 12 of 300, 128 32.8 / 23.8; one
+    // sub-chunk a segment all the way, f32, 4 of 4096, 64 61.5.
+    if (q <= 64 && (a.path & 2) == 0) {
+        size_t k2 = 1;
+        while (k2 * k2 * 32 < nsub) k2 *= 2;
+        for (; k2 < kmin; k2 *= 2) {
+            const size_t kk = std::min(std::max(k, k2), nsub), nseg = (nsub + kk - 1) / kk;
+            if (chunked_layout(bh * nseg, a.d_state, a.bf16 != 0).total <= kNoAllocScratchBytes) break;
+        }
+        kmin = std::min(kmin, k2);
+    }
     if (k < kmin) k = kmin;
     if (k < 1) k = 1;
     if (k > nsub) k = nsub;

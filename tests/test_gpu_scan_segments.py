@@ -9,9 +9,10 @@ import test_gpu_scan as scan
 import test_zz_no_alloc as no_alloc
 from cases import rel_l2
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
 
+@gpu
 @pytest.mark.parametrize("B,T,H,N,theta,state,skip", [
     (1, 65, 2, 128, True, True, True),      # two segments of one sub-chunk
     (1, 63, 2, 64, True, True, False),      # one ragged segment, nothing published
@@ -28,6 +29,7 @@ def test_segments_and_walks(B, T, H, N, theta, state, skip):
     scan.test_fused_launch_matches_the_three_launches_and_f64(B, T, H, N, theta, state, skip)
 
 
+@gpu
 @pytest.mark.parametrize("B,T,H,N,R,dtype", [
     (1, 1024, 2, 64, 1, "f32"), (1, 1025, 2, 64, 1, "f32"),     # 32 and 33 sub-chunks
     (1, 1024, 1, 128, 4, "f32"), (1, 1032, 1, 64, 4, "f32"),    # 128 and 129
@@ -39,18 +41,42 @@ def test_three_launch_segments_against_f64(B, T, H, N, R, dtype):
     scan.test_segments_against_f64(B, T, H, N, R, dtype, 64)
 
 
-def test_no_alloc_takes_longer_segments_where_the_short_ones_do_not_fit():
-    """24 sequences of 600 f32 tokens at rank 4 and d_state 128: 58 MB in
-    segments of 16 tokens, under the static scratch in segments of 64."""
-    inp = no_alloc._inputs(77, B=2, L=600, H=12, N=128, R=4, dtype=torch.float32)
+@gpu
+@pytest.mark.parametrize("B,T,H,N,R,dtype", [
+    (2, 600, 12, 128, 4, torch.float32),    # 58 MB of records in segments of 16 tokens
+    (2, 700, 12, 128, 1, torch.float32),    # 34 MB in segments of 32
+    (4, 1000, 8, 128, 2, torch.bfloat16),   # 33 MB in segments of 32
+    (1, 1000, 4, 64, 4, torch.float32),     # short ones fit
+])
+def test_no_alloc_cuts_as_the_workspace_scan(B, T, H, N, R, dtype):
+    """Where short segments' records exceed the static scratch both calls take
+    the next longer ones that fit: equal bit for bit, as everywhere."""
+    inp = no_alloc._inputs(77, B=B, L=T, H=H, N=N, R=R, dtype=dtype)
     ref = no_alloc._call(inp, no_alloc=False)
     got = no_alloc._call(inp, no_alloc=True)
-    assert ref[4] > 32 << 20
-    for r, g in zip(ref[:3], got[:3]):
-        # both within F32_TOL of the f64 recurrence
-        assert rel_l2(np.asarray(g.float().cpu()), np.asarray(r.float().cpu())) <= 2 * scan.F32_TOL
+    assert 0 < ref[4] <= 32 << 20
+    for r, g in zip(ref[:4], got[:4]):
+        assert torch.equal(r, g)
 
 
+def test_records_of_short_segments_stay_within_the_scratch():
+    """Sizes only: no shape whose 64-token segments fit the static scratch asks
+    for more (and so for another cut than m3_scan_no_alloc's)."""
+    import ctypes as C
+    from mamba3 import _lib
+    L = _lib.lib()
+    for dt, R, N, BH, T in [(d, r, n, bh, t) for d in (_lib.M3_F32, _lib.M3_BF16) for r in (1, 2, 4)
+                            for n in (64, 128) for bh in (1, 6, 24, 48, 64) for t in (64, 200, 600, 1000, 4096)]:
+        need = L.m3_scan_workspace_bytes(C.byref(_lib.ScanInputsC(
+            BH, T, 1, 64, N, R, dt, None, None, None, None, None, None, None, None, None, 64, 1,
+            None, 0)))
+        # a segment's U and S, its decay and its angle totals
+        record = 2 * 64 * N * (4 if dt == _lib.M3_F32 else 2) + 4 + 3 * (N // 2) * 4
+        if BH * ((T + 63) // 64) * record + 6 * 256 <= 32 << 20:
+            assert need <= 32 << 20, (dt, R, N, BH, T)
+
+
+@gpu
 @pytest.mark.parametrize("B,T,H,N,R,dtype", [(2, 600, 3, 128, 4, torch.float32),
                                              (2, 600, 3, 64, 1, torch.bfloat16)])
 def test_a_smaller_workspace_takes_longer_segments(B, T, H, N, R, dtype, monkeypatch):
