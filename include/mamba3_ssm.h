@@ -203,8 +203,9 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
  * dtype are read; pointers are not); 0 when the shape runs single-pass only.
  * For small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4; 128 rows of
  * (token, rank) or more, up to 512 sequences) it holds zero-padded f32 copies
- * the chunk-parallel kernels run on; without it those shapes run as one
- * workgroup per sequence.
+ * the chunk-parallel kernels run on, at most 512 MiB (a larger call runs in
+ * parts of its batch or heads through them); without it those shapes run as
+ * one workgroup per sequence.
  * No reference counterpart (see m3_scan_inputs.workspace). */
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
 
@@ -271,7 +272,9 @@ typedef struct m3_scan_grads {
  * chunk kernels take head_dim 64, d_state 64/128, rank 1/2/4 with aligned
  * buffers; every sum has a fixed order, so repeated calls agree bit for bit.
  * Small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens
- * on) run them on zero-padded copies in the workspace.  Other shapes (and
+ * on) run them on zero-padded copies in the workspace, at most 512 MiB (a
+ * larger call runs in parts of its batch, whose shares of da_log and dd_skip
+ * add up in order, or of its heads).  Other shapes (and
  * alignments) take the reverse mode of the recurrence token by token, one
  * workgroup per sequence with states recomputed from checkpoints
  * every 32 tokens (deterministic, and slow: a fallback), up to per-token

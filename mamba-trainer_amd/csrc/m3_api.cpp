@@ -5,7 +5,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -844,21 +843,17 @@ m3_status m3_scan_backward(const m3_scan_inputs *in, const m3_scan_grads *g, voi
     gr.dh0 = st ? g->dh0 : nullptr;
     gr.dlast_u0 = st ? g->dlast_u0 : nullptr;
     gr.dangle0 = (st && st->angle && in->theta) ? g->dangle0 : nullptr;
-    // the chunk kernels' launches
-    const uint64_t launches = (in->theta ? 5 : 4) + (g->dlast_u ? 2 : 0);
+    int launches = 0;
     if (pad) {
-        e = m3::launch_scan_backward_pad(a, gr, in->workspace, s);
-        if (e != hipSuccess) return hip_fail(e, "scan backward launch");
-        g_launches.fetch_add(launches + 2, std::memory_order_relaxed);
+        e = m3::launch_scan_backward_pad(a, gr, in->workspace, s, launches);
     } else if (generic) {
         e = m3::launch_scan_backward_generic(a, gr, in->workspace, s);
-        if (e != hipSuccess) return hip_fail(e, "scan backward launch");
-        g_launches.fetch_add(2, std::memory_order_relaxed);
+        launches = 2;
     } else {
-        e = m3::launch_scan_backward(a, gr, in->workspace, s);
-        if (e != hipSuccess) return hip_fail(e, "scan backward launch");
-        g_launches.fetch_add(launches, std::memory_order_relaxed);
+        e = m3::launch_scan_backward(a, gr, in->workspace, s, launches);
     }
+    if (e != hipSuccess) return hip_fail(e, "scan backward launch");
+    g_launches.fetch_add(launches, std::memory_order_relaxed);
     if (g->dd_skip != nullptr && in->d_skip == nullptr) {
         e = hipMemsetAsync(g->dd_skip, 0, H * sizeof(float), s);
         if (e != hipSuccess) return hip_fail(e, "dd_skip");
@@ -875,7 +870,8 @@ size_t m3_scan_backward_workspace_bytes(const m3_scan_inputs *in) {
     a.h0 = a.last_u0 = nullptr;
     const size_t w = m3::scan_backward_workspace(a);
     if (w) return w;
-    return std::max(m3::scan_backward_pad_workspace(a), m3::scan_backward_generic_workspace(a));
+    const size_t pad = m3::scan_backward_pad_workspace(a);
+    return pad ? pad : m3::scan_backward_generic_workspace(a);
 }
 
 m3_status m3_ssd_chunked(const m3_ssd_args *in, void *y, float *final_state, void *stream) {

@@ -118,6 +118,9 @@ struct ScanLaunch {
     // than 128 tokens (fused) or 64 (three launches), whose records are fewer,
     // for a workspace that holds no more
     int path;
+    // sequences (batch x heads) by which the chunk-parallel form decides on its
+    // cut; 0: this launch's own.  A part of a call is cut as the whole.
+    size_t plan_seqs;
     // the fused launch's look-back: lb_mode 1 gives up at once (tests);
     // lb_spin polls of one flag before giving up (0: the default)
     int lb_mode, lb_spin;
@@ -150,11 +153,12 @@ struct ScanGrads {
     float *dd_skip;                 // [H] or null
     float *dh0, *dlast_u0;          // [B,H,P,N] or null
     float *dangle0;                 // [B,H,N/2] or null
+    int add_sums;                   // da_log and dd_skip are added to (a later part of a batch)
 };
 bool scan_backward_supported(const ScanLaunch &a);
 size_t scan_backward_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &g, void *workspace,
-                                hipStream_t stream);
+                                hipStream_t stream, int &launches);
 // The same gradients for any other shape whose per-token vectors fit 64 KB
 // of LDS (2 P R + 4 N R + 3 N/2 floats): the reverse mode of the recurrence,
 // token by token, one workgroup per sequence (ssd_scan_backward_generic.hip).
@@ -165,15 +169,17 @@ hipError_t launch_scan_backward_generic(const ScanLaunch &a, const ScanGrads &g,
 
 // The heads of small models (head_dim up to 32, d_state up to 64, rank 1, 2 or
 // 4) on zero-padded copies through the kernels above (scan_pad.hip): whether
-// that is the faster form, the workspace it takes (0 where it is not) and the
-// launch, which adds its kernels to `launches`.
+// that is the faster form, the workspace it takes (0 where it is not; at most
+// kPadBytes, through which a larger call runs part by part) and the launch,
+// which adds its kernels to `launches`.
+constexpr size_t kPadBytes = size_t(512) << 20;
 bool scan_pad_wanted(const ScanLaunch &a);
 size_t scan_pad_workspace(const ScanLaunch &a);
 hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches);
 bool scan_backward_pad_wanted(const ScanLaunch &a);
 size_t scan_backward_pad_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,
-                                    hipStream_t stream);
+                                    hipStream_t stream, int &launches);
 
 // The static scratch of m3_scan_no_alloc (M3_NO_ALLOC_SCRATCH_MIB).
 constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;

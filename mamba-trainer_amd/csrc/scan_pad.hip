@@ -24,13 +24,15 @@ constexpr size_t kPadP = 64, kPadN = 64;
 constexpr int kPadThreads = 256;
 
 // How an array's elements move: as they are, or bf16 in the caller's array and
-// f32 in the padded one.
-enum PadKind : uint32_t { kPad16, kPad32, kPadWiden };
+// f32 in the padded one; kMove32: one f32 a row, unpadded.
+enum PadKind : uint32_t { kPad16, kPad32, kPadWiden, kMove32 };
 
 // One array of rows: a source row of `lo` + `hi` elements stands at the front
 // of each half of a padded row of 2 `half` elements (hi = 0: at the front of
 // the row, lo <= 2 half).  Rows come in groups of `live` source rows padded to
-// 1 << group_log rows (1 and 0 for token rows).
+// 1 << group_log rows (1 and 0 for token rows).  The caller's groups are those
+// of `nh` heads out of `heads`: group g of the copy is (g / nh) heads + g % nh
+// from `src` on.
 struct PadArray {
     const void *src;      // the caller's (written by the unpad)
     void *dst;            // the padded copy
@@ -40,11 +42,16 @@ struct PadArray {
     uint32_t quad_log;    // log2 of a padded row's four-element pieces
     uint32_t live, group_log;
     uint32_t kind;
+    uint32_t nh, heads;
 };
-constexpr int kPadArrays = 12;
+constexpr int kPadArrays = 13;   // the backward's inputs: x, b, c, theta, dt, lambda, dy, six of states
 struct PadTable {
     PadArray a[kPadArrays];
 };
+
+__device__ __forceinline__ uint32_t src_group(const PadArray &A, uint32_t g) {
+    return A.nh == A.heads ? g : g / A.nh * A.heads + g % A.nh;
+}
 
 template <typename S, typename D>
 __device__ __forceinline__ void pad_rows(const PadArray &A) {
@@ -59,7 +66,8 @@ __device__ __forceinline__ void pad_rows(const PadArray &A) {
         const bool second = A.hi != 0 && e >= A.half;
         const uint32_t j = second ? e - A.half : e;
         const uint32_t n = p < A.live ? (second ? A.hi : A.lo) : 0;
-        const size_t s = (static_cast<size_t>(g) * A.live + p) * (A.lo + A.hi) + (second ? A.lo : 0) + j;
+        const size_t s = (static_cast<size_t>(src_group(A, g)) * A.live + p) * (A.lo + A.hi) +
+                         (second ? A.lo : 0) + j;
         typedef D D4 __attribute__((ext_vector_type(4)));
         D4 v;
 #pragma unroll
@@ -76,6 +84,18 @@ __device__ __forceinline__ void pad_rows(const PadArray &A) {
     }
 }
 
+// One f32 a row, to the copy or back.
+template <bool OUT>
+__device__ __forceinline__ void move_rows(const PadArray &A) {
+    float *src = static_cast<float *>(const_cast<void *>(A.src)), *dst = static_cast<float *>(A.dst);
+    for (uint32_t g = blockIdx.x * kPadThreads + threadIdx.x; g < A.groups; g += gridDim.x * kPadThreads) {
+        if constexpr (OUT)
+            src[src_group(A, g)] = dst[g];
+        else
+            dst[g] = src[src_group(A, g)];
+    }
+}
+
 // src -> dst zero-padded, one array per blockIdx.y; bound by the writes.
 __global__ void __launch_bounds__(kPadThreads) pad_kernel(PadTable t) {
     const PadArray &A = t.a[blockIdx.y];
@@ -83,8 +103,10 @@ __global__ void __launch_bounds__(kPadThreads) pad_kernel(PadTable t) {
         pad_rows<float, float>(A);
     else if (A.kind == kPad16)
         pad_rows<uint16_t, uint16_t>(A);
-    else
+    else if (A.kind == kPadWiden)
         pad_rows<uint16_t, float>(A);
+    else
+        move_rows<false>(A);
 }
 
 template <typename S, typename D>
@@ -99,10 +121,11 @@ __device__ __forceinline__ void unpad_rows(const PadArray &A) {
         const uint32_t p = row - g * A.live;
         const size_t o = ((static_cast<size_t>(g) << A.group_log) + p) * (4u << A.quad_log) +
                          (e < A.lo ? e : A.half + e - A.lo);
+        const size_t d = (static_cast<size_t>(src_group(A, g)) * A.live + p) * len + e;
         if constexpr (sizeof(S) == sizeof(D))
-            dst[it] = src[o];
+            dst[d] = src[o];
         else
-            dst[it] = from_f32<bf16_t>(src[o]);
+            dst[d] = from_f32<bf16_t>(src[o]);
     }
 }
 
@@ -113,8 +136,10 @@ __global__ void __launch_bounds__(kPadThreads) unpad_kernel(PadTable t) {
         unpad_rows<float, float>(A);
     else if (A.kind == kPad16)
         unpad_rows<uint16_t, uint16_t>(A);
-    else
+    else if (A.kind == kPadWiden)
         unpad_rows<bf16_t, float>(A);
+    else
+        move_rows<true>(A);
 }
 
 // The table's arrays and the largest one's items (four-element pieces to pad,
@@ -135,18 +160,39 @@ struct Pads {
 
 size_t up256(size_t v) { return (v + 255) & ~size_t(255); }
 
-// Sections of the padded copies in the workspace; the kernels' own workspace
-// follows.  Sized for every optional array, present or not.
+// A call's sequences are copied and run in parts, of whole batch entries or of
+// some heads of one, whose copies and kernels' workspace fit the room there is:
+// the padded rows are up to 16 times the caller's and the backward's records 64 x
+// 64 a chunk, 3.4 KB of both a token of a head of 16, so all of a long batch at
+// once would take gigabytes.
+struct PadPart {
+    size_t b0, nb, h0, nh;
+};
+
+// The part as a call of its own, but for the pointers into the arrays.
+ScanLaunch part_of(const ScanLaunch &a, const PadPart &q) {
+    ScanLaunch p = a;
+    p.batch = q.nb;
+    p.heads = q.nh;
+    p.a_log = a.a_log ? a.a_log + q.h0 : nullptr;
+    p.d_skip = a.d_skip ? a.d_skip + q.h0 : nullptr;
+    return p;
+}
+
+// Sections of a part's padded copies in the workspace; the kernels' own
+// workspace follows.  Sized for every optional array, present or not; dt,
+// lambda and their gradients are copied for some heads of a batch entry only.
 struct PadLayout {
     size_t x, b, c, theta, y, h, lu, ang, dh, dlu, dang;         // inputs
     size_t dx, db, dc, dtheta, dh0, dlu0, dang0, hout, luout, angout;
+    size_t dt, lam, ddt, dlam;
     size_t total;
 };
-PadLayout pad_layout(const ScanLaunch &a, bool backward) {
-    const size_t es = backward && a.bf16 ? 2 : 4, rows = a.batch * a.seq * a.heads, bh = a.batch * a.heads;
+PadLayout pad_layout(const ScanLaunch &a, const PadPart &q, bool backward) {
+    const size_t es = backward && a.bf16 ? 2 : 4, rows = q.nb * a.seq * q.nh, bh = q.nb * q.nh;
     const size_t xr = up256(rows * kPadP * a.rank * es), br = up256(rows * kPadN * a.rank * es);
     const size_t tr = up256(rows * (kPadN / 2) * es), st = up256(bh * kPadP * kPadN * 4);
-    const size_t an = up256(bh * (kPadN / 2) * 4);
+    const size_t an = up256(bh * (kPadN / 2) * 4), sc = q.nh < a.heads ? up256(rows * 4) : 0;
     PadLayout l{};
     size_t o = 0;
     auto take = [&o](size_t v) { const size_t at = o; o += v; return at; };
@@ -158,6 +204,8 @@ PadLayout pad_layout(const ScanLaunch &a, bool backward) {
     l.h = take(st);
     l.lu = take(st);
     l.ang = take(an);
+    l.dt = take(sc);
+    l.lam = take(sc);
     if (backward) {
         l.dh = take(st);
         l.dlu = take(st);
@@ -169,6 +217,8 @@ PadLayout pad_layout(const ScanLaunch &a, bool backward) {
         l.dh0 = take(st);
         l.dlu0 = take(st);
         l.dang0 = take(an);
+        l.ddt = take(sc);
+        l.dlam = take(sc);
     } else {
         l.hout = take(st);
         l.luout = take(st);
@@ -184,12 +234,18 @@ uint32_t log2u(size_t v) {
     return k;
 }
 
-// The arrays of a launch in the padded layout.
+// The arrays of a part in the padded layout; `first`: the byte of the caller's
+// array that the part begins at.
+struct PadShape {
+    PadArray a;
+    size_t first;
+};
 struct PadShapes {
-    PadArray x, bc, theta, state, angle;
-    PadShapes(const ScanLaunch &a, bool backward) {
-        const uint32_t rows = static_cast<uint32_t>(a.batch * a.seq * a.heads);
-        const uint32_t bh = static_cast<uint32_t>(a.batch * a.heads);
+    PadShape x, bc, theta, state, angle, scalar;
+    PadShapes(const ScanLaunch &a, const PadPart &part, bool backward) {
+        const uint32_t rows = static_cast<uint32_t>(part.nb * a.seq * part.nh);
+        const uint32_t bh = static_cast<uint32_t>(part.nb * part.nh);
+        const uint32_t nh = static_cast<uint32_t>(part.nh), H = static_cast<uint32_t>(a.heads);
         const uint32_t P = static_cast<uint32_t>(a.head_dim), N = static_cast<uint32_t>(a.d_state);
         const uint32_t R = static_cast<uint32_t>(a.rank);
         // rotation pairs keep their places in the two halves; an odd d_state
@@ -197,39 +253,70 @@ struct PadShapes {
         const uint32_t lo = N / 2 > 0 ? N / 2 : N, hi = N - lo;
         const uint32_t q = log2u(kPadP * R / 4);
         const PadKind t = !a.bf16 ? kPad32 : backward ? kPad16 : kPadWiden;
-        x = PadArray{nullptr, nullptr, rows, P * R, 0, static_cast<uint32_t>(kPadP) * R / 2, q, 1, 0, t};
-        bc = PadArray{nullptr, nullptr, rows, lo * R, hi * R, static_cast<uint32_t>(kPadN) * R / 2, q, 1, 0, t};
-        theta = PadArray{nullptr, nullptr, rows, N / 2, 0, static_cast<uint32_t>(kPadN) / 4, log2u(kPadN / 8), 1, 0, t};
-        state = PadArray{nullptr, nullptr, bh, lo, hi, static_cast<uint32_t>(kPadN) / 2, log2u(kPadN / 4), P, log2u(kPadP), kPad32};
-        angle = PadArray{nullptr, nullptr, bh, N / 2, 0, static_cast<uint32_t>(kPadN) / 4, log2u(kPadN / 8), 1, 0, kPad32};
+        const size_t row0 = part.b0 * a.seq * a.heads + part.h0, seq0 = part.b0 * a.heads + part.h0;
+        const size_t es = a.bf16 ? 2 : 4;
+        x = {{nullptr, nullptr, rows, P * R, 0, static_cast<uint32_t>(kPadP) * R / 2, q, 1, 0, t, nh, H},
+             row0 * P * R * es};
+        bc = {{nullptr, nullptr, rows, lo * R, hi * R, static_cast<uint32_t>(kPadN) * R / 2, q, 1, 0, t, nh, H},
+              row0 * N * R * es};
+        theta = {{nullptr, nullptr, rows, N / 2, 0, static_cast<uint32_t>(kPadN) / 4, log2u(kPadN / 8), 1, 0, t, nh, H},
+                 row0 * (N / 2) * es};
+        state = {{nullptr, nullptr, bh, lo, hi, static_cast<uint32_t>(kPadN) / 2, log2u(kPadN / 4), P,
+                  log2u(kPadP), kPad32, nh, H},
+                 seq0 * P * N * 4};
+        angle = {{nullptr, nullptr, bh, N / 2, 0, static_cast<uint32_t>(kPadN) / 4, log2u(kPadN / 8), 1, 0, kPad32,
+                  nh, H},
+                 seq0 * (N / 2) * 4};
+        scalar = {{nullptr, nullptr, rows, 1, 0, 0, 0, 1, 0, kMove32, nh, H}, row0 * 4};
     }
 };
 
-PadArray with(PadArray p, const void *src, void *dst) {
-    p.src = src;
-    p.dst = dst;
-    return p;
-}
+// A part's arrays as the kernels take them: those copied into `in` before them
+// and out of `out` after them.
+struct PadCopies {
+    char *base;
+    bool some_heads;
+    Pads in, out;
+    const void *put(const PadShape &s, const void *src, size_t off) {
+        return add(in, s, const_cast<void *>(src), off);
+    }
+    void *get(const PadShape &s, void *dst, size_t off) { return add(out, s, dst, off); }
+    // one value a row: in place where the part's rows are the caller's
+    const float *put_row(const PadShape &s, const float *src, size_t off) {
+        return some_heads ? static_cast<const float *>(put(s, src, off)) : src + s.first / 4;
+    }
+    float *get_row(const PadShape &s, float *dst, size_t off) {
+        return some_heads ? static_cast<float *>(get(s, dst, off)) : dst + s.first / 4;
+    }
 
-// The launch on the padded copies under `base` (inputs only; states where the
-// caller has them).
-ScanLaunch padded(const ScanLaunch &a, const PadLayout &l, char *base, const PadShapes &s, Pads &in) {
-    ScanLaunch p = a;
+private:
+    void *add(Pads &to, const PadShape &s, void *ptr, size_t off) {
+        if (ptr == nullptr) return nullptr;
+        PadArray p = s.a;
+        p.src = static_cast<char *>(ptr) + s.first;
+        p.dst = base + off;
+        to.add(p);
+        return base + off;
+    }
+};
+
+// The launch on a part's padded copies (inputs only; states where the caller
+// has them).
+ScanLaunch padded(const ScanLaunch &a, const PadPart &part, const PadLayout &l, const PadShapes &s,
+                  PadCopies &c) {
+    ScanLaunch p = part_of(a, part);
     p.head_dim = kPadP;
     p.d_state = kPadN;
-    p.bf16 = s.x.kind == kPad16;
-    auto put = [&](const PadArray &shape, const void *src, size_t off) -> void * {
-        if (src == nullptr) return nullptr;
-        in.add(with(shape, src, base + off));
-        return base + off;
-    };
-    p.x = put(s.x, a.x, l.x);
-    p.b = put(s.bc, a.b, l.b);
-    p.c = put(s.bc, a.c, l.c);
-    p.theta = put(s.theta, a.theta, l.theta);
-    p.h0 = static_cast<const float *>(put(s.state, a.h0, l.h));
-    p.last_u0 = static_cast<const float *>(put(s.state, a.last_u0, l.lu));
-    p.angle0 = static_cast<const float *>(put(s.angle, a.angle0, l.ang));
+    p.bf16 = s.x.a.kind == kPad16;
+    p.x = c.put(s.x, a.x, l.x);
+    p.b = c.put(s.bc, a.b, l.b);
+    p.c = c.put(s.bc, a.c, l.c);
+    p.theta = c.put(s.theta, a.theta, l.theta);
+    p.dt = c.put_row(s.scalar, a.dt, l.dt);
+    p.lambda = c.put_row(s.scalar, a.lambda, l.lam);
+    p.h0 = static_cast<const float *>(c.put(s.state, a.h0, l.h));
+    p.last_u0 = static_cast<const float *>(c.put(s.state, a.last_u0, l.lu));
+    p.angle0 = static_cast<const float *>(c.put(s.angle, a.angle0, l.ang));
     return p;
 }
 
@@ -257,6 +344,66 @@ bool pad_shape(const ScanLaunch &a, bool backward) {
            scan_fast_supported(padded_shape(a, backward));
 }
 
+size_t part_bytes(const ScanLaunch &a, const PadPart &q, bool backward) {
+    const ScanLaunch p = padded_shape(part_of(a, q), backward);
+    return pad_layout(a, q, backward).total + (backward ? scan_backward_workspace(p) : scan_chunked_workspace(p));
+}
+
+// The largest of n counts from 1 on that fits; 0 if none does.
+template <typename F>
+size_t largest(size_t n, F fits) {
+    size_t lo = 0, hi = n;
+    while (lo < hi) {
+        const size_t mid = lo + (hi - lo + 1) / 2;
+        if (fits(mid))
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+// The first (and largest) part within `room` bytes: the whole call, else as
+// many batch entries as fit, shared out evenly, else as many heads of one;
+// nb = 0 where one sequence does not fit.  Parts of 64 / 256 / 512 / 1024 MiB, us
+// a call, heads of 16, f32: backward, 512 sequences of 512 tokens 1022 / 611 /
+// 608 / 591, 256 of 2048 3642 / 1387 / 1241 / 1157 (1137 at once, in 1.7 GB), 8 of
+// 16384 4410 / 1279 / 793 / 795; forward, 256 of 2048 889 / 503 / 480 / 428.  The
+// kernels these shapes took before need 8 ms and 40 ms for the first two.
+PadPart pad_part(const ScanLaunch &a, bool backward, size_t room) {
+    auto fits = [&](size_t nb, size_t nh) {
+        return part_bytes(a, PadPart{0, nb, 0, nh}, backward) <= room;
+    };
+    if (fits(a.batch, a.heads)) return PadPart{0, a.batch, 0, a.heads};
+    // the most of n that fit, or fewer in as many parts of one size
+    auto share = [](size_t n, auto ok) {
+        const size_t most = largest(n, ok);
+        if (most == 0) return most;
+        const size_t parts = (n + most - 1) / most, even = (n + parts - 1) / parts;
+        return ok(even) ? even : most;
+    };
+    const size_t nb = share(a.batch, [&](size_t v) { return fits(v, a.heads); });
+    if (nb > 0) return PadPart{0, nb, 0, a.heads};
+    const size_t nh = share(a.heads, [&](size_t v) { return fits(1, v); });
+    return nh > 0 ? PadPart{0, 1, 0, nh} : PadPart{};
+}
+
+// f(part) for every part of the call, whose first is q.
+template <typename F>
+hipError_t each_part(const ScanLaunch &a, PadPart q, F f) {
+    const size_t nb = q.nb, nh = q.nh;
+    if (nb == 0) return hipErrorNotSupported;
+    for (q.b0 = 0; q.b0 < a.batch; q.b0 += nb) {
+        q.nb = std::min(nb, a.batch - q.b0);
+        for (q.h0 = 0; q.h0 < a.heads; q.h0 += nh) {
+            q.nh = std::min(nh, a.heads - q.h0);
+            const hipError_t e = f(q);
+            if (e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
 hipError_t launch_pads(const Pads &p, bool out, hipStream_t s) {
     if (p.n == 0) return hipSuccess;
     if (out)
@@ -282,35 +429,34 @@ bool scan_pad_wanted(const ScanLaunch &a) {
 
 size_t scan_pad_workspace(const ScanLaunch &a) {
     if (!scan_pad_wanted(a)) return 0;
-    return pad_layout(a, false).total + scan_chunked_workspace(padded_shape(a, false));
+    const PadPart q = pad_part(a, false, kPadBytes);
+    return q.nb > 0 ? part_bytes(a, q, false) : 0;
 }
 
 hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches) {
-    const PadLayout l = pad_layout(a, false);
-    const PadShapes s(a, false);
-    char *base = static_cast<char *>(workspace);
-    Pads in, out;
-    ScanLaunch p = padded(a, l, base, s, in);
-    auto get = [&](const PadArray &shape, void *dst, size_t off) -> void * {
-        if (dst == nullptr) return nullptr;
-        out.add(with(shape, dst, base + off));
-        return base + off;
-    };
-    p.y = get(s.x, a.y, l.y);
-    p.h_out = static_cast<float *>(get(s.state, a.h_out, l.hout));
-    p.last_u_out = static_cast<float *>(get(s.state, a.last_u_out, l.luout));
-    p.angle_out = static_cast<float *>(get(s.angle, a.angle_out, l.angout));
-    hipError_t e = launch_pads(in, false, stream);
-    if (e != hipSuccess) return e;
-    if (scan_chunked_workspace(p) > 0) {
-        e = launch_scan_chunked(p, base + l.total, stream, launches);
-    } else {
-        e = launch_scan(p, stream);
-        ++launches;
-    }
-    if (e != hipSuccess) return e;
-    launches += 2;
-    return launch_pads(out, true, stream);
+    const PadPart first = pad_part(a, false, kPadBytes);
+    return each_part(a, first, [&](const PadPart &q) {
+        const PadLayout l = pad_layout(a, q, false);
+        const PadShapes s(a, q, false);
+        PadCopies c{static_cast<char *>(workspace), q.nh < a.heads, {}, {}};
+        ScanLaunch p = padded(a, q, l, s, c);
+        p.plan_seqs = first.nb * first.nh;   // a short last part is cut as the others
+        p.y = c.get(s.x, a.y, l.y);
+        p.h_out = static_cast<float *>(c.get(s.state, a.h_out, l.hout));
+        p.last_u_out = static_cast<float *>(c.get(s.state, a.last_u_out, l.luout));
+        p.angle_out = static_cast<float *>(c.get(s.angle, a.angle_out, l.angout));
+        hipError_t e = launch_pads(c.in, false, stream);
+        if (e != hipSuccess) return e;
+        if (scan_chunked_workspace(p) > 0) {
+            e = launch_scan_chunked(p, c.base + l.total, stream, launches);
+        } else {
+            e = launch_scan(p, stream);
+            ++launches;
+        }
+        if (e != hipSuccess) return e;
+        launches += 2;
+        return launch_pads(c.out, true, stream);
+    });
 }
 
 // The token walk against padded (f32, head_dim and d_state 16, us per call): 2
@@ -323,43 +469,42 @@ bool scan_backward_pad_wanted(const ScanLaunch &a) { return a.seq >= 8 && pad_sh
 
 size_t scan_backward_pad_workspace(const ScanLaunch &a) {
     if (!scan_backward_pad_wanted(a)) return 0;
-    return pad_layout(a, true).total + scan_backward_workspace(padded_shape(a, true));
+    const PadPart q = pad_part(a, true, kPadBytes);
+    return q.nb > 0 ? part_bytes(a, q, true) : 0;
 }
 
 hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,
-                                    hipStream_t stream) {
-    const PadLayout l = pad_layout(a, true);
-    const PadShapes s(a, true);
-    char *base = static_cast<char *>(workspace);
-    Pads in, out;
-    const ScanLaunch p = padded(a, l, base, s, in);
-    ScanGrads q = g;
-    auto put = [&](const PadArray &shape, const void *src, size_t off) -> void * {
-        if (src == nullptr) return nullptr;
-        in.add(with(shape, src, base + off));
-        return base + off;
-    };
-    auto get = [&](const PadArray &shape, void *dst, size_t off) -> void * {
-        if (dst == nullptr) return nullptr;
-        out.add(with(shape, dst, base + off));
-        return base + off;
-    };
-    q.dy = put(s.x, g.dy, l.y);
-    q.dh_out = static_cast<const float *>(put(s.state, g.dh_out, l.dh));
-    q.dlast_u_out = static_cast<const float *>(put(s.state, g.dlast_u_out, l.dlu));
-    q.dangle_out = static_cast<const float *>(put(s.angle, g.dangle_out, l.dang));
-    q.dx = get(s.x, g.dx, l.dx);
-    q.db = get(s.bc, g.db, l.db);
-    q.dc = get(s.bc, g.dc, l.dc);
-    q.dtheta = get(s.theta, g.dtheta, l.dtheta);
-    q.dh0 = static_cast<float *>(get(s.state, g.dh0, l.dh0));
-    q.dlast_u0 = static_cast<float *>(get(s.state, g.dlast_u0, l.dlu0));
-    q.dangle0 = static_cast<float *>(get(s.angle, g.dangle0, l.dang0));
-    hipError_t e = launch_pads(in, false, stream);
-    if (e != hipSuccess) return e;
-    e = launch_scan_backward(p, q, base + l.total, stream);
-    if (e != hipSuccess) return e;
-    return launch_pads(out, true, stream);
+                                    hipStream_t stream, int &launches) {
+    return each_part(a, pad_part(a, true, kPadBytes), [&](const PadPart &part) {
+        const PadLayout l = pad_layout(a, part, true);
+        const PadShapes s(a, part, true);
+        PadCopies c{static_cast<char *>(workspace), part.nh < a.heads, {}, {}};
+        const ScanLaunch p = padded(a, part, l, s, c);
+        ScanGrads q = g;
+        q.dy = c.put(s.x, g.dy, l.y);
+        q.dh_out = static_cast<const float *>(c.put(s.state, g.dh_out, l.dh));
+        q.dlast_u_out = static_cast<const float *>(c.put(s.state, g.dlast_u_out, l.dlu));
+        q.dangle_out = static_cast<const float *>(c.put(s.angle, g.dangle_out, l.dang));
+        q.dx = c.get(s.x, g.dx, l.dx);
+        q.db = c.get(s.bc, g.db, l.db);
+        q.dc = c.get(s.bc, g.dc, l.dc);
+        q.ddt = c.get_row(s.scalar, g.ddt, l.ddt);
+        q.dlambda = c.get_row(s.scalar, g.dlambda, l.dlam);
+        q.dtheta = c.get(s.theta, g.dtheta, l.dtheta);
+        q.dh0 = static_cast<float *>(c.get(s.state, g.dh0, l.dh0));
+        q.dlast_u0 = static_cast<float *>(c.get(s.state, g.dlast_u0, l.dlu0));
+        q.dangle0 = static_cast<float *>(c.get(s.angle, g.dangle0, l.dang0));
+        // the sums over the batch, part after part
+        q.da_log = g.da_log + part.h0;
+        q.dd_skip = g.dd_skip ? g.dd_skip + part.h0 : nullptr;
+        q.add_sums = part.b0 > 0;
+        hipError_t e = launch_pads(c.in, false, stream);
+        if (e != hipSuccess) return e;
+        e = launch_scan_backward(p, q, c.base + l.total, stream, launches);
+        if (e != hipSuccess) return e;
+        launches += 2;
+        return launch_pads(c.out, true, stream);
+    });
 }
 
 }  // namespace m3

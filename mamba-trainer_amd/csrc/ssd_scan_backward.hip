@@ -54,6 +54,7 @@ struct BwdArgs {
     float *dd_skip;           // [H] or null
     float *dh0, *dlast_u0;    // [B,H,P,N] or null
     float *dangle0;           // [B,H,N/2] or null
+    bool add_sums;            // da_log and dd_skip are added to
 };
 
 // Backward workspace, 256-byte aligned sections.  Per (batch, head, chunk):
@@ -1343,8 +1344,8 @@ __global__ void __launch_bounds__(256) bwd_head_kernel(ScanLaunch a, BwdArgs g, 
     sa = block_sum(sa, red);
     sd = block_sum(sd, red + 8);
     if (threadIdx.x == 0) {
-        g.da_log[hh] = sa;
-        if (g.dd_skip != nullptr) g.dd_skip[hh] = sd;
+        g.da_log[hh] = g.add_sums ? g.da_log[hh] + sa : sa;
+        if (g.dd_skip != nullptr) g.dd_skip[hh] = g.add_sums ? g.dd_skip[hh] + sd : sd;
     }
 }
 
@@ -1451,8 +1452,13 @@ hipError_t set_lds(K kern, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
 
+hipError_t launched(int &launches) {
+    ++launches;
+    return hipGetLastError();
+}
+
 template <typename T, int N, int R>
-hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStream_t s) {
+hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStream_t s, int &launches) {
     constexpr int QT = kRows / R;
     const int nck = static_cast<int>((a.seq + QT - 1) / QT);
     const size_t bh = a.batch * a.heads, bhk = bh * nck;
@@ -1484,41 +1490,41 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
     if (g.dlast_u_out != nullptr) {
         // the outgoing last_u's terms; its angle term seeds the angle passes
         hipLaunchKernelGGL((bwd_last_u_kernel<T, N, R>), dim3(bh), dim3(256), 0, s, a, g, w);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launched(launches)) != hipSuccess) return e;
         if (a.theta != nullptr) gm.dangle_out = w.seed;
     }
     const BwdArgs &g2 = gm;
     hipLaunchKernelGGL((bwd_passes_kernel<T, N, R>), dim3(2 * bh * (N / 32)), dim3(256), 0, s, a, g2, w,
                        nck);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launched(launches)) != hipSuccess) return e;
     hipLaunchKernelGGL((bwd_chunk_kernel<T, N, R>), dim3(bhk), dim3(kBT), lds, s, a, g2, w, nck);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launched(launches)) != hipSuccess) return e;
     if (a.theta != nullptr) {
         hipLaunchKernelGGL((bwd_angle_kernel<N>), dim3(bh), dim3(64), 0, s, a, g2, w, nck);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launched(launches)) != hipSuccess) return e;
     }
     hipLaunchKernelGGL((bwd_token_kernel<T, N, R>), dim3(bhk), dim3(256), 0, s, a, g2, w, nck);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launched(launches)) != hipSuccess) return e;
     hipLaunchKernelGGL(bwd_head_kernel, dim3(a.heads), dim3(256), 0, s, a, g2, w, nck);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launched(launches)) != hipSuccess) return e;
     if (g.dlast_u_out != nullptr) {
         hipLaunchKernelGGL((bwd_last_add_kernel<T, N, R>), dim3(bh), dim3(256), 0, s, a, g, w);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launched(launches)) != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
 template <typename T>
-hipError_t launch_bwd_t(const ScanLaunch &a, const BwdArgs &g, char *ws, hipStream_t s) {
+hipError_t launch_bwd_t(const ScanLaunch &a, const BwdArgs &g, char *ws, hipStream_t s, int &launches) {
     const size_t n = a.d_state, r = a.rank;
     if (n == 128) {
-        if (r == 1) return launch_bwd<T, 128, 1>(a, g, ws, s);
-        if (r == 2) return launch_bwd<T, 128, 2>(a, g, ws, s);
-        if (r == 4) return launch_bwd<T, 128, 4>(a, g, ws, s);
+        if (r == 1) return launch_bwd<T, 128, 1>(a, g, ws, s, launches);
+        if (r == 2) return launch_bwd<T, 128, 2>(a, g, ws, s, launches);
+        if (r == 4) return launch_bwd<T, 128, 4>(a, g, ws, s, launches);
     } else if (n == 64) {
-        if (r == 1) return launch_bwd<T, 64, 1>(a, g, ws, s);
-        if (r == 2) return launch_bwd<T, 64, 2>(a, g, ws, s);
-        if (r == 4) return launch_bwd<T, 64, 4>(a, g, ws, s);
+        if (r == 1) return launch_bwd<T, 64, 1>(a, g, ws, s, launches);
+        if (r == 2) return launch_bwd<T, 64, 2>(a, g, ws, s, launches);
+        if (r == 4) return launch_bwd<T, 64, 4>(a, g, ws, s, launches);
     }
     return hipErrorNotSupported;
 }
@@ -1537,7 +1543,7 @@ size_t scan_backward_workspace(const ScanLaunch &a) {
 }
 
 hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *workspace,
-                                hipStream_t stream) {
+                                hipStream_t stream, int &launches) {
     if (!scan_backward_supported(a)) return hipErrorNotSupported;
     BwdArgs g;
     g.dy = gr.dy;
@@ -1555,9 +1561,10 @@ hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *
     g.dh0 = gr.dh0;
     g.dlast_u0 = gr.dlast_u0;
     g.dangle0 = gr.dangle0;
+    g.add_sums = gr.add_sums != 0;
     char *ws = static_cast<char *>(workspace);
-    if (a.bf16) return launch_bwd_t<bf16_t>(a, g, ws, stream);
-    return launch_bwd_t<float>(a, g, ws, stream);
+    if (a.bf16) return launch_bwd_t<bf16_t>(a, g, ws, stream, launches);
+    return launch_bwd_t<float>(a, g, ws, stream, launches);
 }
 
 }  // namespace m3

@@ -3258,6 +3258,8 @@ struct SegPlan {
     int nsub, kseg, nseg;
 };
 
+size_t plan_seqs(const ScanLaunch &a) { return a.plan_seqs ? a.plan_seqs : a.batch * a.heads; }
+
 SegPlan seg_plan(const ScanLaunch &a) {
     const size_t qt = static_cast<size_t>(rows_for(a)) / a.rank;
     const size_t nsub = (a.seq + qt - 1) / qt;
@@ -3279,7 +3281,7 @@ SegPlan seg_plan(const ScanLaunch &a) {
     const size_t rounds = a.rank > 1 && !mimo4 ? 6 : 1;
     // segments per sequence that fill the rounds without spilling into one
     // more, then the sub-chunks each needs
-    const size_t bh = a.batch * a.heads;
+    const size_t bh = plan_seqs(a);
     const size_t fill = bh < rounds * slots ? rounds * slots / bh : 1;
     size_t k = (nsub + fill - 1) / fill;
     // A segment is a serial walk over its sub-chunks in both heavy kernels (7 to
@@ -3479,8 +3481,8 @@ hipError_t launch_t(const ScanLaunch &a, char *ws, hipStream_t s) {
 size_t scan_chunked_workspace(const ScanLaunch &a) {
     if (!scan_fast_supported(a) || a.seq == 0) return 0;
     const size_t seqs = a.batch * a.heads, cus = device_cus();
-    const size_t rounds = (seqs + cus - 1) / cus;
-    if (seqs * 100 >= rounds * cus * 85) return 0;
+    const size_t rounds = (plan_seqs(a) + cus - 1) / cus;
+    if (plan_seqs(a) * 100 >= rounds * cus * 85) return 0;
     if (fused_covered(a)) return fused_layout(seqs * fused_plan(a).nseg, a.d_state).total;
     return chunked_layout(seqs * seg_plan(a).nseg, a.d_state, a.bf16 != 0).total;
 }

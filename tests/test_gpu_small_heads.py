@@ -103,6 +103,79 @@ def test_workspace_queries_at_the_edges():
     assert _query(2, 256, 4, 16, 16, 1, bf16)[1] < _query(2, 256, 4, 16, 16, 1, f32)[1]
 
 
+def test_workspace_queries_are_bounded():
+    """Large calls run part by part: neither query passes 512 MiB where the
+    padded copies are asked for, whatever the batch, the window or the heads;
+    a sequence whose own copies do not fit takes the kernels of before."""
+    from mamba3 import _lib
+    for dt in (_lib.M3_F32, _lib.M3_BF16):
+        for B, T, H, P, N, R in ((256, 2048, 4, 16, 16, 1), (64, 4096, 16, 16, 16, 1), (512, 8192, 4, 16, 16, 1),
+                                 (1, 40000, 8, 32, 64, 1), (3, 9000, 9, 8, 64, 4), (128, 512, 4, 16, 16, 1)):
+            fw, bw = _query(B, T, H, P, N, R, dt)
+            assert 0 < bw <= 512 << 20, (B, T, H, bw)
+            assert (0 < fw <= 512 << 20) if B * H <= 512 else fw == 0, (B, T, H, fw)
+
+
+# more rows than 512 MiB of copies hold: parts of the batch, the last one short;
+# parts of the heads of one entry, forward and backward, with every option
+LARGE = [(64, 1000, 8, 16, 16, 1, "f32"), (63, 1000, 8, 16, 16, 1, "bf16"), (1, 70000, 7, 8, 16, 1, "f32"),
+         (2, 20000, 9, 6, 12, 4, "bf16")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", LARGE, ids=[repr(c) for c in LARGE])
+def test_parts_equal_calls_of_their_own(case):
+    """Each batch entry's and head's outputs and gradients against a call on
+    that sequence alone (whose segments are cut for one sequence: to f32
+    rounding, and the rounding of bf16 storage), the heads' sums against the
+    sum of those calls."""
+    from mamba3.ssm import ScanInputs, SsmState, mamba3_scan, mamba3_scan_backward
+    B, T, H, P, N, R, dtype = case
+    ty = torch.bfloat16 if dtype == "bf16" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(B * T)
+    r = lambda *s: torch.randn(s, device="cuda", generator=g)
+    u = lambda *s: torch.rand(s, device="cuda", generator=g)
+    x, b, c = r(B, T, H, P, R).to(ty), (r(B, T, H, N, R) / N ** 0.5).to(ty), (r(B, T, H, N, R) / N ** 0.5).to(ty)
+    dt, a_log, lam, theta, skip = u(B, T, H) * 0.1, u(H) * 2.7, u(B, T, H), (u(B, T, H, N // 2) * 3).to(ty), r(H)
+    st = (r(B, H, P, N) * 0.1, r(B, H, P, N) * 0.1, u(B, H, N // 2) * 3)
+    dy, dh, dang, dlu = r(B, T, H, P, R).to(ty), r(B, H, P, N), r(B, H, N // 2), r(B, H, P, N)
+
+    def call(bs, hs):
+        pick = lambda t: t[bs][:, :, hs].contiguous()
+        seq = lambda t: t[bs][:, hs].contiguous()
+        si = ScanInputs(pick(x), pick(b), pick(c), pick(dt), a_log[hs].contiguous(), pick(lam))
+        si = si.with_theta(pick(theta)).with_skip(skip[hs].contiguous()).with_state(
+            SsmState(*[seq(t) for t in st]))
+        out = mamba3_scan(si)
+        gr = mamba3_scan_backward(si, pick(dy), seq(dh), seq(dang), seq(dlu))
+        return out, gr
+
+    all_b, all_h = slice(None), slice(None)
+    (out, gr), n = _launches(lambda: call(all_b, all_h))
+    assert n >= 10 + 18, "one part would be 5 and 9 launches"
+    tol = 2 * (BF16_TOL if dtype == "bf16" else F32_TOL)
+    picks = [(bb, hh) for bb in sorted({0, 1 % B, B // 2, B - 1}) for hh in sorted({0, H // 2, H - 1})]
+    for bb, hh in picks:
+        bs, hs = slice(bb, bb + 1), slice(hh, hh + 1)
+        o1, g1 = call(bs, hs)
+        near = lambda a, e, t: rel_l2(host(a), host(e)) <= t
+        assert near(out.y[bs][:, :, hs], o1.y, tol), (bb, hh)
+        assert near(out.state.h[bs, hs], o1.state.h, 2 * F32_TOL), (bb, hh)
+        assert near(out.state.last_u[bs, hs], o1.state.last_u, 2 * F32_TOL), (bb, hh)
+        for k in ("x", "b", "c", "theta"):
+            assert near(getattr(gr, k)[bs][:, :, hs], getattr(g1, k), tol), (bb, hh, k)
+        for k in ("dt", "lam"):
+            assert near(getattr(gr, k)[bs][:, :, hs], getattr(g1, k), 2 * F32_TOL), (bb, hh, k)
+        for k in ("h0", "last_u0", "angle0"):
+            assert near(getattr(gr, k)[bs, hs], getattr(g1, k), 2 * F32_TOL), (bb, hh, k)
+    for hh in (0, H - 1):
+        each = [call(slice(bb, bb + 1), slice(hh, hh + 1))[1] for bb in range(B)]
+        for k in ("a_log", "d_skip"):
+            e = np.array([float(getattr(t, k)[0]) for t in each], np.float64)
+            # f32 sums of terms that cancel: against the terms' own size
+            assert abs(float(getattr(gr, k)[hh]) - e.sum()) <= 2 * F32_TOL * np.sqrt((e * e).sum()), (hh, k)
+
+
 @pytest.mark.gpu
 def test_a_smaller_workspace_runs_the_kernels_of_before():
     from mamba3 import _lib
