@@ -204,8 +204,9 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
  * For small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4; 128 rows of
  * (token, rank) or more, up to 512 sequences) it holds zero-padded f32 copies
  * the chunk-parallel kernels run on, at most 512 MiB (a larger call runs in
- * parts of its batch or heads through them); without it those shapes run as
- * one workgroup per sequence.
+ * parts of its batch or heads through them); without it, and where one
+ * sequence's copies exceed M3_NO_ALLOC_SCRATCH_MIB (from some 20,000 tokens
+ * of rank 1 on, 7,000 of rank 4), those shapes run as one workgroup per sequence.
  * No reference counterpart (see m3_scan_inputs.workspace). */
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
 
@@ -216,7 +217,8 @@ size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
  * that cannot allocate device memory (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  The chunk-parallel path's workspace
  * is a file-scope device array of M3_NO_ALLOC_SCRATCH_MIB MiB instead of the
- * caller's buffer (in->workspace and in->workspace_bytes are ignored).  Each GPU
+ * caller's buffer (in->workspace and in->workspace_bytes are ignored); small
+ * heads' padded copies pass through it in as many parts as they need.  Each GPU
  * holds its own copy of that array from the moment the library's code object is
  * loaded on that device (the first launch of any of its kernels there) until
  * the process ends, so every process that uses the library on a GPU holds those

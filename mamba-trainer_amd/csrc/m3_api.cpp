@@ -254,7 +254,8 @@ static std::atomic<int> g_scan_path{0}, g_lb_mode{0}, g_lb_spin{0};
 // the specialised kernels only.
 static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
                             const void *gate_z, size_t gate_stride, void *stream,
-                            int path = -1, size_t theta_stride = 0);
+                            int path = -1, size_t theta_stride = 0,
+                            size_t pad_room = m3::kPadBytes);
 
 // The step kernel's LDS holds B~, C~ (d_state x rank each) and x (head_dim x
 // rank) as f32: 64 KB.
@@ -366,7 +367,7 @@ static m3_status scan_f16(const m3_scan_inputs *in, const m3_scan_output *out, v
 
 static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
                             const void *gate_z, size_t gate_stride, void *stream,
-                            int path, size_t theta_stride) {
+                            int path, size_t theta_stride, size_t pad_room) {
     if (in == nullptr || out == nullptr) return fail(M3_ERR_ARGUMENT, "inputs/outputs are NULL");
     if (!dtype_ok(in->dtype)) return fail(M3_ERR_ARGUMENT, "unknown dtype %d", in->dtype);
     if (in->rank == 0) return fail(M3_ERR_CONFIG, "MIMO rank must be positive");
@@ -495,10 +496,10 @@ static m3_status scan_entry(const m3_scan_inputs *in, const m3_scan_output *out,
         a.gate_z = gate_z;
         a.gate_stride = gate_stride;
     }
-    const size_t pad_need = need > 0 || !ws_aligned ? 0 : m3::scan_pad_workspace(a);
+    const size_t pad_need = need > 0 || !ws_aligned ? 0 : m3::scan_pad_workspace(a, pad_room);
     int launches = 0;
     if (pad_need > 0 && in->workspace != nullptr && in->workspace_bytes >= pad_need) {
-        e = m3::launch_scan_pad(a, in->workspace, s, launches);
+        e = m3::launch_scan_pad(a, in->workspace, pad_room, s, launches);
     } else if (chunked) {
         e = m3::launch_scan_chunked(a, in->workspace, s, launches);
     } else {
@@ -539,9 +540,8 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
 
 }  // extern "C"
 
-// pads: the padded copies of small heads included (m3_scan_no_alloc's static
-// scratch runs those shapes without a workspace, as a caller who passes none).
-static size_t workspace_bytes_for(const m3_scan_inputs *in, int path, bool pads) {
+// pad_room: the bytes the padded copies of small heads may take.
+static size_t workspace_bytes_for(const m3_scan_inputs *in, int path, size_t pad_room) {
     if (in == nullptr || !dtype_ok(in->dtype) || in->seq == 0) return 0;
     m3::ScanLaunch a{};
     a.path = path;
@@ -559,13 +559,13 @@ static size_t workspace_bytes_for(const m3_scan_inputs *in, int path, bool pads)
     a.x = a.b = a.c = dummy;
     a.y = dummy;
     const size_t need = m3::scan_chunked_workspace(a);
-    return need == 0 && pads ? m3::scan_pad_workspace(a) : need;
+    return need == 0 ? m3::scan_pad_workspace(a, pad_room) : need;
 }
 
 extern "C" {
 
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in) {
-    return workspace_bytes_for(in, g_scan_path.load(std::memory_order_relaxed), true);
+    return workspace_bytes_for(in, g_scan_path.load(std::memory_order_relaxed), m3::kPadBytes);
 }
 
 m3_status m3_debug_scan_options(int32_t path, int32_t lookback_mode, int32_t lookback_spin) {
@@ -650,10 +650,10 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
     local.workspace = nullptr;
     local.workspace_bytes = 0;
     int path = g_scan_path.load(std::memory_order_relaxed);
-    size_t need = workspace_bytes_for(&local, path, false);
+    size_t need = workspace_bytes_for(&local, path, kNoAllocScratchBytes);
     if (need > kNoAllocScratchBytes && path == 0) {
         // the fused launch's records do not fit: the three launches' may
-        const size_t three = workspace_bytes_for(&local, 1, false);
+        const size_t three = workspace_bytes_for(&local, 1, kNoAllocScratchBytes);
         if (three <= kNoAllocScratchBytes) {
             path = 1;
             need = three;
@@ -664,7 +664,8 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
                     "this scan needs %zu bytes of scratch; m3_scan_no_alloc's static scratch holds "
                     "%zu (%d MiB): call m3_scan with a caller workspace instead",
                     need, kNoAllocScratchBytes, M3_NO_ALLOC_SCRATCH_MIB);
-    if (need == 0) return scan_entry(&local, out, nullptr, 0, stream, path);
+    auto run = [&] { return scan_entry(&local, out, nullptr, 0, stream, path, 0, kNoAllocScratchBytes); };
+    if (need == 0) return run();
     int dev = -1;
     m3_status st = M3_ERR_HIP;
     void *p = scratch_for_current_device(dev, &st);
@@ -675,7 +676,7 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(s, &cap);
     if (e != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
-    if (cap != hipStreamCaptureStatusNone) return scan_entry(&local, out, nullptr, 0, stream, path);
+    if (cap != hipStreamCaptureStatusNone) return run();
     std::lock_guard<std::mutex> lock(g_guard_mu);
     if (g_guard_set[dev] && g_guard_stream[dev] != s) {
         e = hipEventQuery(g_guard_event[dev]);
@@ -687,7 +688,7 @@ m3_status m3_scan_no_alloc(const m3_scan_inputs *in, const m3_scan_output *out, 
         }
         if (e != hipSuccess) return hip_fail(e, "hipEventQuery");
     }
-    st = scan_entry(&local, out, nullptr, 0, stream, path);
+    st = run();
     if (st != M3_OK) return st;
     if (g_guard_event[dev] == nullptr) {
         e = hipEventCreateWithFlags(&g_guard_event[dev], hipEventDisableTiming);

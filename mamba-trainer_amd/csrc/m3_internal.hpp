@@ -170,12 +170,14 @@ hipError_t launch_scan_backward_generic(const ScanLaunch &a, const ScanGrads &g,
 // The heads of small models (head_dim up to 32, d_state up to 64, rank 1, 2 or
 // 4) on zero-padded copies through the kernels above (scan_pad.hip): whether
 // that is the faster form, the workspace it takes (0 where it is not; at most
-// kPadBytes, through which a larger call runs part by part) and the launch,
-// which adds its kernels to `launches`.
+// kPadBytes, or the forward's `room` from the static scratch's size on, through
+// which a larger call runs part by part) and the launch, which adds its kernels
+// to `launches`.
 constexpr size_t kPadBytes = size_t(512) << 20;
 bool scan_pad_wanted(const ScanLaunch &a);
-size_t scan_pad_workspace(const ScanLaunch &a);
-hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches);
+size_t scan_pad_workspace(const ScanLaunch &a, size_t room);
+hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, size_t room, hipStream_t stream,
+                           int &launches);
 bool scan_backward_pad_wanted(const ScanLaunch &a);
 size_t scan_backward_pad_workspace(const ScanLaunch &a);
 hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, void *workspace,

@@ -427,20 +427,32 @@ bool scan_pad_wanted(const ScanLaunch &a) {
     return a.seq * a.rank >= 128 && a.batch * a.heads <= 512 && pad_shape(a, false);
 }
 
-size_t scan_pad_workspace(const ScanLaunch &a) {
-    if (!scan_pad_wanted(a)) return 0;
+// The call with its cut decided, by the part that kPadBytes hold: the same
+// results through any room, and m3_scan_no_alloc's those of m3_scan.
+static ScanLaunch planned(const ScanLaunch &a) {
     const PadPart q = pad_part(a, false, kPadBytes);
-    return q.nb > 0 ? part_bytes(a, q, false) : 0;
+    ScanLaunch p = a;
+    p.plan_seqs = q.nb * q.nh;
+    return p;
 }
 
-hipError_t launch_scan_pad(const ScanLaunch &a, void *workspace, hipStream_t stream, int &launches) {
-    const PadPart first = pad_part(a, false, kPadBytes);
-    return each_part(a, first, [&](const PadPart &q) {
+size_t scan_pad_workspace(const ScanLaunch &a, size_t room) {
+    if (!scan_pad_wanted(a)) return 0;
+    const ScanLaunch p = planned(a);
+    // a sequence that the static scratch does not hold (from some 20,000 tokens of
+    // rank 1 on, 7,000 of rank 4) takes one workgroup in either call
+    if (p.plan_seqs == 0 || part_bytes(p, PadPart{0, 1, 0, 1}, false) > kNoAllocScratchBytes) return 0;
+    return part_bytes(p, pad_part(p, false, room), false);
+}
+
+hipError_t launch_scan_pad(const ScanLaunch &call, void *workspace, size_t room, hipStream_t stream,
+                           int &launches) {
+    const ScanLaunch a = planned(call);
+    return each_part(a, pad_part(a, false, room), [&](const PadPart &q) {
         const PadLayout l = pad_layout(a, q, false);
         const PadShapes s(a, q, false);
         PadCopies c{static_cast<char *>(workspace), q.nh < a.heads, {}, {}};
         ScanLaunch p = padded(a, q, l, s, c);
-        p.plan_seqs = first.nb * first.nh;   // a short last part is cut as the others
         p.y = c.get(s.x, a.y, l.y);
         p.h_out = static_cast<float *>(c.get(s.state, a.h_out, l.hout));
         p.last_u_out = static_cast<float *>(c.get(s.state, a.last_u_out, l.luout));
