@@ -272,7 +272,8 @@ typedef struct m3_scan_grads {
  * m3_scan_backward_workspace_bytes(in) bytes, 256-byte aligned).  The forward
  * chunk states are recomputed; the forward outputs are not needed.  The
  * chunk kernels take head_dim 64, d_state 64/128, rank 1/2/4 with aligned
- * buffers; every sum has a fixed order, so repeated calls agree bit for bit.
+ * buffers (bf16 storage at d_state 64 also in some half of the workspace, with
+ * the sequential passes run twice); every sum has a fixed order, so repeated calls agree bit for bit.
  * Small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens
  * on) run them on zero-padded copies in the workspace, at most 512 MiB (a
  * larger call runs in parts of its batch, whose shares of da_log and dd_skip

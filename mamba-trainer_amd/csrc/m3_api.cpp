@@ -823,7 +823,7 @@ m3_status m3_scan_backward(const m3_scan_inputs *in, const m3_scan_grads *g, voi
     const bool pad = pad_need > 0 && in->workspace_bytes >= pad_need;
     const size_t need = pad ? pad_need
                             : generic ? m3::scan_backward_generic_workspace(a)
-                                      : m3::scan_backward_workspace(a);
+                                      : m3::scan_backward_workspace_least(a);
     if (in->workspace == nullptr || in->workspace_bytes < need ||
         (reinterpret_cast<uintptr_t>(in->workspace) & 255u) != 0)
         return fail(M3_ERR_ARGUMENT, "the backward needs a 256-byte aligned workspace of %zu bytes",
@@ -851,7 +851,7 @@ m3_status m3_scan_backward(const m3_scan_inputs *in, const m3_scan_grads *g, voi
         e = m3::launch_scan_backward_generic(a, gr, in->workspace, s);
         launches = 2;
     } else {
-        e = m3::launch_scan_backward(a, gr, in->workspace, s, launches);
+        e = m3::launch_scan_backward(a, gr, in->workspace, in->workspace_bytes, s, launches);
     }
     if (e != hipSuccess) return hip_fail(e, "scan backward launch");
     g_launches.fetch_add(launches, std::memory_order_relaxed);

@@ -157,7 +157,8 @@ struct ScanGrads {
 };
 bool scan_backward_supported(const ScanLaunch &a);
 size_t scan_backward_workspace(const ScanLaunch &a);
-hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &g, void *workspace,
+size_t scan_backward_workspace_least(const ScanLaunch &a);   // the smallest that runs, slower
+hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &g, void *workspace, size_t bytes,
                                 hipStream_t stream, int &launches);
 // The same gradients for any other shape whose per-token vectors fit 64 KB
 // of LDS (2 P R + 4 N R + 3 N/2 floats): the reverse mode of the recurrence,

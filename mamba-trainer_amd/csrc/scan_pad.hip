@@ -512,7 +512,7 @@ hipError_t launch_scan_backward_pad(const ScanLaunch &a, const ScanGrads &g, voi
         q.add_sums = part.b0 > 0;
         hipError_t e = launch_pads(c.in, false, stream);
         if (e != hipSuccess) return e;
-        e = launch_scan_backward(p, q, c.base + l.total, stream, launches);
+        e = launch_scan_backward(p, q, c.base + l.total, scan_backward_workspace(p), stream, launches);
         if (e != hipSuccess) return e;
         launches += 2;
         return launch_pads(c.out, true, stream);

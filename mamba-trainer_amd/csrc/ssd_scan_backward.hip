@@ -59,31 +59,33 @@ struct BwdArgs {
 
 // Backward workspace, 256-byte aligned sections.  Per (batch, head, chunk):
 // S_k and Gh_k as f32 [p-tile][n-tile][lane][4] MFMA D-layout records of the
-// [P][N] state and the chunk decay e_k.
+// [P][N] state and the chunk decay e_k, for a window of `wn` chunks of every
+// sequence (all of them where the workspace holds that): the passes and the
+// chunk kernel run once a window, each of whose passes walks the whole sequence
+// and writes its own chunks' records.  pd and pa add up over the windows.
 // With an upstream gradient of the outgoing last_u: the angle seed (that
 // gradient's angle term plus dL/dangle) and the last token's dx and db terms.
 struct BwdLayout {
-    size_t s, gh, eda, cin, ctot, off, da, dg, dw, pd, pa, pfirst;
+    size_t s, gh, eda, cin, ctot, da, dg, dw, pd, pa, pfirst;
     size_t seed, lux, lub, total;
 };
 
 size_t balign(size_t v) { return (v + 255) & ~size_t(255); }
 
-BwdLayout bwd_layout(size_t bh, size_t nck, size_t seq, size_t n, size_t r) {
-    const size_t bhk = bh * nck, rec = bhk * kP * n * 4, pairs = bhk * (n / 2) * 4;
+BwdLayout bwd_layout(size_t bh, size_t nck, size_t wn, size_t seq, size_t n, size_t r) {
+    const size_t bhw = bh * wn, rec = bhw * kP * n * 4, pairs = bh * nck * (n / 2) * 4;
     BwdLayout l;
     size_t o = 0;
     l.s = o;      o = balign(o + rec);
     l.gh = o;     o = balign(o + rec);
-    l.eda = o;    o = balign(o + bhk * 4);
+    l.eda = o;    o = balign(o + bhw * 4);
     l.cin = o;    o = balign(o + bh * seq * (n / 2) * 4);
     l.ctot = o;   o = balign(o + pairs);
-    l.off = o;    o = balign(o + pairs);
     l.da = o;     o = balign(o + bh * seq * 4);
     l.dg = o;     o = balign(o + bh * seq * 4);
     l.dw = o;     o = balign(o + bh * seq * 4);
-    l.pd = o;     o = balign(o + bhk * 4);
-    l.pa = o;     o = balign(o + bhk * 4);
+    l.pd = o;     o = balign(o + bhw * 4);
+    l.pa = o;     o = balign(o + bhw * 4);
     l.pfirst = o; o = balign(o + bh * (n / 32) * 4);
     l.seed = o;   o = balign(o + bh * (n / 2) * 4);
     l.lux = o;    o = balign(o + bh * kP * r * 4);
@@ -94,8 +96,9 @@ BwdLayout bwd_layout(size_t bh, size_t nck, size_t seq, size_t n, size_t r) {
 
 struct BwdWs {
     float *s, *gh, *eda;
-    float *cin, *ctot, *off, *da, *dg, *dw, *pd, *pa, *pfirst;
+    float *cin, *ctot, *da, *dg, *dw, *pd, *pa, *pfirst;
     float *seed, *lux, *lub;
+    int k0, wn;   // the window: chunks k0 .. k0 + wn - 1 of each sequence
 };
 
 // element access in the storage type
@@ -519,9 +522,11 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             ps[u] = rot ? sm.asn[sb][u][(QT - 1) * AP + c] : 0.0f;
         }
     };
+    const uint32_t nw = static_cast<uint32_t>(min(w.wn, nck - w.k0));   // chunks in the window
     auto put_record = [&](float *base, int k, f32x4 lo, f32x4 hi) {
-        if (k >= nck) return;
-        float *o = base + (bh * nck + k) * kP * N + ((pt * NTN + i1) * 64 + lane) * 4;
+        const uint32_t kw = static_cast<uint32_t>(k - w.k0);
+        if (kw >= nw) return;
+        float *o = base + (bh * w.wn + kw) * kP * N + ((pt * NTN + i1) * 64 + lane) * 4;
         *reinterpret_cast<f32x4 *>(o) = lo;
         *reinterpret_cast<f32x4 *>(o + HT * 256) = hi;
     };
@@ -570,7 +575,8 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
                         lo = lo * e[u] + ulo[u];
                         hi = hi * e[u] + uhi[u];
                         if (rot && 2 * st + u < nck) rot4(lo, hi, pc[u], ps[u]);   // R(Phi_k)
-                        if (i1 == 0 && tid == 0 && 2 * st + u < nck) w.eda[bh * nck + 2 * st + u] = e[u];
+                        const uint32_t kw = static_cast<uint32_t>(2 * st + u - w.k0);
+                        if (i1 == 0 && tid == 0 && kw < nw) w.eda[bh * w.wn + kw] = e[u];
                     }
                     __syncthreads();
                 }
@@ -659,7 +665,7 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             rot4(lo, hi, cs, -sn);
         }
         float dfirst = 0.0f;
-        if (a.h0 != nullptr) {
+        if (a.h0 != nullptr && w.k0 + w.wn >= nck) {   // (the last window: every read of dh is done)
             if (g.dh0 != nullptr) st_state(g.dh0, lo, hi);
             if (a.last_u0 != nullptr) {
                 const size_t i0 = (bb * L) * H + hh;
@@ -671,7 +677,7 @@ __device__ void state_pass(const ScanLaunch &a, const BwdArgs &g, const BwdWs &w
             }
         }
         dfirst = block_sum(dfirst, sm.red);
-        if (tid == 0) w.pfirst[blk] = dfirst;
+        if (tid == 0) w.pfirst[blk] = dfirst;   // of the last window in the end
     }
 }
 
@@ -731,9 +737,10 @@ __global__ void __launch_bounds__(kBT, 4) bwd_chunk_kernel(ScanLaunch a, BwdArgs
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, gq = lane >> 4;
-    const size_t bhk = blockIdx.x;
-    const int ck = static_cast<int>(bhk % nck);
-    const size_t bh = bhk / nck;
+    const size_t bhw = blockIdx.x;   // the record
+    const int ck = w.k0 + static_cast<int>(bhw % w.wn);
+    const size_t bh = bhw / w.wn;
+    if (ck >= nck) return;           // the last window's end
     const size_t H = a.heads, L = a.seq;
     const size_t bb = bh / H, hh = bh % H;
     const bool rot = a.theta != nullptr;
@@ -785,8 +792,8 @@ __global__ void __launch_bounds__(kBT, 4) bwd_chunk_kernel(ScanLaunch a, BwdArgs
     static_assert(2 * PT * (2 / JR) == kWaves, "one job a wave");
     const bool isb = wave >= kWaves / 2;
     const int ji = wave % PT, rt0 = PT == 4 ? 0 : (wave / PT) & 1;
-    const size_t rec = bhk * kP * N;
-    const float eda = w.eda[bhk];
+    const size_t rec = bhw * kP * N;
+    const float eda = w.eda[bhw];
     f32x4 fl[4], fh[4];
     {
         const f32x4 *r4 = reinterpret_cast<const f32x4 *>((isb ? w.gh : w.s) + rec) + lane;
@@ -1158,7 +1165,7 @@ __global__ void __launch_bounds__(kBT, 4) bwd_chunk_kernel(ScanLaunch a, BwdArgs
         }
         if (tl == QT - 1) {
 #pragma unroll
-            for (int j = 0; j < PN; ++j) w.ctot[bhk * NH + i0 + j] = v[j];
+            for (int j = 0; j < PN; ++j) w.ctot[(bh * nck + ck) * NH + i0 + j] = v[j];
         }
     }
     // ---- per-token scalars (lane = row, then the row's token at lane t R)
@@ -1213,8 +1220,12 @@ __global__ void __launch_bounds__(kBT, 4) bwd_chunk_kernel(ScanLaunch a, BwdArgs
         float da = __shfl(d, (rt < 0 ? 0 : rt) * R, 64);
         da = seg_scan<32>(tl < QT ? da : 0.0f);
         if (lane == 0) {
-            w.pd[bhk] = ds;
-            w.pa[bhk] = pa;
+            if (w.k0 > 0) {
+                ds += w.pd[bhw];
+                pa += w.pa[bhw];
+            }
+            w.pd[bhw] = ds;
+            w.pa[bhw] = pa;
         }
         if (lane < QT && t0 + rt < L) w.da[bh * L + t0 + rt] = da;
         if (lane < kRows && tl % R == 0 && t0 + t < L) {
@@ -1232,7 +1243,7 @@ __global__ void bwd_angle_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
     const int i = threadIdx.x;
     if (i >= NH) return;
     float run = g.dangle_out ? g.dangle_out[bh * NH + i] : 0.0f;
-    // eight chunk totals in flight ahead of the running sum
+    // eight chunk totals in flight ahead of the running sum, which takes their place
     for (int k0 = nck - 1; k0 >= 0; k0 -= D) {
         float v[D];
 #pragma unroll
@@ -1240,7 +1251,7 @@ __global__ void bwd_angle_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             if (k0 - j < 0) break;
-            w.off[(bh * nck + k0 - j) * NH + i] = run;
+            w.ctot[(bh * nck + k0 - j) * NH + i] = run;
             run += v[j];
         }
     }
@@ -1296,7 +1307,7 @@ __global__ void __launch_bounds__(256) bwd_token_kernel(ScanLaunch a, BwdArgs g,
         cin[j] = live ? u : 0.0f;
         th[j] = live ? v : 0.0f;
     }
-    const float off = rot ? w.off[bhk * NH + pl] : 0.0f;
+    const float off = rot ? w.ctot[bhk * NH + pl] : 0.0f;   // the later chunks' sum
     float mine = 0.0f;   // lane j keeps token wave + 4 j's angle part
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
@@ -1329,17 +1340,17 @@ __global__ void __launch_bounds__(256) bwd_token_kernel(ScanLaunch a, BwdArgs g,
 }
 
 // ---------------------------------------------------------------- per head
-__global__ void __launch_bounds__(256) bwd_head_kernel(ScanLaunch a, BwdArgs g, BwdWs w, int nck) {
+__global__ void __launch_bounds__(256) bwd_head_kernel(ScanLaunch a, BwdArgs g, BwdWs w) {
     __shared__ float red[16];
     const size_t hh = blockIdx.x;
     const size_t H = a.heads;
     float sa = 0.0f, sd = 0.0f;
-    const size_t n = a.batch * static_cast<size_t>(nck);
+    const size_t n = a.batch * static_cast<size_t>(w.wn);
     for (size_t j = threadIdx.x; j < n; j += blockDim.x) {
-        const size_t bb = j / nck, k = j % nck;
-        const size_t bhk = (bb * H + hh) * nck + k;
-        sa += w.pa[bhk];
-        sd += w.pd[bhk];
+        const size_t bb = j / w.wn, k = j % w.wn;
+        const size_t bhw = (bb * H + hh) * w.wn + k;
+        sa += w.pa[bhw];
+        sd += w.pd[bhw];
     }
     sa = block_sum(sa, red);
     sd = block_sum(sd, red + 8);
@@ -1458,11 +1469,17 @@ hipError_t launched(int &launches) {
 }
 
 template <typename T, int N, int R>
-hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStream_t s, int &launches) {
+hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, size_t bytes, hipStream_t s,
+                      int &launches) {
     constexpr int QT = kRows / R;
     const int nck = static_cast<int>((a.seq + QT - 1) / QT);
     const size_t bh = a.batch * a.heads, bhk = bh * nck;
-    const BwdLayout l = bwd_layout(bh, nck, a.seq, N, R);
+    BwdLayout l = bwd_layout(bh, nck, nck, a.seq, N, R);
+    int wn = nck;
+    if (l.total > bytes) {   // two windows (scan_backward_workspace_least)
+        wn = (nck + 1) / 2;
+        l = bwd_layout(bh, nck, wn, a.seq, N, R);
+    }
     BwdWs w;
     auto f = [base](size_t off) { return reinterpret_cast<float *>(base + off); };
     w.s = f(l.s);
@@ -1470,7 +1487,6 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
     w.eda = f(l.eda);
     w.cin = f(l.cin);
     w.ctot = f(l.ctot);
-    w.off = f(l.off);
     w.da = f(l.da);
     w.dg = f(l.dg);
     w.dw = f(l.dw);
@@ -1480,6 +1496,8 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
     w.seed = f(l.seed);
     w.lux = f(l.lux);
     w.lub = f(l.lub);
+    w.k0 = 0;
+    w.wn = wn;
 
     static_assert(sizeof(Smem<N, R>) <= 80 * 1024, "two chunk workgroups a CU");
     const size_t lds = sizeof(Smem<N, R>);
@@ -1494,18 +1512,20 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
         if (a.theta != nullptr) gm.dangle_out = w.seed;
     }
     const BwdArgs &g2 = gm;
-    hipLaunchKernelGGL((bwd_passes_kernel<T, N, R>), dim3(2 * bh * (N / 32)), dim3(256), 0, s, a, g2, w,
-                       nck);
-    if ((e = launched(launches)) != hipSuccess) return e;
-    hipLaunchKernelGGL((bwd_chunk_kernel<T, N, R>), dim3(bhk), dim3(kBT), lds, s, a, g2, w, nck);
-    if ((e = launched(launches)) != hipSuccess) return e;
+    for (w.k0 = 0; w.k0 < nck; w.k0 += wn) {
+        hipLaunchKernelGGL((bwd_passes_kernel<T, N, R>), dim3(2 * bh * (N / 32)), dim3(256), 0, s, a, g2, w,
+                           nck);
+        if ((e = launched(launches)) != hipSuccess) return e;
+        hipLaunchKernelGGL((bwd_chunk_kernel<T, N, R>), dim3(bh * wn), dim3(kBT), lds, s, a, g2, w, nck);
+        if ((e = launched(launches)) != hipSuccess) return e;
+    }
     if (a.theta != nullptr) {
         hipLaunchKernelGGL((bwd_angle_kernel<N>), dim3(bh), dim3(64), 0, s, a, g2, w, nck);
         if ((e = launched(launches)) != hipSuccess) return e;
     }
     hipLaunchKernelGGL((bwd_token_kernel<T, N, R>), dim3(bhk), dim3(256), 0, s, a, g2, w, nck);
     if ((e = launched(launches)) != hipSuccess) return e;
-    hipLaunchKernelGGL(bwd_head_kernel, dim3(a.heads), dim3(256), 0, s, a, g2, w, nck);
+    hipLaunchKernelGGL(bwd_head_kernel, dim3(a.heads), dim3(256), 0, s, a, g2, w);
     if ((e = launched(launches)) != hipSuccess) return e;
     if (g.dlast_u_out != nullptr) {
         hipLaunchKernelGGL((bwd_last_add_kernel<T, N, R>), dim3(bh), dim3(256), 0, s, a, g, w);
@@ -1515,16 +1535,17 @@ hipError_t launch_bwd(const ScanLaunch &a, const BwdArgs &g, char *base, hipStre
 }
 
 template <typename T>
-hipError_t launch_bwd_t(const ScanLaunch &a, const BwdArgs &g, char *ws, hipStream_t s, int &launches) {
+hipError_t launch_bwd_t(const ScanLaunch &a, const BwdArgs &g, char *ws, size_t bytes, hipStream_t s,
+                        int &launches) {
     const size_t n = a.d_state, r = a.rank;
     if (n == 128) {
-        if (r == 1) return launch_bwd<T, 128, 1>(a, g, ws, s, launches);
-        if (r == 2) return launch_bwd<T, 128, 2>(a, g, ws, s, launches);
-        if (r == 4) return launch_bwd<T, 128, 4>(a, g, ws, s, launches);
+        if (r == 1) return launch_bwd<T, 128, 1>(a, g, ws, bytes, s, launches);
+        if (r == 2) return launch_bwd<T, 128, 2>(a, g, ws, bytes, s, launches);
+        if (r == 4) return launch_bwd<T, 128, 4>(a, g, ws, bytes, s, launches);
     } else if (n == 64) {
-        if (r == 1) return launch_bwd<T, 64, 1>(a, g, ws, s, launches);
-        if (r == 2) return launch_bwd<T, 64, 2>(a, g, ws, s, launches);
-        if (r == 4) return launch_bwd<T, 64, 4>(a, g, ws, s, launches);
+        if (r == 1) return launch_bwd<T, 64, 1>(a, g, ws, bytes, s, launches);
+        if (r == 2) return launch_bwd<T, 64, 2>(a, g, ws, bytes, s, launches);
+        if (r == 4) return launch_bwd<T, 64, 4>(a, g, ws, bytes, s, launches);
     }
     return hipErrorNotSupported;
 }
@@ -1539,12 +1560,23 @@ size_t scan_backward_workspace(const ScanLaunch &a) {
     if (!scan_backward_supported(a)) return 0;
     const size_t qt = kRows / a.rank;
     const size_t nck = (a.seq + qt - 1) / qt;
-    return bwd_layout(a.batch * a.heads, nck, a.seq, a.d_state, a.rank).total;
+    return bwd_layout(a.batch * a.heads, nck, nck, a.seq, a.d_state, a.rank).total;
 }
 
-hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *workspace,
+// bf16 storage at d_state 64 took 64-row chunks once, and half the records;
+// their workspace still runs, in two windows.  Batch 12 x 1024, 24 heads, us:
+// 64-row chunks 790 in 194 MB, 32-row ones 479 in 345 MB, in two windows 592 in
+// 194; 2 x 512, 4 heads 73.5, 42.8 and 73.5.
+size_t scan_backward_workspace_least(const ScanLaunch &a) {
+    if (!scan_backward_supported(a)) return 0;
+    const size_t qt = kRows / a.rank;
+    const size_t nck = (a.seq + qt - 1) / qt, wn = a.bf16 && a.d_state == 64 ? (nck + 1) / 2 : nck;
+    return bwd_layout(a.batch * a.heads, nck, wn, a.seq, a.d_state, a.rank).total;
+}
+
+hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *workspace, size_t bytes,
                                 hipStream_t stream, int &launches) {
-    if (!scan_backward_supported(a)) return hipErrorNotSupported;
+    if (!scan_backward_supported(a) || bytes < scan_backward_workspace_least(a)) return hipErrorNotSupported;
     BwdArgs g;
     g.dy = gr.dy;
     g.dh_out = gr.dh_out;
@@ -1563,8 +1595,8 @@ hipError_t launch_scan_backward(const ScanLaunch &a, const ScanGrads &gr, void *
     g.dangle0 = gr.dangle0;
     g.add_sums = gr.add_sums != 0;
     char *ws = static_cast<char *>(workspace);
-    if (a.bf16) return launch_bwd_t<bf16_t>(a, g, ws, stream, launches);
-    return launch_bwd_t<float>(a, g, ws, stream, launches);
+    if (a.bf16) return launch_bwd_t<bf16_t>(a, g, ws, bytes, stream, launches);
+    return launch_bwd_t<float>(a, g, ws, bytes, stream, launches);
 }
 
 }  // namespace m3

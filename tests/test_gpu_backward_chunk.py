@@ -46,6 +46,61 @@ def test_gradients_repeat_bit_for_bit(N, R):
         assert torch.equal(getattr(a, k), getattr(b, k)), k
 
 
+def _former_bytes(BH, T, N, R):
+    """The workspace of 64-row chunks, which bf16 storage at d_state 64 had."""
+    up = lambda v: (v + 255) // 256 * 256
+    nck = -(-T // (64 // R))
+    pairs, tok = BH * nck * (N // 2) * 4, BH * T * 4
+    return (2 * up(BH * nck * 64 * N * 4) + 3 * up(BH * nck * 4) + up(BH * T * (N // 2) * 4) + 2 * up(pairs)
+            + 3 * up(tok) + up(BH * (N // 32) * 4) + up(BH * (N // 2) * 4) + up(BH * 64 * R * 4)
+            + up(BH * N * R * 4))
+
+
+@pytest.mark.parametrize("B,T,H,R", [(1, 1, 1, 1), (1, 33, 1, 1), (2, 64, 3, 1), (5, 65, 13, 1), (1, 1000, 2, 1),
+                                     (2, 150, 3, 2), (3, 40, 5, 4)])
+def test_a_workspace_of_64_row_chunks_still_runs(B, T, H, R):
+    """Half the records: the chunks in two windows, the same gradients (those
+    summed over chunks to f32 rounding); a byte less than the least is refused."""
+    import ctypes as C
+    from mamba3 import _lib
+    L = _lib.lib()
+    P = N = 64
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(s, device="cuda", generator=g)
+    bf = lambda t: t.bfloat16()
+    x, b, c, th = bf(r(B, T, H, P, R)), bf(r(B, T, H, N, R) / 8), bf(r(B, T, H, N, R) / 8), bf(r(B, T, H, N // 2))
+    dt, lam, a_log, skip = r(B, T, H).abs() * 0.05, torch.sigmoid(r(B, T, H)), r(H).abs(), r(H)
+    st = (r(B, H, P, N), r(B, H, P, N), r(B, H, N // 2))
+    dy, dh, dang, dlu = bf(r(B, T, H, P, R)), r(B, H, P, N), r(B, H, N // 2), r(B, H, P, N)
+    st_c = _lib.SsmStateC(*[t.data_ptr() for t in st])
+
+    def call(size):
+        ins = _lib.ScanInputsC(B, T, H, P, N, R, _lib.M3_BF16, *[t.data_ptr() for t in (x, b, c, dt, a_log, lam, th,
+                               skip)], C.pointer(st_c), 64, 0, None, 0)
+        full = int(L.m3_scan_backward_workspace_bytes(C.byref(ins)))
+        ws = torch.full((max(full, size or 0),), 255, dtype=torch.uint8, device="cuda")   # NaN wherever unwritten
+        ins.workspace, ins.workspace_bytes = ws.data_ptr(), size or full
+        out = [torch.full_like(t, float("nan")) for t in (x, b, c, dt, lam, a_log, th, skip, *st)]
+        gc = _lib.ScanGradsC(dy.data_ptr(), dh.data_ptr(), dang.data_ptr(), *[t.data_ptr() for t in out], dlu.data_ptr())
+        n = L.m3_launch_count()
+        status = L.m3_scan_backward(C.byref(ins), C.byref(gc), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return status, out, L.m3_launch_count() - n, full
+
+    former = _former_bytes(B * H, T, N, R)
+    ok, whole, n, full = call(None)
+    ok2, two, n2, _ = call(former)
+    assert ok == ok2 == _lib.M3_OK
+    assert n2 == (n + 2 if former < full else n) and (former < full or T <= 32 // R)
+    for i, (e, t) in enumerate(zip(whole, two)):
+        if i in (5, 7):   # a_log, d_skip
+            assert rel_l2(host(t), host(e)) <= F32_TOL, i
+        else:
+            assert torch.equal(t, e), i
+    if T > 32 // R:
+        assert call(former // 2)[0] == _lib.M3_ERR_ARGUMENT
+
+
 def test_dy_off_the_dword_grid():
     """A bf16 dy that starts two bytes past a 4-byte boundary gives the same bytes."""
     def shifted(t):
