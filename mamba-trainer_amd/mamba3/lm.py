@@ -155,8 +155,8 @@ class DecodeGraph:
 
     def __init__(self, lm: Mamba3Lm, cache: List[MixerCache], batch: int):
         dev = cache[0].ssm.h.device
-        # int32, as the embedding reads them: the copy into it converts
-        self.ids = torch.zeros((batch, 1), dtype=torch.int32, device=dev)
+        # torch's own index type, so that a caller's argmax may write it in place
+        self.ids = torch.zeros((batch, 1), dtype=torch.int64, device=dev)
         scratch = [c.clone() for c in cache]
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))

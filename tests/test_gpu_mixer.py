@@ -584,6 +584,29 @@ def test_decode_graph_replays_match_eager_steps(conv, factored):
     assert torch.isfinite(got.float()).all()
 
 
+def test_decode_graph_ids_take_an_argmax_in_place():
+    """A caller's loop may write the next ids straight into the graph's buffer
+    (int64, as torch's argmax gives them) and replay: the greedy tokens of step()."""
+    rng = np.random.default_rng(63)
+    model = mo.random_model(rng, vocab=64, d_model=64, n_layers=2, heads=4, head_dim=16, d_state=16,
+                            int8=True, bias_scale=0.3)
+    lm = gpu_lm_from_oracle(model, True)
+    B = 3
+    first = torch.arange(B, device=DEV).view(B, 1)
+    graphs = [lm.capture_decode(lm.empty_cache(B, DEV), B) for _ in range(2)]
+    ids, want, got = first, [], []
+    for _ in range(4):
+        ids = graphs[0].step(ids).view(B, -1).argmax(-1, keepdim=True)
+        want.append(ids.clone())
+    graphs[1].ids.copy_(first)
+    for _ in range(4):
+        graphs[1].graph.replay()
+        torch.argmax(graphs[1].logits.view(B, -1), -1, keepdim=True, out=graphs[1].ids)
+        got.append(graphs[1].ids.clone())
+    torch.cuda.synchronize()
+    assert torch.equal(torch.cat(want), torch.cat(got))
+
+
 def _default_mixer_and_layer(rng):
     """A Mamba3Mixer of the reference's default SsmConfig (config.rs:131-156:
     d_model 768, 24 heads x 64, d_state 64, 24 groups, conv_kernel 4, bc_norm,
