@@ -18,7 +18,7 @@ import torch
 
 from .error import ShapeError, UnsupportedError
 from .mixer import Mamba3Mixer, MixerCache
-from .nn import Embedding, Linear, RmsNorm, normal, tensor_param
+from .nn import Embedding, Linear, RmsNorm, as_written, linear_normed, normal, tensor_param
 from .ssm import SsmConfig
 
 
@@ -125,8 +125,13 @@ class Mamba3Lm:
         x = self.embed.lookup(ids)
         if ids.shape[1] == 1:
             for (norm, mixer), c in zip(self.layers, cache):
-                mixer.step_normed_(x, norm, c, residual=x, out=x)
-            return self.head.apply_normed(x, self.norm_f)
+                if as_written(mixer, Mamba3Mixer, "step_"):
+                    mixer.step_normed_(x, norm, c, residual=x, out=x)
+                else:
+                    mixer.step_(norm.apply(x), c, residual=x, out=x)
+            if as_written(self, Mamba3Lm, "logits_from"):
+                return linear_normed(self.head, x, self.norm_f)
+            return self.logits_from(self.norm_f.apply(x))
         normed = torch.empty_like(x)
         for i, (norm, mixer) in enumerate(self.layers):
             norm.apply(x, out=normed)

@@ -21,7 +21,8 @@ import torch
 
 from . import _lib
 from .error import ShapeError, UnsupportedError
-from .nn import Linear, RmsNorm, _bf16_dev, _stream, normal, residual_scaled, tensor_param
+from .nn import (Linear, RmsNorm, _bf16_dev, _stream, linear_normed, normal, residual_scaled,
+                 tensor_param)
 from .ssm import (ScanInputs, SsmConfig, SsmState, SsmStateFactored, StateDynamics, mamba3_scan,
                   mamba3_scan_gated,
                   mamba3_step_, mamba3_step_factored_)
@@ -340,7 +341,7 @@ class Mamba3Mixer:
         dims = self._dims(B)
         input = _bf16_dev(input, "mixer input")
         projected = (self.in_proj.apply(input) if norm is None
-                     else self.in_proj.apply_normed(input, norm))
+                     else linear_normed(self.in_proj, input, norm))
         gated = torch.empty((B, 1, c.d_inner()), dtype=torch.bfloat16, device=input.device)
         ptr = lambda t: None if t is None else t.data_ptr()
         ang = ptr(st.angle) if rot else None

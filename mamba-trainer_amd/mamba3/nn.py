@@ -27,6 +27,12 @@ def _bf16_dev(t: torch.Tensor, what: str) -> torch.Tensor:
     return t.contiguous()
 
 
+def as_written(obj, cls, name: str) -> bool:
+    """Whether obj.<name> is the method of cls itself, which a call past it may
+    stand for: no subclass's, none set on the object, no other object's."""
+    return getattr(type(obj), name, None) is getattr(cls, name) and name not in vars(obj)
+
+
 def normal(shape, std: float, device, gen: torch.Generator) -> torch.Tensor:
     """Initializer::Normal {mean 0, std} (init.rs:98-100)."""
     return torch.randn(shape, device=device, generator=gen, dtype=torch.float32) * std
@@ -170,7 +176,8 @@ class Linear:
         row's factor instead of after it; elsewhere as two calls."""
         x = _bf16_dev(x, "Linear input")
         m = x.numel() // max(x.shape[-1], 1)
-        if m <= 4 and x.shape[-1] == self.in_features == norm.dim:
+        if (m <= 4 and as_written(self, Linear, "apply") and as_written(norm, RmsNorm, "apply")
+                and x.shape[-1] == self.in_features == norm.dim):
             y = torch.empty(tuple(x.shape[:-1]) + (self.out_features,), dtype=torch.bfloat16,
                             device=x.device)
             st = _lib.lib().m3_norm_linear_nt(
@@ -182,6 +189,13 @@ class Linear:
                 _lib.check(st)
                 return y
         return self.apply(norm.apply(x))
+
+
+def linear_normed(linear, x: torch.Tensor, norm) -> torch.Tensor:
+    """linear.apply(norm.apply(x)), in one launch where `linear` is a Linear."""
+    if isinstance(linear, Linear):
+        return linear.apply_normed(x, norm)
+    return linear.apply(norm.apply(x))
 
 
 class Embedding:

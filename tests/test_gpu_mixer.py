@@ -584,6 +584,63 @@ def test_decode_graph_replays_match_eager_steps(conv, factored):
     assert torch.isfinite(got.float()).all()
 
 
+def test_cached_token_runs_what_the_caller_put_in_place():
+    """forward_cached of one token calls a subclass's logits_from and step_, a
+    projection or norm that is not the library's, and a method set on one that
+    is: none of them is passed by for the fused norm and product."""
+    from mamba3.lm import Mamba3Lm
+    from mamba3.mixer import Mamba3Mixer
+    rng = np.random.default_rng(64)
+    model = mo.random_model(rng, vocab=64, d_model=64, n_layers=2, heads=4, head_dim=16, d_state=16,
+                            int8=True, bias_scale=0.3)
+    ids = torch.tensor([[3]], device=DEV)
+    calls = []
+
+    class Wrap:
+        def __init__(self, inner, name):
+            self.inner, self.name = inner, name
+
+        def apply(self, *a, **k):
+            calls.append(self.name)
+            return self.inner.apply(*a, **k)
+
+        def __getattr__(self, k):
+            return getattr(self.inner, k)
+
+    class OwnLm(Mamba3Lm):
+        def logits_from(self, hidden):
+            calls.append("logits_from")
+            return super().logits_from(hidden)
+
+    class OwnMixer(Mamba3Mixer):
+        def step_(self, *a, **k):
+            calls.append("step_")
+            return super().step_(*a, **k)
+
+    def run(change):
+        lm = gpu_lm_from_oracle(model, True)
+        change(lm)
+        calls.clear()
+        return lm.forward_cached(ids, lm.empty_cache(1, DEV)).clone(), list(calls)
+
+    def set_apply(lm):
+        plain = lm.norm_f.apply
+        lm.norm_f.apply = lambda x, **k: (calls.append("set"), plain(x, **k))[1]
+
+    ref, _ = run(lambda lm: None)
+    for change, want in [
+            (lambda lm: setattr(lm, "__class__", OwnLm), ["logits_from"]),
+            (lambda lm: setattr(lm.layers[1][1], "__class__", OwnMixer), ["step_"]),
+            (lambda lm: setattr(lm, "head", Wrap(lm.head, "head")), ["head"]),
+            (lambda lm: setattr(lm.layers[0][1], "in_proj", Wrap(lm.layers[0][1].in_proj, "in")), ["in"]),
+            (lambda lm: lm.layers.__setitem__(0, (Wrap(lm.layers[0][0], "norm"), lm.layers[0][1])), ["norm"]),
+            (set_apply, ["set"])]:
+        got, seen = run(change)
+        assert seen == want, (seen, want)
+        # the norm's output rounded to bf16, or its operand: as many roundings
+        assert rel_l2(host(got), host(ref)) <= 3e-2, want
+
+
 def test_decode_graph_ids_take_an_argmax_in_place():
     """A caller's loop may write the next ids straight into the graph's buffer
     (int64, as torch's argmax gives them) and replay: the greedy tokens of step()."""
