@@ -97,8 +97,10 @@ m3_status m3_linear_nt(size_t m, size_t k, size_t n, const void *x, const void *
  * stack (src/models/hybrid.rs:446-456) for the rows of a decode step.  The
  * operand is bf16(x * gain) and the row's factor multiplies the f32 sums, so
  * one rounding to bf16 stands where m3_rms_norm's output has one.  Up to 4
- * rows, k a multiple of 64, n of 4, 16-byte aligned buffers; anything else is
- * M3_ERR_UNSUPPORTED before any device work. */
+ * rows whose operands fit 50 KB together (m (2 k + 16) bytes: k to 6336 for
+ * four, 8512 for three, 12736 for two, 25536 for one), k a multiple of 64, n
+ * of 4 and at least 16, a weight under 2 GiB, 16-byte aligned buffers (residual
+ * and y 8); anything else is M3_ERR_UNSUPPORTED before any device work. */
 m3_status m3_norm_linear_nt(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,
                             const void *w_t, const float *col_scale, const void *residual, void *y,
                             void *stream);

@@ -104,8 +104,9 @@ m3_status m3_norm_linear_nt(size_t m, size_t k, size_t n, const void *x, const f
     if (x == nullptr || w_t == nullptr || y == nullptr)
         return m3::api_fail(M3_ERR_ARGUMENT, "linear buffers are NULL");
     if (!m3::norm_few_rows_supported(m, k, n, x, gain, w_t, col_scale, residual, y))
-        return m3::api_fail(M3_ERR_UNSUPPORTED, "the normed product covers up to 4 rows, k a "
-                            "multiple of 64, n of 4 and 16-byte aligned buffers (got %zu, %zu, %zu)",
+        return m3::api_fail(M3_ERR_UNSUPPORTED, "the normed product covers up to 4 rows with "
+                            "m (2 k + 16) <= 51200, k a multiple of 64, n of 4 and at least 16, a "
+                            "weight under 2 GiB and 16-byte aligned buffers (got %zu, %zu, %zu)",
                             m, k, n);
     return launched(m3::launch_norm_few_rows(m, k, n, x, gain, eps, w_t, col_scale, residual, y,
                                              as_stream(stream)),

@@ -15,7 +15,7 @@ import torch
 import mixer_oracle as mo
 from test_gpu_mixer import host, t_bf16, t_f32
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
 CASES = [
     # m, k, n, int8, residual
@@ -27,6 +27,7 @@ CASES = [
 ]
 
 
+@gpu
 @pytest.mark.parametrize("m,k,n,int8,resid", CASES)
 def test_few_rows_against_f64(m, k, n, int8, resid):
     from mamba3.nn import Linear
@@ -54,6 +55,7 @@ def test_few_rows_against_f64(m, k, n, int8, resid):
     assert torch.all(buf[m] == 7.0)
 
 
+@gpu
 def test_few_rows_repeat_bit_for_bit():
     from mamba3.nn import Linear
     rng = np.random.default_rng(2)
@@ -65,6 +67,7 @@ def test_few_rows_repeat_bit_for_bit():
     assert torch.equal(lin.apply(x[2:5].contiguous())[1], lin.apply(x[3:4].contiguous())[0])
 
 
+@gpu
 @pytest.mark.parametrize("m,k,n,int8,gain", [(1, 64, 16, True, True), (1, 1536, 1540, True, True),
                                              (4, 768, 5400, True, False), (3, 320, 4100, False, True),
                                              (4, 2560, 516, True, True), (2, 512, 1000, True, True)])
@@ -105,6 +108,43 @@ def test_normed_few_rows_against_f64(m, k, n, int8, gain):
     assert err(got) <= 1.2 * err(two) + 1e-4
 
 
+@gpu
+@pytest.mark.parametrize("m,k", [(1, 25536), (2, 12736), (3, 8512), (4, 6336)])
+def test_normed_rows_at_the_edge_of_their_lds(m, k):
+    """The largest k whose m operand rows fit, against f64 in one launch, and
+    64 more, which runs as the two calls, equal to them."""
+    from mamba3 import _lib
+    from mamba3.nn import Linear, RmsNorm
+    rng = np.random.default_rng(k)
+    n = 20
+    for kk, launches in ((k, 1), (k + 64, 2)):
+        w = rng.normal(0, 0.02, (kk, n)).astype(np.float32)
+        lin, norm = Linear(t_f32(w)), RmsNorm(kk, torch.device("cuda"))
+        x = mo.bf16(rng.normal(0, 1, (m, kk)))
+        xt = t_bf16(x)
+        before = _lib.lib().m3_launch_count()
+        y = lin.apply_normed(xt, norm)
+        assert _lib.lib().m3_launch_count() - before == launches
+        two = lin.apply(norm.apply(xt))
+        if launches == 2:
+            assert torch.equal(y, two)
+        normed, w_eff = mo.rms_norm(x, np.ones(kk, np.float32), 1e-5), mo.bf16(w)
+        ref = normed @ w_eff
+        bound = 2.0 ** -8 * np.abs(ref) + (2.0 ** -9 + (kk + 4) * 2.0 ** -24) * (np.abs(normed) @ np.abs(w_eff))
+        assert np.all(np.abs(host(y) - ref) <= bound)
+
+
+def test_normed_product_refuses_before_device_work():
+    """Past each limit M3_ERR_UNSUPPORTED, from the shapes alone."""
+    from mamba3 import _lib
+    L = _lib.lib()
+    for m, k, n in [(5, 64, 16), (4, 6400, 16), (1, 96, 16), (1, 64, 12), (1, 64, 18), (1, 16384, 1 << 16)]:
+        st = L.m3_norm_linear_nt(m, k, n, 4096, 4096, 1e-5, 4096, 4096, None, 4096, None)
+        assert st == _lib.M3_ERR_UNSUPPORTED, (m, k, n)
+        assert b"normed product covers" in L.m3_last_error()
+
+
+@gpu
 def test_normed_rows_past_the_kernel_run_as_two_calls():
     from mamba3 import _lib
     from mamba3.nn import Linear, RmsNorm
