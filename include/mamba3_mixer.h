@@ -85,9 +85,9 @@ m3_status m3_linear(size_t m, size_t k, size_t n, const void *x, const void *w,
  * at large m; a caller that holds the weight only for the product (the
  * int8 codes) keeps it this way.  Up to 512 rows and 4096 columns (k a
  * multiple of 128, n of 8, 16-byte aligned buffers) both forms run on the
- * library's own few-row kernel instead of hipBLASLt; this one also up to 16
- * rows at any width, and up to 64 where it is faster (k a multiple of 64, n
- * of 4). */
+ * library's own few-row kernel instead of hipBLASLt; this one also up to 32
+ * rows under 4096 columns and, where that is the faster route, up to 64 from
+ * there on (k a multiple of 64, n of 4). */
 m3_status m3_linear_nt(size_t m, size_t k, size_t n, const void *x, const void *w_t,
                        const float *col_scale, const void *residual, void *y, void *workspace,
                        size_t workspace_bytes, void *stream);

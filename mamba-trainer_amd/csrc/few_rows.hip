@@ -220,25 +220,46 @@ size_t x_reads(size_t m, size_t k, size_t n) { return (n + 31) / 32 * m * k * 2;
 
 }  // namespace
 
-// Where the lines lie (us per call, this kernel against the other route):
-// - to 16 rows it is the faster one at every size (above).
-// - 17 to 32 rows, under 4096 columns: 1536 x 1536 5.8 against 7.6 (17 rows),
-//   6.6 against 7.6 (32); 768 x 768 4.4 against 4.9 (32).  At 48 rows 8.6
-//   against 7.7 and 5.4 against 4.9: x's re-reads by every column tile take
-//   over, and skinny_gemm.hip's tiles hold more rows.
-// - from 4096 columns on, x's re-reads bound it: 768 x 5400 (8 MB of them at
-//   32 rows, 17 at 64) 5.8 against 7.2 and 7.4 against 7.7, 768 x 6192 (19 MB
-//   at 64) 7.6 against 7.8; 1536 x 10800 (33 MB at 32 rows) 15.7 against 13.5.
-bool few_rows_supported(size_t m, size_t k, size_t n, const void *x, const void *w, bool w_transposed,
-                        const float *scale, const void *res, const void *y) {
+// What the kernel takes.
+static bool fits(size_t m, size_t k, size_t n, const void *x, const void *w, bool w_transposed,
+                 const float *scale, const void *res, const void *y) {
     auto al = [](const void *p, uintptr_t b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
     if (!w_transposed || m < 1 || k < 64 || k % 64 != 0 || n < 16 || n % 4 != 0) return false;
     if (k * n * 2 >= (size_t(1) << 31) || !al(x, 16) || !al(w, 16) || !al(scale, 16) || !al(res, 8) ||
         !al(y, 8))
         return false;
-    if (m <= 16) return true;
+    return true;
+}
+
+// Where the lines lie (us per call, hipBLASLt's plan of its own probe / this
+// kernel; K x N).  Under 4096 columns, against skinny_gemm.hip, it is the faster
+// one to 32 rows at every size: 16384 x 1024 54 / 20 (1 row), 1536 x 1536 7.3 / 6.5 (32),
+// 3072 x 768 12.1 / 10.5 (32), 4096 x 4088 16.4 / 13.7 (32); at 48 rows 8.6 against 7.7
+// the other way round: x's re-reads by every column tile take over.  From 4096 columns
+// on hipBLASLt splits a long K where the columns leave CUs idle, and has tiles
+// of 32 and 64 rows:
+// - to 4 rows: 2048 x 4096 6.4 / 6.0, 2816 x 6144 10.7 / 10.2, 4096 x 12288 24.0 / 20.8; but
+//   3072 x 6144 9.4 / 10.3, 4096 x 4608 9.9 / 12.8, 8192 x 8192 27.8 / 29.1; 64 x 65536, one
+//   block of K for four waves, 5.5 / 6.3.
+// - to 16: 1536 x 4608 and up to 1536 x 16384 11.1 / 10.7 (16 rows), any K to 4096 x 32000
+//   56.1 / 55.0; but 2048 x 12288 12.3 / 14.0, 3072 x 10240 13.4 / 18.6, 8192 x 4608 19.8 /
+//   24.8; at 4096 columns, half the CUs, 1024 6.4 / 5.4, 1536 5.9 / 6.3, 3072 7.7 / 10.6.
+// - to 32: 2048 x 4608 11.7 / 9.8 (28), 1024 x 12288 10.4 / 9.5 (24), 512 x 32000 11.3 / 10.7
+//   (20); but at exactly 32 2048 x 4608 9.1 / 10.2, 1536 x 4608 7.6 / 8.0; 1536 x 10800 11.7 /
+//   12.8 (20), 3072 x 4608 11.2 / 12.2 (20), 256 x 32000 6.9 / 7.9 (28).
+// - to 64, while each of its workgroups has a CU (8192 columns): 768 x 5400 10.0 / 6.7
+//   (48) and 7.6 / 7.2 (64), 512 x 8192 8.1 / 6.0 (64); but 1024 x 4608 8.4 / 8.6 (64), 256 x
+//   16384 6.6 / 7.9, 256 x 32000 7.4 / 11.9 (33).
+bool few_rows_supported(size_t m, size_t k, size_t n, const void *x, const void *w, bool w_transposed,
+                        const float *scale, const void *res, const void *y) {
+    if (!fits(m, k, n, x, w, w_transposed, scale, res, y)) return false;
     if (n < 4096) return m <= 32;
-    return m <= 64 && x_reads(m, k, n) <= (size_t(20) << 20);
+    if (m <= 4) return (k <= 2816 || (n > 8192 && k <= 4096)) && (k >= 128 || n <= 32768);
+    if (m <= 16) return k <= (n > 16384 ? 4096 : n >= 4608 ? 1536 : 1024);
+    if (x_reads(m, k, n) > (size_t(20) << 20)) return false;
+    if (m <= 32)
+        return k <= (n >= 4608 && n <= 8192 && m < 32 ? 2048 : 1024) && (n <= 16384 || k >= 512);
+    return m <= 64 && n <= 8192 && m * k <= 57344;
 }
 
 hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const void *w,
@@ -263,10 +284,12 @@ hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const vo
 
 bool norm_few_rows_supported(size_t m, size_t k, size_t n, const void *x, const float *gain,
                              const void *w, const float *scale, const void *res, const void *y) {
-    // (the rows' copies in LDS, beside the partial sums)
+    // (the rows' copies in LDS, beside the partial sums).  With the norm's launch
+    // and row in it this is the faster form at any K and N: 4096 x 4608 18.5 / 12.8 us
+    // (1 row), 4096 x 12288 33.9 / 22.7 (4), 64 x 32000 6.5 / 5.9.
     return m <= kNormRows && m * (2 * k + 16) <= (size_t(50) << 10) &&
            reinterpret_cast<uintptr_t>(gain) % 16 == 0 &&
-           few_rows_supported(m, k, n, x, w, true, scale, res, y);
+           fits(m, k, n, x, w, true, scale, res, y);
 }
 
 hipError_t launch_norm_few_rows(size_t m, size_t k, size_t n, const void *x, const float *gain, float eps,

@@ -15,9 +15,9 @@
 //
 // Up to 512 rows and 4096 columns (K a multiple of 128, N of 8, 16-byte
 // aligned buffers) the product runs on the weight-streaming kernel of
-// skinny_gemm.hip instead, with the same epilogue; up to 16 rows, and up to 64
-// where few_rows_supported says, on the one of few_rows.hip (a transposed
-// weight, K a multiple of 64, N of 4).
+// skinny_gemm.hip instead, with the same epilogue; up to 64 rows, where
+// few_rows_supported says, on the one of few_rows.hip (a transposed weight, K a
+// multiple of 64, N of 4).
 //
 // Plan choice follows the reference's tuned plans (tensor/matmul.rs:1636-1943:
 // timing probes once per shape): the first call for a shape asks hipBLASLt's

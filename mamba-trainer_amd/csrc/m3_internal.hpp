@@ -243,7 +243,7 @@ hipError_t launch_skinny_gemm(size_t m, size_t k, size_t n, const void *x, const
                               bool w_transposed, const float *scale, const void *res, void *y,
                               hipStream_t s);
 // The product of a handful of rows with a transposed weight (few_rows.hip):
-// up to 16 rows, and up to 64 where it is the faster kernel.
+// up to 64 rows, where it is the faster route.
 bool few_rows_supported(size_t m, size_t k, size_t n, const void *x, const void *w, bool w_transposed,
                         const float *scale, const void *res, const void *y);
 hipError_t launch_few_rows(size_t m, size_t k, size_t n, const void *x, const void *w,

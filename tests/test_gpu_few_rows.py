@@ -24,6 +24,11 @@ CASES = [
     (16, 320, 300, True, True), (17, 1024, 516, True, True), (31, 768, 768, False, False),
     (32, 512, 4092, True, True), (32, 512, 4640, True, True), (33, 768, 5400, True, False),
     (64, 768, 4100, True, True), (49, 64, 6192, False, True),
+    # both sides of the lines from 4096 columns on
+    (4, 2816, 4096, True, True), (4, 2880, 4096, True, True), (1, 64, 32772, True, False),
+    (16, 1024, 4096, True, True), (16, 1088, 4096, True, True), (5, 1536, 4608, True, False),
+    (31, 2048, 4608, True, True), (32, 2048, 4608, True, True), (17, 448, 16388, True, False),
+    (33, 64, 8192, True, True), (33, 64, 8196, True, True),
 ]
 
 
