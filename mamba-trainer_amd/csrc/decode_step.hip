@@ -350,7 +350,11 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
     const int rows_per_wave = 64 / G;
     const int rows_per_pass = rows_per_wave * (NT / 64);
     const int col4 = (lane % G) * 4;
-    const float dskip = a.d_skip ? a.d_skip[bh % a.heads] : 0.0f;
+    // before the prologue where that is long enough to hide it (the step of 256
+    // threads without the mixer's: 5.12 us after it, 5.34 before, heads of 16)
+    constexpr bool kSkipFirst = EARLY || MIX;
+    float dskip = 0.0f;
+    auto load_skip = [&] { dskip = a.d_skip ? a.d_skip[bh % a.heads] : 0.0f; };
     f32x4 *h4 = reinterpret_cast<f32x4 *>(a.h + bh * P * N);
     f32x4 *u4 = reinterpret_cast<f32x4 *>(a.last_u + bh * P * N);
     constexpr int kBatch = NT > kStepThreads ? 2 : 4;   // rows in flight per lane
@@ -384,6 +388,7 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
                 }
         }
     };
+    if constexpr (kSkipFirst) load_skip();
     if constexpr (EARLY) {
         load_rows(base0);
         load_z(base0);
@@ -418,6 +423,7 @@ __device__ __forceinline__ void step_body_vec(const StepLaunch &a, size_t bh,
         }
     }
 
+    if constexpr (!kSkipFirst) load_skip();
     // B~ columns this lane touches, hoisted out of the row loop.
     float bcol[4][R], ccol[4][R], pcol[4][FACT ? R : 1];
 #pragma unroll
@@ -583,29 +589,43 @@ step_kernel_generic(StepLaunch a) {
 
 // The form of a launch of (batch, head) workgroups.  Measured on MI355X
 // (head_dim 64, us per layer, captured, caches from HBM; workgroups: 256
-// threads / the form taken).  A grid of at most one workgroup per CU is the
-// chain of its memory round trips, which kWide shortens (all loads first, two
-// rows a lane); to three per CU that still holds for kEarly; past it the
-// occupancy that the early loads cost counts for more, except for the fused
+// threads / the form taken, in brackets one not taken).  A grid of at most one
+// workgroup per CU is the chain of its memory round trips, which kWide shortens
+// (all loads first, two rows a lane); to three per CU, or the two that the
+// convolution's registers leave room for, that still holds for kEarly; past it
+// the occupancy that the early loads cost counts for more, except for the fused
 // mixer step, whose prologue is the longest.
-//   mixer step, d_state 128:  24 9.95 / 5.63, 240 11.8 / 7.6 (kWide); 384 15.5 /
-//     13.1, 768 22.3 / 19.9, 1536 39.7 / 36.2, 6144 145.5 / 135.7 (kEarly); with
-//     the convolution 24 10.9 / 6.6, 6144 146 / 143 (kHalf; kEarly 147)
-//   mixer step, factored:     24 9.9 / 6.6, 768 15.9 / 13.4, 1536 23.5 / (24.0)
+//   mixer step, d_state 128:  24 9.1 / 5.9, 240 11.9 / 7.8 (kWide); 384 15.5 /
+//     13.4, 768 22.4 / 20.1, 1024 28.4 / 27.4, 1536 40.1 / 36.9, 6144 143 / 135
+//     (kEarly); with the convolution 24 11.1 / 6.9, 512 18.4 / 16.5, 640 21.6 / (kEarly
+//     22.8), 768 23.9 / (24.5), 1024 30.3 / (kHalf 33.1), 3072 78.5 / 77.1, 6144 147 /
+//     142 (kHalf; kEarly 146)
+//   mixer step, d_state 64:   24 6.4 / 4.9, 240 7.8 / 5.9, 512 10.1 / 8.1, 768 12.2 / 10.2
+//     (kEarly), 1024 15.6 / (kEarly 15.2, kHalf 18.0), 1536 21.8 / (20.3, 22.1), 3072
+//     40.1 / (39.7, 38.6), 6144 73.3 / (72.2, 69.4); with the convolution 512 11.1 /
+//     8.9, 768 13.5 / (14.6), 1536 23.5 / (24.0, 25.1), 6144 75.9 / (87.4, 78.6)
+//   mixer step, factored:     24 9.9 / 6.8, 768 16.0 / 13.5, 1536 23.7 / (23.6); with the
+//     convolution 24 10.9 / 7.7, 512 14.7 / 12.5, 640 16.8 / (19.0), 768 17.9 / (20.2)
 //   step, d_state 128, f32:   24 7.9 / 5.0, 768 21.4 / 20.2, 6144 138.5 / 135.0
 //     (kHalf; kEarly 137.5); factored 24 7.9 / 5.1, 768 14.5 / 13.2, 1536 23.6 /
 //     (24.4); d_state 64 16 5.0 / 3.8, 512 9.3 / 7.5, 4096 48.6 / 46.8 (kHalf)
+//   step, heads of 16, d_state 64: 800 6.4 / (kHalf 7.3), 2048 10.6 / (12.2); of 33 2048
+//     16.3 / (17.0); d_state 16, heads of 16 768 5.1 / (kEarly 5.3)
+//   step, rank 8, factored, d_state 64: 4 18.8 / (kEarly 19.5), 256 20.0 / (20.8)
 //   step, rank 4:             24 16.6 / 13.1, 240 19.1 / 16.3 (kEarly; kWide spills
 //     from rank 4 on), 384 22.0 / (21.5), 768 28.8 / (31.7)
 enum class StepForm { kBase, kHalf, kEarly, kWide };   // 256, 512, 512 and 1024 threads
 StepForm step_form(const StepLaunch &a, bool mix, bool conv) {
     const size_t wg = a.batch * a.heads, N = a.d_state;
     const bool fact = a.last_u == nullptr;
-    if (wg <= 256) return a.rank <= 2 ? StepForm::kWide : StepForm::kEarly;
-    if (a.rank != 1) return StepForm::kBase;
-    if (wg <= 768) return StepForm::kEarly;
-    if (fact || (mix ? N != 128 : N < 64)) return StepForm::kBase;
-    return mix && !conv ? StepForm::kEarly : StepForm::kHalf;
+    if (wg <= 256)
+        return a.rank <= 2 ? StepForm::kWide : a.rank < 8 || !fact ? StepForm::kEarly : StepForm::kBase;
+    if (a.rank != 1 || a.head_dim * N < 1024) return StepForm::kBase;
+    if (wg <= (conv ? 512 : 768)) return StepForm::kEarly;
+    // 512 threads need two rows a lane each
+    if (fact || (mix ? N != 128 : N < 64) || a.head_dim * N < 4096) return StepForm::kBase;
+    if (mix && !conv) return StepForm::kEarly;
+    return conv && wg < 1536 ? StepForm::kBase : StepForm::kHalf;
 }
 
 template <typename T, int RK, bool FACT>

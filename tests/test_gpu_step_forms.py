@@ -23,6 +23,10 @@ STEP_CASES = [
     (769, 1, 50, 64, 1, False, torch.float32, True),       # 769
     (97, 8, 64, 32, 1, False, torch.bfloat16, True),       # 776, d_state under 64
     (97, 8, 64, 128, 1, True, torch.float32, False),
+    (97, 8, 63, 64, 1, False, torch.float32, True),        # rows short of 512 threads' two passes
+    (65, 4, 15, 64, 1, False, torch.float32, True),        # and of any form past 256
+    (3, 5, 16, 64, 8, True, torch.bfloat16, True),         # rank 8, factored and not
+    (3, 5, 16, 64, 8, False, torch.bfloat16, True),
 ]
 
 
@@ -48,7 +52,7 @@ def test_step_forms_agree_bit_for_bit(B, H, P, N, R, factored, dtype, rot):
                 assert torch.equal(getattr(a, k), getattr(b, k)), (step, k)
 
 
-@pytest.mark.parametrize("B", [1, 64, 65, 192, 193])
+@pytest.mark.parametrize("B", [1, 64, 65, 128, 129, 192, 193, 383, 384])
 @pytest.mark.parametrize("N,R,conv,factored", [(128, 1, False, False), (128, 1, True, False),
                                                (64, 1, False, False), (128, 1, False, True),
                                                (32, 2, True, True), (128, 4, False, False)])
