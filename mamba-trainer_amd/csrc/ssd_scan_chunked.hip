@@ -3289,23 +3289,32 @@ SegPlan seg_plan(const ScanLaunch &a) {
     // (0.4 us): the least sum is near k = sqrt(nsub / 18), taken as the power of
     // two 1, 2, 4 .. up to 32, 128, 512 .. sub-chunks, where a chunk_size of at
     // most 64 tokens does not ask for longer ones, and the next powers up to 64
-    // tokens where its records are more than the static scratch of
-    // m3_scan_no_alloc holds: both calls then cut alike and agree bit for bit,
-    // and past those 32 MiB the grid is full and short segments lose (rank 2, 32
-    // sequences of 1000 tokens, d_state 128, 68 MB of f32 records 83.5 us against
-    // 79.9, 34 MB of bf16 ones 49.1 against 46.0; rank 4, 48 of 2000, 64, 100 MB
-    // of f32 263 against 243).  Segments of 64 tokens against these, us a call:
-    // f32, 8 sequences of 512 tokens, d_state 64 25.8 / 22.1; 12 of 128, 128
-    // 33.1 / 22.6; 4 of 4096, 64 45.6 / 45.5; rank 2, 8 of 300, 64 40.6 / 24.7;
-    // rank 4, 8 of 1000, 128 119 / 73, 8 of 2000, 64 94.2 / 77.5; bf16, rank 2,
-    // 12 of 300, 128 32.2 / 25.0; rank 4, 12 of 300, 128 32.8 / 23.8; one
-    // sub-chunk a segment all the way, f32, 4 of 4096, 64 61.5.
+    // tokens
+    // - where the workgroups are more than share the CUs without slowing each
+    //   other's walk: five for four CUs, ten for four in the f32 kernels that
+    //   matrix units bound (rank 2 and 4, d_state 128);
+    // - where the records are more than the static scratch of m3_scan_no_alloc
+    //   holds: both calls then cut alike and agree bit for bit.
+    // Segments of 64 tokens against these, us a call: f32, 8 sequences of 512
+    // tokens, d_state 64 25.8 / 22.1; 12 of 128, 128 33.1 / 22.6; 24 of 700, 128
+    // 45.9 / (34 MB of records: 41.4); rank 2, 8 of 300, 64 40.6 / 24.7; rank 4, 8 of
+    // 1000, 128 119 / 73, 8 of 2000, 64 94.2 / 77.5; bf16, rank 2, 12 of 300, 128
+    // 32.2 / 25.0; rank 4, 12 of 300, 128 32.8 / 23.8; with more workgroups: f32, 24
+    // of 630, 64 28.4 / (31.0), 12 of 1024, 64 28.4 / (32.4); rank 4, 8 of 3774, 64
+    // 114 / (132); bf16, rank 2, 32 of 1024, 64 36.9 / (42.3); rank 4, 8 of 2048, 128
+    // 39.6 / (45.4).  Over 952 shapes of 2 to 96 sequences of 96 to 4096 tokens the
+    // geometric mean is 0.80 of 64-token segments, the best of every cut 0.785, and
+    // four shapes lose 4 to 6 %.
     if (q <= 64 && (a.path & 2) == 0) {
+        const bool heavy = !a.bf16 && (a.rank > 1 || a.d_state == 128);
+        const size_t most = device_cus() * (heavy ? 10 : 5) / 4;
         size_t k2 = 1;
         while (k2 * k2 * 32 < nsub) k2 *= 2;
         for (; k2 < kmin; k2 *= 2) {
             const size_t kk = std::min(std::max(k, k2), nsub), nseg = (nsub + kk - 1) / kk;
-            if (chunked_layout(bh * nseg, a.d_state, a.bf16 != 0).total <= kNoAllocScratchBytes) break;
+            if (bh * nseg <= most &&
+                chunked_layout(bh * nseg, a.d_state, a.bf16 != 0).total <= kNoAllocScratchBytes)
+                break;
         }
         kmin = std::min(kmin, k2);
     }
