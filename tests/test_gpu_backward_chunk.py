@@ -139,3 +139,38 @@ def test_wide_angles_against_f64(scale):
         return
     for k in ("x", "b", "c", "lam"):
         assert rel_l2(host(getattr(g, k)), ref[k]) <= tol, (k, rel_l2(host(getattr(g, k)), ref[k]))
+
+
+@pytest.mark.parametrize("N,R", [(64, 1), (128, 1), (64, 4)])
+@pytest.mark.parametrize("lo,hi", [(200, 900), (1 << 15, 1 << 17)])
+def test_exact_angles_past_the_short_reduction(N, R, lo, hi):
+    """Angles that f32 holds exactly, whole numbers of radians below 2^24 (dt =
+    1/16, theta whole multiples of 16), on both sides of 2^13 within a chunk,
+    where the sine's short reduction hands over to the library's, and far past
+    it: no angle is rounded, so the gradients hold F32_TOL as those of small
+    angles do.  A sine past its range or a wrong hand-over would be off by its
+    whole size."""
+    import oracle
+    from cases import baseline_inputs
+    from gpu_util import dev
+    from mamba3.ssm import ScanInputs, mamba3_scan_backward
+    rng = np.random.default_rng(lo + N + R)
+    B, T, H, P = 1, 70, 2, 64
+    inp = baseline_inputs(rng, B, T, H, P, N, R, theta=True, theta_per_head=False)
+    inp["dt"] = np.full((B, T, H), 1 / 16, np.float32)
+    turn = rng.integers(lo, hi, (B, T, H, N // 2)) * rng.choice([-1, 1], (1, 1, H, N // 2))
+    turn[..., 0] = 256      # exactly 2^13 at the 32nd token
+    inp["theta"] = (16 * turn).astype(np.float32)
+    phi = np.cumsum(turn, 1)
+    assert np.abs(phi).max() < 1 << 24
+    if lo < 1000:
+        first = np.abs(phi[:, : 32 // R])
+        assert R == 4 or (first.min() < 8192 < first.max())
+    dy = rng.standard_normal((B, T, H, P, R)).astype(np.float32)
+    si = ScanInputs(dev(inp["x"]), dev(inp["b"]), dev(inp["c"]), dev(inp["dt"]), dev(inp["a_log"]),
+                    dev(inp["lam"])).with_theta(dev(inp["theta"]))
+    g = mamba3_scan_backward(si, dev(dy))
+    ref = oracle.scan_backward_f64(inp["x"], inp["b"], inp["c"], inp["dt"], inp["a_log"], inp["lam"], dy,
+                                   inp["theta"], None, None, None, None, None, None, None)
+    for k in ("x", "b", "c", "lam", "theta"):
+        assert rel_l2(host(getattr(g, k)), ref[k]) <= F32_TOL, (k, rel_l2(host(getattr(g, k)), ref[k]))
