@@ -147,10 +147,12 @@ __device__ __forceinline__ float clamp_exp(float d) {
 // exact as the step between them.  One f32 prefix of a long, fast-decaying
 // chunk (about -50 at its end) holds 4e-6, which came out whole in every decay
 // factor of its last rows and in da_log.
+// A decay past -1e30 (infinite ones too) is taken there, where a prefix of 32
+// and its grid still have a finite difference of zero with itself.
 __device__ __forceinline__ void split_decay(float dt, float A, float &hi, float &lo) {
-    const float v = dt * A;
+    const float v0 = dt * A, v = fmaxf(v0, -1e30f);
     hi = rintf(v * 16384.0f) * (1.0f / 16384.0f);
-    lo = (v - hi) + __builtin_fmaf(dt, A, -v);
+    lo = (v - hi) + (v == v0 ? __builtin_fmaf(dt, A, -v) : 0.0f);
 }
 
 // sin and cos of an angle, to about an ulp: the argument less the nearest

@@ -114,6 +114,34 @@ def test_dy_off_the_dword_grid():
         assert torch.equal(getattr(a, k), getattr(b, k)), k
 
 
+@pytest.mark.parametrize("a_log", [40.0, 85.0, 100.0])
+@pytest.mark.parametrize("P,N,R,dtype", [(64, 64, 1, "f32"), (64, 128, 2, "bf16"), (16, 16, 1, "f32")])
+def test_decays_that_end_a_state_at_once(P, N, R, dtype, a_log):
+    """exp(a_log) dt from 1e16 to past f32's range: every token forgets all
+    before it, and the gradients of x, b, c, lambda and theta are those of the
+    token itself (theta's, zero without a past, small against b's)."""
+    import oracle
+    from cases import baseline_inputs
+    from gpu_util import dev
+    from mamba3.ssm import ScanInputs, mamba3_scan_backward
+    rng = np.random.default_rng(int(a_log) + N)
+    B, T, H = 1, 70, 2
+    inp = baseline_inputs(rng, B, T, H, P, N, R, theta=True, theta_per_head=False, dtype=dtype)
+    inp["a_log"] = np.full((H,), a_log, np.float32)
+    ty = torch.bfloat16 if dtype == "bf16" else torch.float32
+    dy = dev(rng.standard_normal((B, T, H, P, R)), ty)
+    si = ScanInputs(dev(inp["x"], ty), dev(inp["b"], ty), dev(inp["c"], ty), dev(inp["dt"]), dev(inp["a_log"]),
+                    dev(inp["lam"])).with_theta(dev(inp["theta"], ty))
+    g = mamba3_scan_backward(si, dy)
+    ref = oracle.scan_backward_f64(inp["x"], inp["b"], inp["c"], inp["dt"], np.minimum(inp["a_log"], 60),
+                                   inp["lam"], host(dy), inp["theta"], None, None, None, None, None, None, None)
+    for k in ("x", "b", "c", "lam"):
+        tol = F32_TOL if dtype == "f32" or k == "lam" else BF16_TOL
+        assert rel_l2(host(getattr(g, k)), ref[k]) <= tol, (k, rel_l2(host(getattr(g, k)), ref[k]))
+    assert np.abs(host(g.theta)).max() <= 1e-4 * np.abs(ref["b"]).max()
+    assert a_log > 90 or np.isfinite(host(g.a_log)).all() and np.isfinite(host(g.dt)).all()
+
+
 @pytest.mark.parametrize("scale", [1.0, 300.0, 3e5])
 def test_wide_angles_against_f64(scale):
     """In-chunk angles of a few turns, of hundreds and past the range of the
