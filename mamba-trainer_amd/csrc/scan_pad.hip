@@ -10,7 +10,7 @@
 // bounds them is that serial chain, not work: at batch 4 x 512, 4 heads of 16,
 // d_state 16, f32, 16 of the 256 CUs are busy for 233 us (forward) and
 // 5613 us (backward).  Padded, the 16 sequences are cut in chunks that run side by
-// side: 33 and 59 us, for the most part launches and their gaps.
+// side: 32 and 57 us, for the most part launches and their gaps.
 #include <algorithm>
 
 #include "m3_device.hpp"
@@ -415,14 +415,19 @@ hipError_t launch_pads(const Pads &p, bool out, hipStream_t s) {
 
 }  // namespace
 
-// Measured on MI355X (f32, head_dim and d_state 16, us per call, one workgroup
-// per sequence against padded): 8 sequences of 128 tokens 65 against 24; 16 of
-// 512 233 against 33; 64 of 400 (heads of 32) 153 against 50; 512 of 512 340
-// against 211; 1024 of 512 344 against 403, for a thousand sequences fill the
-// chip as they are.  The line at 128 rows is where the two met (8 of 64 / 96
-// 38 / 51 against 38 / 53) before the padded windows were cut into as many
-// segments as they are now; 4 of 33 at rank 4 were 54 against 56, 4096 of 64 160
-// against 268.
+// Measured on MI355X (f32, us per call, one workgroup per sequence / padded):
+// - head_dim and d_state 16, 8 sequences of 33 tokens 28.8 / 24.5, 64 34.3 / 24.4, 96
+//   47.9 / 26.1, 128 61.7 / 25.7; 16 of 512 227 / 32; rank 4, 8 of 8 tokens 16.8 / 24.9, 16
+//   26.1 / 25.7, 24 35.7 / 26.7, 32 44.9 / 26.1;
+// - heads of 32, d_state 32: 8 of 33 25.2 / 25.5, 64 28.8 / 25.6, 96 39.7 / 26.5, 128 50.5 /
+//   26.2; 64 of 400 148 / 48; d_state 64, 8 of 33 32.9 / 26.5, 64 37.8 / 25.8;
+// - many sequences of 512 tokens, heads of 16: 256 314 / 98, 512 322 / 206, 640 326 /
+//   427, 768 326 / 329, 1024 326 / 469; of 128 tokens 512 88 / 55, 1024 95 / 92.
+// The line at 512 sequences lies where a thousand fill the chip as they are.  The
+// line at 128 rows is older than the segments of less than 64 tokens, which moved
+// the meeting point to some 33 rows (rank 4: 64): windows between are left on the
+// slower kernel.  Heads of 33 to 63, and head_dim 64 at d_state below 64, were not
+// measured.
 bool scan_pad_wanted(const ScanLaunch &a) {
     return a.seq * a.rank >= 128 && a.batch * a.heads <= 512 && pad_shape(a, false);
 }
@@ -471,12 +476,12 @@ hipError_t launch_scan_pad(const ScanLaunch &call, void *workspace, size_t room,
     });
 }
 
-// The token walk against padded (f32, head_dim and d_state 16, us per call): 2
-// sequences of 8 / 64 tokens 98 / 701 against 32 / 33; 16 of 512 5613 against 59;
-// 1024 of 512 8507 against 1160; 8192 of 32 4471 against 815; 2 of 1 token 20 by
-// the walk.  The line at 8 tokens was drawn with the chunk kernels at 50 us, which
+// The token walk / padded (f32, head_dim and d_state 16, us per call): 2 sequences
+// of 8 tokens 94 / 34, of 64 701 / 38; 16 of 512 5637 / 57; 1024 of 512 8445 / 1219 (in
+// parts, 447 MB; at once 1155 in 1.8 GB), 8192 of 32 5248 / 802; 2 of 1 token 20 by the
+// walk.  The line at 8 tokens was drawn with the chunk kernels at 50 us, which
 // met the walk at 4 (52).  Heads over 32, states over 64 and other ranks keep the
-// walk's two launches.
+// walk's two launches; its line against them was not measured.
 bool scan_backward_pad_wanted(const ScanLaunch &a) { return a.seq >= 8 && pad_shape(a, true); }
 
 size_t scan_backward_pad_workspace(const ScanLaunch &a) {
