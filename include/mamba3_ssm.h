@@ -204,9 +204,9 @@ m3_status m3_scan_gated(const m3_scan_inputs *in, const m3_scan_output *out, con
  * For small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4; 128 rows of
  * (token, rank) or more, up to 512 sequences) it holds zero-padded f32 copies
  * the chunk-parallel kernels run on, at most 512 MiB (a larger call runs in
- * parts of its batch or heads through them); without it, and where one
- * sequence's copies exceed M3_NO_ALLOC_SCRATCH_MIB (from some 20,000 tokens
- * of rank 1 on, 7,000 of rank 4), those shapes run as one workgroup per sequence.
+ * parts of its batch or heads through them; a sequence whose copies exceed
+ * M3_NO_ALLOC_SCRATCH_MIB, from some 20,000 tokens of rank 1 on, in windows);
+ * without it those shapes run as one workgroup per sequence.
  * No reference counterpart (see m3_scan_inputs.workspace). */
 size_t m3_scan_workspace_bytes(const m3_scan_inputs *in);
 

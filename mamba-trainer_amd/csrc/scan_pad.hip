@@ -164,9 +164,11 @@ size_t up256(size_t v) { return (v + 255) & ~size_t(255); }
 // some heads of one, whose copies and kernels' workspace fit the room there is:
 // the padded rows are up to 16 times the caller's and the backward's records 64 x
 // 64 a chunk, 3.4 KB of both a token of a head of 16, so all of a long batch at
-// once would take gigabytes.
+// once would take gigabytes.  A forward sequence whose own copies do not fit the
+// static scratch runs in windows of its tokens, the state of one entering the
+// next.
 struct PadPart {
-    size_t b0, nb, h0, nh;
+    size_t b0, nb, h0, nh, t0, nt;
 };
 
 // The part as a call of its own, but for the pointers into the arrays.
@@ -174,6 +176,7 @@ ScanLaunch part_of(const ScanLaunch &a, const PadPart &q) {
     ScanLaunch p = a;
     p.batch = q.nb;
     p.heads = q.nh;
+    p.seq = q.nt;
     p.a_log = a.a_log ? a.a_log + q.h0 : nullptr;
     p.d_skip = a.d_skip ? a.d_skip + q.h0 : nullptr;
     return p;
@@ -189,7 +192,7 @@ struct PadLayout {
     size_t total;
 };
 PadLayout pad_layout(const ScanLaunch &a, const PadPart &q, bool backward) {
-    const size_t es = backward && a.bf16 ? 2 : 4, rows = q.nb * a.seq * q.nh, bh = q.nb * q.nh;
+    const size_t es = backward && a.bf16 ? 2 : 4, rows = q.nb * q.nt * q.nh, bh = q.nb * q.nh;
     const size_t xr = up256(rows * kPadP * a.rank * es), br = up256(rows * kPadN * a.rank * es);
     const size_t tr = up256(rows * (kPadN / 2) * es), st = up256(bh * kPadP * kPadN * 4);
     const size_t an = up256(bh * (kPadN / 2) * 4), sc = q.nh < a.heads ? up256(rows * 4) : 0;
@@ -243,7 +246,7 @@ struct PadShape {
 struct PadShapes {
     PadShape x, bc, theta, state, angle, scalar;
     PadShapes(const ScanLaunch &a, const PadPart &part, bool backward) {
-        const uint32_t rows = static_cast<uint32_t>(part.nb * a.seq * part.nh);
+        const uint32_t rows = static_cast<uint32_t>(part.nb * part.nt * part.nh);
         const uint32_t bh = static_cast<uint32_t>(part.nb * part.nh);
         const uint32_t nh = static_cast<uint32_t>(part.nh), H = static_cast<uint32_t>(a.heads);
         const uint32_t P = static_cast<uint32_t>(a.head_dim), N = static_cast<uint32_t>(a.d_state);
@@ -253,7 +256,7 @@ struct PadShapes {
         const uint32_t lo = N / 2 > 0 ? N / 2 : N, hi = N - lo;
         const uint32_t q = log2u(kPadP * R / 4);
         const PadKind t = !a.bf16 ? kPad32 : backward ? kPad16 : kPadWiden;
-        const size_t row0 = part.b0 * a.seq * a.heads + part.h0, seq0 = part.b0 * a.heads + part.h0;
+        const size_t row0 = (part.b0 * a.seq + part.t0) * a.heads + part.h0, seq0 = part.b0 * a.heads + part.h0;
         const size_t es = a.bf16 ? 2 : 4;
         x = {{nullptr, nullptr, rows, P * R, 0, static_cast<uint32_t>(kPadP) * R / 2, q, 1, 0, t, nh, H},
              row0 * P * R * es};
@@ -314,9 +317,11 @@ ScanLaunch padded(const ScanLaunch &a, const PadPart &part, const PadLayout &l, 
     p.theta = c.put(s.theta, a.theta, l.theta);
     p.dt = c.put_row(s.scalar, a.dt, l.dt);
     p.lambda = c.put_row(s.scalar, a.lambda, l.lam);
-    p.h0 = static_cast<const float *>(c.put(s.state, a.h0, l.h));
-    p.last_u0 = static_cast<const float *>(c.put(s.state, a.last_u0, l.lu));
-    p.angle0 = static_cast<const float *>(c.put(s.angle, a.angle0, l.ang));
+    if (part.t0 == 0) {   // a later window's state is where the one before left it
+        p.h0 = static_cast<const float *>(c.put(s.state, a.h0, l.h));
+        p.last_u0 = static_cast<const float *>(c.put(s.state, a.last_u0, l.lu));
+        p.angle0 = static_cast<const float *>(c.put(s.angle, a.angle0, l.ang));
+    }
     return p;
 }
 
@@ -345,8 +350,13 @@ bool pad_shape(const ScanLaunch &a, bool backward) {
 }
 
 size_t part_bytes(const ScanLaunch &a, const PadPart &q, bool backward) {
-    const ScanLaunch p = padded_shape(part_of(a, q), backward);
-    return pad_layout(a, q, backward).total + (backward ? scan_backward_workspace(p) : scan_chunked_workspace(p));
+    ScanLaunch p = padded_shape(part_of(a, q), backward);
+    size_t kernels = backward ? scan_backward_workspace(p) : scan_chunked_workspace(p);
+    if (a.seq % q.nt != 0) {   // the last window may be cut into more segments than a longer one
+        p.seq = a.seq % q.nt;
+        kernels = std::max(kernels, scan_chunked_workspace(p));
+    }
+    return pad_layout(a, q, backward).total + kernels;
 }
 
 // The largest of n counts from 1 on that fits; 0 if none does.
@@ -370,11 +380,14 @@ size_t largest(size_t n, F fits) {
 // 608 / 591, 256 of 2048 3642 / 1387 / 1241 / 1157 (1137 at once, in 1.7 GB), 8 of
 // 16384 4410 / 1279 / 793 / 795; forward, 256 of 2048 889 / 503 / 480 / 428.  The
 // kernels these shapes took before need 8 ms and 40 ms for the first two.
+// A sequence past the static scratch is cut into windows by that, whatever the
+// room, so that both of the forward's callers cut alike: 2 of 31000 tokens 421 us in
+// windows, 156 at once in 93 MB, 15816 by one workgroup each; 8 of them 1692, 253 and
+// 18702.
 PadPart pad_part(const ScanLaunch &a, bool backward, size_t room) {
     auto fits = [&](size_t nb, size_t nh) {
-        return part_bytes(a, PadPart{0, nb, 0, nh}, backward) <= room;
+        return part_bytes(a, PadPart{0, nb, 0, nh, 0, a.seq}, backward) <= room;
     };
-    if (fits(a.batch, a.heads)) return PadPart{0, a.batch, 0, a.heads};
     // the most of n that fit, or fewer in as many parts of one size
     auto share = [](size_t n, auto ok) {
         const size_t most = largest(n, ok);
@@ -382,23 +395,34 @@ PadPart pad_part(const ScanLaunch &a, bool backward, size_t room) {
         const size_t parts = (n + most - 1) / most, even = (n + parts - 1) / parts;
         return ok(even) ? even : most;
     };
+    if (!backward && part_bytes(a, PadPart{0, 1, 0, 1, 0, a.seq}, false) > kNoAllocScratchBytes) {
+        const size_t tiles = share((a.seq + 63) / 64, [&](size_t v) {
+            return part_bytes(a, PadPart{0, 1, 0, 1, 0, 64 * v}, false) <= kNoAllocScratchBytes;
+        });
+        return tiles > 0 ? PadPart{0, 1, 0, 1, 0, 64 * tiles} : PadPart{};
+    }
+    if (fits(a.batch, a.heads)) return PadPart{0, a.batch, 0, a.heads, 0, a.seq};
     const size_t nb = share(a.batch, [&](size_t v) { return fits(v, a.heads); });
-    if (nb > 0) return PadPart{0, nb, 0, a.heads};
+    if (nb > 0) return PadPart{0, nb, 0, a.heads, 0, a.seq};
     const size_t nh = share(a.heads, [&](size_t v) { return fits(1, v); });
-    return nh > 0 ? PadPart{0, 1, 0, nh} : PadPart{};
+    return nh > 0 ? PadPart{0, 1, 0, nh, 0, a.seq} : PadPart{};
 }
 
-// f(part) for every part of the call, whose first is q.
+// f(part) for every part of the call, whose first is q; a sequence's windows in
+// order.
 template <typename F>
 hipError_t each_part(const ScanLaunch &a, PadPart q, F f) {
-    const size_t nb = q.nb, nh = q.nh;
+    const size_t nb = q.nb, nh = q.nh, nt = q.nt;
     if (nb == 0) return hipErrorNotSupported;
     for (q.b0 = 0; q.b0 < a.batch; q.b0 += nb) {
         q.nb = std::min(nb, a.batch - q.b0);
         for (q.h0 = 0; q.h0 < a.heads; q.h0 += nh) {
             q.nh = std::min(nh, a.heads - q.h0);
-            const hipError_t e = f(q);
-            if (e != hipSuccess) return e;
+            for (q.t0 = 0; q.t0 < a.seq; q.t0 += nt) {
+                q.nt = std::min(nt, a.seq - q.t0);
+                const hipError_t e = f(q);
+                if (e != hipSuccess) return e;
+            }
         }
     }
     return hipSuccess;
@@ -444,27 +468,45 @@ static ScanLaunch planned(const ScanLaunch &a) {
 size_t scan_pad_workspace(const ScanLaunch &a, size_t room) {
     if (!scan_pad_wanted(a)) return 0;
     const ScanLaunch p = planned(a);
-    // a sequence that the static scratch does not hold (from some 20,000 tokens of
-    // rank 1 on, 7,000 of rank 4) takes one workgroup in either call
-    if (p.plan_seqs == 0 || part_bytes(p, PadPart{0, 1, 0, 1}, false) > kNoAllocScratchBytes) return 0;
     return part_bytes(p, pad_part(p, false, room), false);
 }
 
 hipError_t launch_scan_pad(const ScanLaunch &call, void *workspace, size_t room, hipStream_t stream,
                            int &launches) {
     const ScanLaunch a = planned(call);
-    return each_part(a, pad_part(a, false, room), [&](const PadPart &q) {
-        const PadLayout l = pad_layout(a, q, false);
+    const PadPart first = pad_part(a, false, room);
+    return each_part(a, first, [&](const PadPart &q) {
+        PadPart longest = q;   // windows share the layout of the longest
+        longest.nt = first.nt;
+        const PadLayout l = pad_layout(a, longest, false);
         const PadShapes s(a, q, false);
         PadCopies c{static_cast<char *>(workspace), q.nh < a.heads, {}, {}};
         ScanLaunch p = padded(a, q, l, s, c);
         p.y = c.get(s.x, a.y, l.y);
-        p.h_out = static_cast<float *>(c.get(s.state, a.h_out, l.hout));
-        p.last_u_out = static_cast<float *>(c.get(s.state, a.last_u_out, l.luout));
-        p.angle_out = static_cast<float *>(c.get(s.angle, a.angle_out, l.angout));
+        // the state entering and leaving a window change places with each
+        const bool odd = q.t0 / first.nt % 2 != 0;
+        auto at = [&](size_t off) { return reinterpret_cast<float *>(c.base + off); };
+        const size_t hi = odd ? l.hout : l.h, ui = odd ? l.luout : l.lu, ai = odd ? l.angout : l.ang;
+        const size_t ho = odd ? l.h : l.hout, uo = odd ? l.lu : l.luout, ao = odd ? l.ang : l.angout;
+        if (q.t0 > 0) {
+            p.h0 = at(hi);
+            p.last_u0 = at(ui);
+            p.angle0 = a.theta ? at(ai) : nullptr;
+        }
+        if (q.t0 + q.nt < a.seq) {
+            p.h_out = at(ho);
+            p.last_u_out = at(uo);
+            p.angle_out = a.theta ? at(ao) : nullptr;
+        } else {
+            p.h_out = static_cast<float *>(c.get(s.state, a.h_out, ho));
+            p.last_u_out = static_cast<float *>(c.get(s.state, a.last_u_out, uo));
+            p.angle_out = static_cast<float *>(c.get(s.angle, a.angle_out, ao));
+        }
+        const size_t kernels = scan_chunked_workspace(p);
+        if (l.total + kernels > room) return hipErrorInvalidValue;
         hipError_t e = launch_pads(c.in, false, stream);
         if (e != hipSuccess) return e;
-        if (scan_chunked_workspace(p) > 0) {
+        if (kernels > 0) {
             e = launch_scan_chunked(p, c.base + l.total, stream, launches);
         } else {
             e = launch_scan(p, stream);
