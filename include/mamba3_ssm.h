@@ -275,10 +275,10 @@ typedef struct m3_scan_grads {
  * buffers (bf16 storage at d_state 64 also in some half of the workspace, with
  * the sequential passes run twice); every sum has a fixed order, so repeated calls agree bit for bit.
  * Small heads (head_dim <= 32, d_state <= 64, rank 1, 2 or 4, from 8 tokens
- * on) run them on zero-padded copies in the workspace, at most 512 MiB (a
- * larger call runs in parts of its batch, whose shares of da_log and dd_skip
- * add up in order, or of its heads).  Other shapes (and
- * alignments) take the reverse mode of the recurrence token by token, one
+ * on) run them on zero-padded copies in the workspace, at most 512 MiB or
+ * one sequence's, whichever is more (a larger call runs in parts of its batch,
+ * whose shares of da_log and dd_skip add up in order, or of its heads).  Other
+ * shapes (and alignments) take the reverse mode of the recurrence token by token, one
  * workgroup per sequence with states recomputed from checkpoints
  * every 32 tokens (deterministic, and slow: a fallback), up to per-token
  * vectors of 64 KB (2 head_dim rank + 4 d_state rank + 3 d_state/2 floats;

@@ -171,8 +171,8 @@ hipError_t launch_scan_backward_generic(const ScanLaunch &a, const ScanGrads &g,
 // The heads of small models (head_dim up to 32, d_state up to 64, rank 1, 2 or
 // 4) on zero-padded copies through the kernels above (scan_pad.hip): whether
 // that is the faster form, the workspace it takes (0 where it is not; at most
-// kPadBytes, or the forward's `room` from the static scratch's size on, through
-// which a larger call runs part by part) and the launch, which adds its kernels
+// kPadBytes or one sequence's for the backward, or the forward's `room` from the
+// static scratch's size on, through which a larger call runs part by part) and the launch, which adds its kernels
 // to `launches`.
 constexpr size_t kPadBytes = size_t(512) << 20;
 bool scan_pad_wanted(const ScanLaunch &a);

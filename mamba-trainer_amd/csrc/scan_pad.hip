@@ -374,8 +374,10 @@ size_t largest(size_t n, F fits) {
 }
 
 // The first (and largest) part within `room` bytes: the whole call, else as
-// many batch entries as fit, shared out evenly, else as many heads of one;
-// nb = 0 where one sequence does not fit.  Parts of 64 / 256 / 512 / 1024 MiB, us
+// many batch entries as fit, shared out evenly, else as many heads of one; one
+// sequence at the least for the backward (heads of 64 ask for as much; one of
+// 170,000 tokens, rank 1 in f32, 5.8 ms in 522 MiB, where the token walk takes 11 us a
+// token), nb = 0 for the forward where that does not fit.  Parts of 64 / 256 / 512 / 1024 MiB, us
 // a call, heads of 16, f32: backward, 512 sequences of 512 tokens 1022 / 611 /
 // 608 / 591, 256 of 2048 3642 / 1387 / 1241 / 1157 (1137 at once, in 1.7 GB), 8 of
 // 16384 4410 / 1279 / 793 / 795; forward, 256 of 2048 889 / 503 / 480 / 428.  The
@@ -405,7 +407,8 @@ PadPart pad_part(const ScanLaunch &a, bool backward, size_t room) {
     const size_t nb = share(a.batch, [&](size_t v) { return fits(v, a.heads); });
     if (nb > 0) return PadPart{0, nb, 0, a.heads, 0, a.seq};
     const size_t nh = share(a.heads, [&](size_t v) { return fits(1, v); });
-    return nh > 0 ? PadPart{0, 1, 0, nh, 0, a.seq} : PadPart{};
+    if (nh > 0) return PadPart{0, 1, 0, nh, 0, a.seq};
+    return backward ? PadPart{0, 1, 0, 1, 0, a.seq} : PadPart{};
 }
 
 // f(part) for every part of the call, whose first is q; a sequence's windows in

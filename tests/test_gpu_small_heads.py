@@ -105,7 +105,7 @@ def test_workspace_queries_at_the_edges():
 
 def test_workspace_queries_are_bounded():
     """Large calls run part by part: neither query passes 512 MiB where the
-    padded copies are asked for, whatever the batch, the window or the heads."""
+    padded copies are asked for, whatever the batch and the heads."""
     from mamba3 import _lib
     for dt in (_lib.M3_F32, _lib.M3_BF16):
         for B, T, H, P, N, R in ((256, 2048, 4, 16, 16, 1), (64, 4096, 16, 16, 16, 1), (512, 8192, 4, 16, 16, 1),
@@ -115,6 +115,58 @@ def test_workspace_queries_are_bounded():
             assert (0 < fw <= 512 << 20) if B * H <= 512 else fw == 0, (B, T, H, fw)
             one = _query(1, T, 1, P, N, R, dt)[0]   # a sequence, or windows of it, within the static scratch
             assert 0 < one <= 32 << 20, (T, one)
+
+
+def test_a_long_sequence_keeps_the_backward_copies():
+    """One sequence is the backward's least part, past 512 MiB too: the query
+    goes on growing with its length (the token walk's asks for some 90 bytes a
+    token), and neither the batch nor the heads add to it."""
+    from mamba3 import _lib
+    for R, dt, T in ((1, _lib.M3_F32, 170000), (4, _lib.M3_F32, 47000), (4, _lib.M3_BF16, 70000)):
+        one = _query(1, T, 1, 16, 16, R, dt)[1]
+        assert one > 512 << 20 and one < 4000 * R * T, (R, T, one)
+        gathered = 16 * (T + 64)   # dt, lambda and their gradients, where the heads are apart
+        assert one <= _query(2, T, 3, 16, 16, R, dt)[1] <= one + gathered + 4096, (R, T)
+
+
+@pytest.mark.gpu
+def test_a_long_sequence_backward_is_its_padded_call():
+    """Past 512 MiB of copies: the gradients of sequences of 47,000 tokens, two
+    heads of them, against the call on heads of 64 that the zeros are written
+    into here, one head at a time.  Zeros add nothing and the kernels are the
+    same: bit for bit."""
+    from mamba3.ssm import ScanInputs, mamba3_scan_backward
+    T, H, P, N, R = 47000, 2, 16, 16, 4
+    g = torch.Generator(device="cuda").manual_seed(7)
+    r = lambda *s: torch.randn(s, device="cuda", generator=g)
+    u = lambda *s: torch.rand(s, device="cuda", generator=g)
+    x, b, c, dy = r(1, T, H, P, R), r(1, T, H, N, R) / 4, r(1, T, H, N, R) / 4, r(1, T, H, P, R)
+    dt, a_log, lam, theta = u(1, T, H) * 0.1, u(H) * 2.7, u(1, T, H), u(1, T, H, N // 2) * 3
+
+    def grown(t, n):
+        out = t.new_zeros(*t.shape[:3], n, *t.shape[4:])
+        out[:, :, :, :t.shape[3]] = t
+        return out
+
+    def call(hs, p, n):
+        pick = lambda t: t[:, :, hs].contiguous()
+        # a pair's two elements stand in the halves of d_state
+        both = lambda t: torch.cat([grown(t[:, :, :, :N // 2], n // 2), grown(t[:, :, :, N // 2:], n // 2)], dim=3)
+        si = ScanInputs(grown(pick(x), p), both(pick(b)), both(pick(c)), pick(dt), a_log[hs].contiguous(),
+                        pick(lam)).with_theta(grown(pick(theta), n // 2))
+        return mamba3_scan_backward(si, grown(pick(dy), p))
+
+    got = call(slice(0, H), P, N)
+    for h in range(H):
+        want = call(slice(h, h + 1), 64, 64)
+        assert torch.equal(got.x[:, :, h], want.x[:, :, 0, :P]), h
+        assert torch.equal(got.theta[:, :, h], want.theta[:, :, 0, :N // 2]), h
+        pairs = [*range(N // 2), *range(32, 32 + N // 2)]
+        for name in ("b", "c"):
+            assert torch.equal(getattr(got, name)[:, :, h], getattr(want, name)[:, :, 0, pairs]), (name, h)
+        for name in ("dt", "lam"):
+            assert torch.equal(getattr(got, name)[:, :, h], getattr(want, name)[:, :, 0]), (name, h)
+        assert torch.equal(got.a_log[h], want.a_log[0]), h
 
 
 # more rows than 512 MiB of copies hold: parts of the batch, the last one short;
